@@ -34,10 +34,8 @@ template <typename T>
 int qb_getrf_graph(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipiv, int64_t sP,
                    int* info, int batch, bool first_done = false);
 void qb_graphs_clear(qb_ctx* ctx);
-// Triangular-solve leaf kernel for every later launch of the process: 1 the
-// one-wave LDS leaf (k_trsm_leaf), 0 the register leaf (k_trsm_leaf_reg), -1
-// back to the default (QB_TRSM_LEAF=lds, else the register leaf for launches
-// of at least 8 waves per CU and the LDS leaf below).
+// No effect: there is one triangular-solve leaf (kept for callers that chose
+// between two).
 void qb_set_trsm_leaf_lds(int mode);
 // Triangular solves only (the row permutation is applied separately, fused
 // into the gather that fills B).

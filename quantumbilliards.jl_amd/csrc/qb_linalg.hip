@@ -954,22 +954,24 @@ const char* qb_gemm_variant_name(int ty, int v) {
   return (ty >= 0 && ty < 2 && v >= 0 && v < QB_GEMM_VARIANTS) ? kGemmNames[ty][v] : "?";
 }
 
-// ---------------------------------------------------------------------------
-// Leaf panel factorisation: columns [c0, c0+w) of rows [c0, n), w <= 32.
-// One workgroup per matrix, left-looking (Crout) order inside the leaf:
-// step c first forms the U part of column c (rows c0..c0+c-1) by forward
-// substitution with the unit-lower top block kept in LDS, then updates the
-// rest of column c with all previous L columns at once (only loads until the
-// single store per row, so a thread keeps many loads in flight), picks the
-// pivot on max |re|+|im| (LAPACK's izamax measure), swaps the pivot row into
-// place across the w columns and scales the column.  Each step reads c+1
-// columns and writes two, against ~2(w-c) read-modify-written columns in the
-// right-looking order.  A zero pivot leaves the column unscaled and counts
-// in info, the behaviour of zgetf2 behind lu!(check=false).
-// ---------------------------------------------------------------------------
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// Explicit fused operations: every kernel that forms these rounds alike.
 template <typename T>
 __device__ __forceinline__ T cmul_(T a, T b) {
-  return T{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+  return T{fma_(a.re, b.re, -(a.im * b.im)), fma_(a.re, b.im, a.im * b.re)};
+}
+// conj(a) / |a|^2
+template <typename T>
+__device__ __forceinline__ T cinv_(T a) {
+  const auto den = fma_(a.re, a.re, a.im * a.im);
+  return T{a.re / den, -a.im / den};
+}
+// x -= a y, four fused multiply-adds
+template <typename T>
+__device__ __forceinline__ void cnma_(T& x, const T& a, const T& y) {
+  x.re = fma_(a.im, y.im, fma_(-a.re, y.re, x.re));
+  x.im = fma_(-a.im, y.re, fma_(-a.re, y.im, x.im));
 }
 
 // A[i] when ok, else 0, loaded component by component (a conditional
@@ -985,10 +987,332 @@ __device__ __forceinline__ T ld_or0(const T* p, bool ok) {
   return v;
 }
 
+// Workgroup barrier that orders LDS only: outstanding global loads and stores
+// stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One step of a wave maximum: max(x, x of the lane that the DPP control names),
+// x itself where there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_max(double x) {
+  const int lo = __double2loint(x), hi = __double2hiint(x);
+  const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+  const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+  return __builtin_fmax(x, __hiloint2double(h2, l2));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_max(float x) {
+  const int i = __float_as_int(x);
+  return __builtin_fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false)));
+}
+__device__ __forceinline__ double lane_value(double x, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                          __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+__device__ __forceinline__ float lane_value(float x, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+// Maximum over the wave's 64 lanes (x holds no NaN): row shifts by 1, 2, 4 and
+// 8, then the row broadcasts; lane 63 holds the result.
+template <typename S>
+__device__ __forceinline__ S wave_max(S x) {
+  x = dpp_max<0x111, 0xf>(x);
+  x = dpp_max<0x112, 0xf>(x);
+  x = dpp_max<0x114, 0xf>(x);
+  x = dpp_max<0x118, 0xf>(x);
+  x = dpp_max<0x142, 0xa>(x);
+  x = dpp_max<0x143, 0xc>(x);
+  return lane_value(x, 63);
+}
+
+// The row whose content stands in row x after the interchanges (k0 + k, p[k]),
+// k = kb .. np-1, applied in order: x traced back through them.
+__device__ __forceinline__ int swap_source(int x, int k0, const int* p, int kb, int np) {
+  for (int k = np - 1; k >= kb; --k) {
+    const int pk = p[k], ck = k0 + k;
+    x = x == pk ? ck : (x == ck ? pk : x);
+  }
+  return x;
+}
+
+// ---------------------------------------------------------------------------
+// Leaf panel factorisation: columns [c0, c0+w) of rows [c0, n), w <= 32, one
+// workgroup of NT threads per matrix.  The columns are taken W at a time and
+// held in registers, RPT rows per thread (RPT * NT >= n - c0, RPT * W = 32
+// for complex128, 64 for complex64: 128 VGPRs), so a column step touches no
+// global memory on its critical path: the pivot search on max |re|+|im|
+// (LAPACK's izamax measure, first row of the maximum) is a DPP maximum per
+// wave and one LDS candidate per wave (its row with it), and
+// the rank-1 update stays in registers (shifting the columns left by one, so
+// that the current column is always the first).  Finished columns of L and
+// rows of U are stored as they come.  The interchanges of the W steps reach
+// the other columns of the leaf at the end of the sub-block, all at once: each
+// affected row is traced back to its source (swap_source), loaded, and stored
+// after a barrier.  Before its steps a sub-block takes the update with the s
+// columns of L before it (each read once per sub-block).  A zero pivot leaves
+// the column unscaled and counts in info, the behaviour of zgetf2 behind
+// lu!(check=false).
+//
+// What bounds it: the latency of 32 column steps (one LDS barrier each) and of
+// 32/W changes of sub-block, and with many rows the L2 bandwidth of one CU, which
+// reads 32/W * 16 columns.  Four waves of 256 VGPRs (half a CU) find room beside
+// a trailing-update workgroup that ends; eight waited for both of a CU's.  The leaf that this one replaces kept its columns in
+// global memory (one workgroup too) and took, on average over the leaves of an
+// N = 530 and an N = 1792 window (32 matrices), 172 and 254 us; this one takes 90
+// and 93 (up to 512 rows), 106 (1024) and 185 us (2048).  From 4096 rows on it
+// would hold one column at a time, read as much as the leaf in global memory does
+// with fewer loads in flight, and lose to it (5.6 against 1.25 ms beside the
+// trailing update of 8192 x 8192): k_getf2_long takes those.
+// ---------------------------------------------------------------------------
+template <typename T, int NT, int RPT, int W>
+__global__ void __launch_bounds__(NT) k_getf2(T* __restrict__ A, int64_t lda, int64_t sA, int n,
+                                               int c0, int w, int* __restrict__ ipiv, int64_t sP,
+                                               int* __restrict__ info) {
+  typedef typename Scal<T>::S S;
+  constexpr int NWV = NT / 64;
+  constexpr int PH = W >= 16 ? 8 : (W == 8 ? 4 : W);  // steps per phase: the columns still live
+  __shared__ T Lt[32][33];   // Lt[i][k] = L(c0 + i, c0 + k), k < i
+  __shared__ T Us[32][W];    // U(c0 + i, c0 + s + k)
+  // of alternate steps: each wave's candidate (value, row, the row itself) and
+  // the row that the pivot row replaces
+  __shared__ T cand[2][NWV][W], crow[2][W];
+  __shared__ S red_v[2][NWV];
+  __shared__ int red_i[2][NWV];
+  __shared__ int piv[32];
+  const int64_t b = blockIdx.x;
+  A += b * sA + (int64_t)c0 * lda;  // column cc of the leaf at A + cc * lda
+  ipiv += b * sP;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  for (int s = 0; s < w; s += W) {
+    const int nw = w - s < W ? w - s : W;
+    const int r0 = c0 + s + tid;  // own rows r0 + q * NT
+    unsigned ro[RPT];             // clamped to the last row: loads are unconditional
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) ro[q] = r0 + q * NT < n ? r0 + q * NT : n - 1;
+    T a[RPT][W];
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+#pragma unroll
+      for (int q = 0; q < RPT; ++q) {
+        a[q][k] = T{0, 0};
+        if (k < nw) {
+          const T* p = A + (int64_t)(s + k) * lda + ro[q];
+          a[q][k].re = p->re;
+          a[q][k].im = p->im;
+        }
+      }
+    if (W < 32 && s > 0) {
+      // U part of the sub-block's columns: one wave per column, a row per lane
+      for (int k = wv; k < W; k += NWV) {
+        T* Ac = A + c0 + (int64_t)(s + k) * lda;
+        T x = ld_or0(Ac + lane, lane < s && k < nw);
+        for (int i = 0; i + 1 < s; ++i) {
+          const T xi = T{lane_value(x.re, i), lane_value(x.im, i)};
+          if (lane > i && lane < s) {
+            const T l = Lt[lane][i];
+            cnma_(x, l, xi);
+          }
+        }
+        if (lane < s) {
+          Us[lane][k] = x;
+          if (k < nw) Ac[lane] = x;
+        }
+      }
+      lds_barrier();
+      // rows below: a -= L(:, 0..s-1) U
+      constexpr int QC = RPT < 4 ? RPT : 4, UN = RPT == 1 ? 8 : 16 / (2 * QC);
+#pragma unroll
+      for (int q0 = 0; q0 < RPT; q0 += QC) {
+        int i = 0;
+        for (; i + UN <= s; i += UN) {
+          T l[UN][QC];
+#pragma unroll
+          for (int u = 0; u < UN; ++u)
+#pragma unroll
+            for (int q = 0; q < QC; ++q) {
+              const T* p = A + (int64_t)(i + u) * lda + ro[q0 + q];
+              l[u][q].re = p->re;
+              l[u][q].im = p->im;
+            }
+#pragma unroll
+          for (int u = 0; u < UN; ++u) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+              // U read a few columns at a time: few registers
+              if ((k & 3) == 0) asm volatile("" ::: "memory");
+              const T uk = Us[i + u][k];
+#pragma unroll
+              for (int q = 0; q < QC; ++q) cnma_(a[q0 + q][k], l[u][q], uk);
+            }
+          }
+        }
+        for (; i < s; ++i)
+#pragma unroll
+          for (int q = 0; q < QC; ++q) {
+            const T* p = A + (int64_t)i * lda + ro[q0 + q];
+            const T lq = T{p->re, p->im};
+#pragma unroll
+            for (int k = 0; k < W; ++k) cnma_(a[q0 + q][k], lq, Us[i][k]);
+          }
+      }
+    }
+    // the column steps; phase p works on the LIVE columns that may be left
+    static_for<0, W / PH>([&](auto phase) {
+      constexpr int P = decltype(phase)::value, LIVE = W - P * PH;
+      for (int j = P * PH; j < (P + 1) * PH && j < nw; ++j) {
+        const int c = s + j, row = c0 + c;
+        S best = -1;
+        int bi = n;
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+          const int r = r0 + q * NT;
+          const S v = fabs(a[q][0].re) + fabs(a[q][0].im);
+          if (r >= row && r < n && v > best) {
+            best = v;
+            bi = r;
+          }
+        }
+        const S wm = wave_max(best);
+        unsigned long long at = __ballot(best == wm);
+        int wi = __builtin_amdgcn_readlane(bi, __ffsll(at) - 1);
+        for (at &= at - 1; at; at &= at - 1) {  // ties: the smallest row
+          const int o = __builtin_amdgcn_readlane(bi, __ffsll(at) - 1);
+          wi = o < wi ? o : wi;
+        }
+        const int par = j & 1;
+        if (lane == 0) {
+          red_v[par][wv] = wm;
+          red_i[par][wv] = wi;
+        }
+        if (tid == j) {
+#pragma unroll
+          for (int k = 0; k < LIVE; ++k) crow[par][k] = a[0][k];
+        }
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+          if (r0 + q * NT == wi) {
+#pragma unroll
+            for (int k = 0; k < LIVE; ++k) cand[par][wv][k] = a[q][k];
+          }
+        lds_barrier();
+        S bv = red_v[par][0];
+        int p = red_i[par][0], pw = 0;
+#pragma unroll
+        for (int q = 1; q < NWV; ++q) {
+          const S v = red_v[par][q];
+          const int i = red_i[par][q];
+          if (v > bv || (v == bv && i < p)) {
+            bv = v;
+            p = i;
+            pw = q;
+          }
+        }
+        pw = __builtin_amdgcn_readfirstlane(pw);
+        // no candidate (a column of NaN): the row stays
+        const T* prow = p < n ? cand[par][pw] : crow[par];
+        if (p >= n) p = row;
+        if (tid == 0) {
+          ipiv[row] = p;
+          piv[c] = p;
+        }
+        if (p != row) {
+#pragma unroll
+          for (int q = 0; q < RPT; ++q)
+            if (r0 + q * NT == p) {
+#pragma unroll
+              for (int k = 0; k < LIVE; ++k) a[q][k] = crow[par][k];
+            }
+        }
+        if (tid < nw - j) A[row + (int64_t)(c + tid) * lda] = prow[tid];
+        const T pv = prow[0];
+        const bool nz = pv.re != 0 || pv.im != 0;
+        if (!nz && tid == 0 && info) atomicCAS(info + b, 0, row + 1);
+        const T inv = cinv_(pv);
+        T l[RPT];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+          l[q] = nz ? cmul_(a[q][0], inv) : a[q][0];
+          const int r = r0 + q * NT;
+          if (r > row && r < n) {
+            T* d = A + (int64_t)c * lda + (unsigned)r;
+            d->re = l[q].re;
+            d->im = l[q].im;
+          }
+        }
+#pragma unroll
+        for (int k = 1; k < LIVE; ++k) {
+          const T u = prow[k];
+#pragma unroll
+          for (int q = 0; q < RPT; ++q) {
+            T x = a[q][k];
+            cnma_(x, l[q], u);
+            a[q][k - 1] = x;
+          }
+        }
+      }
+    });
+    // the sub-block's interchanges in the other columns of the leaf, and in its
+    // own finished columns from the step after each
+    __syncthreads();
+    constexpr int NI = 64 * W > NT ? 64 * W / NT : 1;
+    T v[NI];
+    int64_t dst[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int e = tid + i * NT, t = e % (2 * W), cc = e / (2 * W);
+      const int k = t < W ? t : t - W;
+      dst[i] = -1;
+      if (cc < w && k < nw) {
+        const int x = t < W ? c0 + s + k : piv[s + k];
+        const int kb = cc >= s && cc < s + nw ? cc - s + 1 : 0;
+        const int y = swap_source(x, c0 + s, piv + s, kb, nw);
+        if (y != x) {
+          dst[i] = x + (int64_t)cc * lda;
+          const T* p = A + y + (int64_t)cc * lda;
+          v[i].re = p->re;
+          v[i].im = p->im;
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // every load has returned before the first store
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (dst[i] >= 0) {
+        A[dst[i]].re = v[i].re;
+        A[dst[i]].im = v[i].im;
+      }
+    __syncthreads();
+    if (W < 32 && s + W < w) {
+      for (int e = tid; e < W * 32; e += NT) {
+        const int i = s + e / 32, k = e % 32;
+        if (k < i) Lt[i][k] = A[c0 + i + (int64_t)k * lda];
+      }
+      __syncthreads();
+    }
+  }
+}
+
+template <typename T, int NT, int RPT, int W>
+static void launch_getf2(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, int w,
+                         int* ipiv, int64_t sP, int* info, int batch) {
+  hipLaunchKernelGGL((k_getf2<T, NT, RPT, W>), dim3(batch), dim3(NT), 0, ctx->stream, A, lda, sA, n,
+                     c0, w, ipiv, sP, info);
+}
+
+// The same leaf for more than 4096 rows: left-looking (Crout) order with the columns in global memory.  Step
+// c forms the U part of column c by forward substitution with the unit-lower
+// top block kept in LDS, updates the rest of column c with all previous L
+// columns at once, picks the pivot, swaps the pivot row into place across the
+// w columns and scales the column.
 template <typename T>
-__global__ void __launch_bounds__(1024) k_getf2(T* __restrict__ A, int64_t lda, int64_t sA,
-                                                int n, int c0, int w, int* __restrict__ ipiv,
-                                                int64_t sP, int* __restrict__ info) {
+__global__ void __launch_bounds__(512) k_getf2_long(T* __restrict__ A, int64_t lda, int64_t sA,
+                                                    int n, int c0, int w, int* __restrict__ ipiv,
+                                                    int64_t sP, int* __restrict__ info) {
   typedef typename Scal<T>::S S;
   __shared__ T Lt[32][33];  // Lt[j][k] = L(c0 + j, c0 + k), k < j
   __shared__ T u[32];       // U(c0 + k, col), k < c
@@ -1132,349 +1456,194 @@ __global__ void __launch_bounds__(1024) k_getf2(T* __restrict__ A, int64_t lda, 
   }
 }
 
-// Row interchanges ipiv[k0..k1) applied in order to columns [cb, ce)
-// (LAPACK zlaswp).  One thread per column.
+// Row interchanges ipiv[k0..k0+np) applied in order to columns [cb, ce)
+// (LAPACK zlaswp).  Every workgroup first turns them into the list of rows
+// that change and their sources: each affected row (the np rows from k0 on and
+// the pivot rows below them) is traced back through the interchanges by a
+// thread of its own.  It then moves its cpw columns, up to eight rows per
+// thread at a time: load all, barrier, store all.  P2 lanes (the next power of
+// two of the list's length, at most 256) take one column.  What bounds it: for
+// few interchanges the latency of one load and one store, where the kernel it
+// replaces (one lane per column, swap after swap) paid a round trip per
+// interchange; for many, the memory lines of the pivot rows, of which each
+// column uses 16 bytes.  Measured, per launch of an N = 530, 1792 and 8192 window
+// on average: 5.7, 12 and 19 us against 9.2, 25 and 68 us.
 template <typename T>
-__global__ void k_laswp(T* __restrict__ A, int64_t lda, int64_t sA, int cb, int ce, int k0, int k1,
-                        const int* __restrict__ ipiv, int64_t sP) {
+__global__ void __launch_bounds__(256) k_laswp(T* __restrict__ A, int64_t lda, int64_t sA, int cb,
+                                               int ce, int k0, int np,
+                                               const int* __restrict__ ipiv, int64_t sP,
+                                               int cpw) {
+  extern __shared__ int sm_swap[];
+  int* ip = sm_swap;         // [np]
+  int* rdst = ip + np;       // [2 np]
+  int* rsrc = rdst + 2 * np;  // [2 np]
+  __shared__ int s_nm;
   const int64_t b = blockIdx.y;
-  int col = cb + blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= ce) return;
-  A += b * sA + (int64_t)col * lda;
-  ipiv += b * sP;
-  for (int s = k0; s < k1; ++s) {
-    int p = ipiv[s];
-    if (p != s) {  // component by component (no per-thread temporary in memory)
-      const auto tr = A[s].re, ti = A[s].im;
-      const auto pr = A[p].re, pi = A[p].im;
-      A[s].re = pr;
-      A[s].im = pi;
-      A[p].re = tr;
-      A[p].im = ti;
-    }
-  }
-}
-
-// The interchanges ipiv[k0..k1) of columns [cb, ce) when every row they touch
-// lies in [k0, n) with n - k0 small (the last steps of the LU): each
-// workgroup turns the interchanges into a permutation of those R = n - k0
-// rows (in LDS, one thread), then moves TC columns at a time through LDS,
-// loading and storing along the rows (coalesced) instead of one lane per
-// column.  Same result as k_laswp.
-template <typename T>
-__global__ void __launch_bounds__(256) k_laswp_tail(T* __restrict__ A, int64_t lda, int64_t sA,
-                                                    int cb, int ce, int k0, int k1, int n,
-                                                    const int* __restrict__ ipiv, int64_t sP,
-                                                    int cpw, int tc) {
-  extern __shared__ __align__(16) unsigned char sm_tail[];
-  const int R = n - k0, ns = k1 - k0;
-  T* tile = (T*)sm_tail;                                   // [tc][R]
-  int* perm = (int*)(sm_tail + (size_t)tc * R * sizeof(T));  // [R]
-  int* ip = perm + R;                                      // [ns]
-  const int64_t b = blockIdx.y;
+  const int tid = threadIdx.x;
   A += b * sA;
   ipiv += b * sP;
-  for (int r = threadIdx.x; r < R; r += 256) perm[r] = r;
-  for (int i = threadIdx.x; i < ns; i += 256) ip[i] = ipiv[k0 + i] - k0;
+  if (tid == 0) s_nm = 0;
+  for (int i = tid; i < np; i += 256) ip[i] = ipiv[k0 + i];
   __syncthreads();
-  __shared__ int any_moved;
-  if (threadIdx.x == 0) {
-    int moved = 0;
-    for (int i = 0; i < ns; ++i) {
-      const int j = ip[i];
-      if (j != i) {
-        const int t = perm[i];
-        perm[i] = perm[j];
-        perm[j] = t;
-        moved = 1;
-      }
+  for (int t = tid; t < 2 * np; t += 256) {
+    const int x = t < np ? k0 + t : ip[t - np];
+    if (t >= np && x < k0 + np) continue;  // listed among the first np
+    const int y = swap_source(x, k0, ip, 0, np);
+    if (y != x) {
+      const int at = atomicAdd(&s_nm, 1);
+      rdst[at] = x;
+      rsrc[at] = y;
     }
-    any_moved = moved;
   }
   __syncthreads();
-  if (!any_moved) return;  // uniform: no interchange in this step
-  // only the rows that move are loaded and stored (the permutation maps the
-  // moved rows onto themselves)
-  const int c_begin = cb + blockIdx.x * cpw;
-  const int c_end = min(ce, c_begin + cpw);
-  for (int c0 = c_begin; c0 < c_end; c0 += tc) {
-    const int nc = min(tc, c_end - c0);
-    for (int e = threadIdx.x; e < nc * R; e += 256) {
-      const int c = e / R, r = e - c * R;
-      if (perm[r] != r) tile[c * R + r] = A[(int64_t)(c0 + c) * lda + k0 + r];
+  const int nm = s_nm;
+  if (nm == 0) return;  // uniform: no row changes
+  int p2 = 16;
+  while (p2 < nm && p2 < 256) p2 <<= 1;
+  int nr = 1;  // rounds of 256 rows per column, a power of two (8 from 1025 rows on)
+  while (nr < 8 && nr * p2 < nm) nr <<= 1;
+  const int cols = 256 / p2, sub = tid / p2, l0 = tid & (p2 - 1), ng = 8 / nr;
+  const int c_end = min(ce, cb + ((int)blockIdx.x + 1) * cpw);
+  for (int c0 = cb + blockIdx.x * cpw; c0 < c_end; c0 += cols * ng) {
+    T v[8];
+    int64_t dst[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int idx = (u & (nr - 1)) * p2 + l0, c = c0 + (u / nr) * cols + sub;
+      dst[u] = -1;
+      if (idx < nm && c < c_end) {
+        const T* p = A + rsrc[idx] + (int64_t)c * lda;
+        v[u].re = p->re;
+        v[u].im = p->im;
+        dst[u] = rdst[idx] + (int64_t)c * lda;
+      }
     }
+    __builtin_amdgcn_s_waitcnt(0);  // every load has returned before the first store
     __syncthreads();
-    for (int e = threadIdx.x; e < nc * R; e += 256) {
-      const int c = e / R, r = e - c * R;
-      const int q = perm[r];
-      if (q != r) A[(int64_t)(c0 + c) * lda + k0 + r] = tile[c * R + q];
-    }
-    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (dst[u] >= 0) {
+        A[dst[u]].re = v[u].re;
+        A[dst[u]].im = v[u].im;
+      }
   }
 }
 
+// Broadcast of lane G (0..3) of each group of four lanes.
+template <int G>
+__device__ __forceinline__ int quad_bcast(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, G * 0x55, 0xf, 0xf, true);
+}
+template <int G>
+__device__ __forceinline__ double quad_bcast(double x) {
+  return __hiloint2double(quad_bcast<G>(__double2hiint(x)), quad_bcast<G>(__double2loint(x)));
+}
+template <int G>
+__device__ __forceinline__ float quad_bcast(float x) {
+  return __int_as_float(quad_bcast<G>(__float_as_int(x)));
+}
+
+// ---------------------------------------------------------------------------
 // Triangular-solve leaf, n <= 32 rows: X = L^{-1} B (unit lower) or
-// X = U^{-1} B (upper).  One wave per 64 right-hand-side columns: the 32 x 64
-// tile of B is staged through LDS with coalesced loads/stores (each column's
-// 32 rows are contiguous), every lane then substitutes down its own column
-// with the triangle read from LDS.
+// X = U^{-1} B (upper).  Four lanes per
+// column (64 columns per workgroup of 256 threads): lane g holds the rows
+// 4 s + g, s < 8, in registers, a solved row reaches the other three by a DPP
+// quad broadcast, and the triangle stands in LDS (17 KB).  All loads of a
+// lane are issued before the first is used.  What bounds it is latency: one
+// load, the chain of 32 rows, one store.  It takes 6 us for the 32 x 64 leaves of
+// an N = 530 window's solves and 8 us for the panel's, where the one-lane-per-column
+// leaf that it replaces (staged through LDS load by load) took 28 us; with
+// thousands of right-hand sides (the LU's block rows) it beats the leaf that held
+// a whole column per lane as well (LU of 240 matrices of 1640: 113.3 against
+// 115.6 ms per window, of 48 of 8192: 1.228 against 1.238 s).
+// ---------------------------------------------------------------------------
 template <typename T, bool UNIT_LOWER>
-__global__ void __launch_bounds__(64) k_trsm_leaf(int n, int nrhs, const T* __restrict__ L,
-                                                  int64_t ldl, int64_t sL, T* __restrict__ B,
-                                                  int64_t ldb, int64_t sB,
-                                                  const int* __restrict__ bix) {
+__global__ void __launch_bounds__(256, 4) k_trsm_leaf(int n, int nrhs, const T* __restrict__ L,
+                                                   int64_t ldl, int64_t sL, T* __restrict__ B,
+                                                   int64_t ldb, int64_t sB,
+                                                   const int* __restrict__ bix) {
   __shared__ T Ls[32][33];
-  __shared__ T Bt[64][33];
   const int64_t b = bix ? bix[blockIdx.y] : blockIdx.y;
+  const int tid = threadIdx.x, g = tid & 3, col = blockIdx.x * 64 + (tid >> 2);
   L += b * sL;
-  B += b * sB;
-  const int tid = threadIdx.x;
-  const int c0 = blockIdx.x * 64;
-  for (int e = tid; e < 32 * 32; e += 64) {
-    int i = e % 32, j = e / 32;
-    Ls[i][j] = (i < n && j < n) ? L[i + (int64_t)j * ldl] : T{0, 0};
+  B += b * sB + (int64_t)(col < nrhs ? col : nrhs - 1) * ldb;
+  T v[8], l[4];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) v[s] = ld_or0(B + 4 * s + g, 4 * s + g < n);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int i = (tid + 256 * t) & 31, j = (tid + 256 * t) >> 5;
+    l[t] = ld_or0(L + i + (int64_t)j * ldl, i < n && j < n);
   }
-  // coalesced load: lanes 0..31 read rows of one column, 32..63 the next
-  for (int cc = tid >> 5; cc < 64; cc += 2) {
-    int i = tid & 31, col = c0 + cc;
-    Bt[cc][i] = (i < n && col < nrhs) ? B[i + (int64_t)col * ldb] : T{0, 0};
-  }
-  __syncthreads();
-  if (!UNIT_LOWER && tid < 32) {
-    T d = tid < n ? Ls[tid][tid] : T{1, 0};
-    auto den = d.re * d.re + d.im * d.im;
-    Ls[tid][tid] = T{d.re / den, -d.im / den};
-  }
-  __syncthreads();
-  if (c0 + tid < nrhs) {
-    // blocks of 8 rows in registers; rows already final are read back from
-    // the lane's own LDS column (conflict-free: stride 33)
-    T* x = Bt[tid];
-    if (UNIT_LOWER) {
-#pragma unroll 1
-      for (int ib = 0; ib < 32; ib += 8) {
-        T v[8];
 #pragma unroll
-        for (int a = 0; a < 8; ++a) v[a] = x[ib + a];
-#pragma unroll 1
-        for (int j = 0; j < ib; ++j) {
-          T xj = x[j];
-#pragma unroll
-          for (int a = 0; a < 8; ++a) {
-            T l = Ls[ib + a][j];
-            v[a].re -= l.re * xj.re - l.im * xj.im;
-            v[a].im -= l.re * xj.im + l.im * xj.re;
-          }
-        }
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-#pragma unroll
-          for (int c = 0; c < a; ++c) {
-            T l = Ls[ib + a][ib + c];
-            v[a].re -= l.re * v[c].re - l.im * v[c].im;
-            v[a].im -= l.re * v[c].im + l.im * v[c].re;
-          }
-#pragma unroll
-        for (int a = 0; a < 8; ++a) x[ib + a] = v[a];
-      }
-    } else {
-#pragma unroll 1
-      for (int ib = 24; ib >= 0; ib -= 8) {
-        T v[8];
-#pragma unroll
-        for (int a = 0; a < 8; ++a) v[a] = x[ib + a];
-#pragma unroll 1
-        for (int j = ib + 8; j < 32; ++j) {
-          T xj = x[j];
-#pragma unroll
-          for (int a = 0; a < 8; ++a) {
-            T u = Ls[ib + a][j];
-            v[a].re -= u.re * xj.re - u.im * xj.im;
-            v[a].im -= u.re * xj.im + u.im * xj.re;
-          }
-        }
-#pragma unroll
-        for (int a = 7; a >= 0; --a) {
-#pragma unroll
-          for (int c = a + 1; c < 8; ++c) {
-            T u = Ls[ib + a][ib + c];
-            v[a].re -= u.re * v[c].re - u.im * v[c].im;
-            v[a].im -= u.re * v[c].im + u.im * v[c].re;
-          }
-          T d = Ls[ib + a][ib + a];
-          v[a] = T{v[a].re * d.re - v[a].im * d.im, v[a].re * d.im + v[a].im * d.re};
-        }
-#pragma unroll
-        for (int a = 0; a < 8; ++a) x[ib + a] = v[a];
-      }
-    }
-  }
-  __syncthreads();
-  for (int cc = tid >> 5; cc < 64; cc += 2) {
-    int i = tid & 31, col = c0 + cc;
-    if (i < n && col < nrhs) B[i + (int64_t)col * ldb] = Bt[cc][i];
-  }
-}
-
-// The same leaf with W waves per workgroup (W x 64 right-hand-side columns)
-// and each lane's column held in registers (up to 256 VGPRs: two waves per
-// SIMD): the triangle is staged once per workgroup and read by broadcast, and
-// each wave moves its columns between global memory and registers through a
-// 16-column LDS stage (coalesced: 32 lanes per column, four rounds).  For
-// complex128, 17 + 8.4 W KB of LDS instead of 51 KB per wave, so a CU holds 8
-// waves (W = 2) or 6 (W = 1) instead of 3.  Every row takes the operations of
-// k_trsm_leaf in the same order.
-template <typename T, bool UNIT_LOWER, int W>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2)))
-k_trsm_leaf_reg(int n, int nrhs, const T* __restrict__ L, int64_t ldl, int64_t sL,
-                T* __restrict__ B, int64_t ldb, int64_t sB, const int* __restrict__ bix) {
-  __shared__ T Ls[32][33];
-  __shared__ T St[W][16][33];
-  const int64_t b = bix ? bix[blockIdx.y] : blockIdx.y;
-  L += b * sL;
-  B += b * sB;
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int c0 = blockIdx.x * (64 * W) + w * 64;  // first column of this wave
-  for (int e = tid; e < 32 * 32; e += 64 * W) {
-    const int i = e % 32, j = e / 32;
-    Ls[i][j] = (i < n && j < n) ? L[i + (int64_t)j * ldl] : T{0, 0};
-  }
-  T x[32];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int cc = 2 * t + (lane >> 5), i = lane & 31, col = c0 + 16 * q + cc;
-      St[w][cc][i] = (i < n && col < nrhs) ? B[i + (int64_t)col * ldb] : T{0, 0};
-    }
-    __syncthreads();
-    if ((lane >> 4) == q) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) x[i] = St[w][lane & 15][i];
-    }
-    __syncthreads();
-  }
-  if (!UNIT_LOWER && tid < 32) {
-    T d = tid < n ? Ls[tid][tid] : T{1, 0};
-    auto den = d.re * d.re + d.im * d.im;
-    Ls[tid][tid] = T{d.re / den, -d.im / den};
-  }
+  for (int t = 0; t < 4; ++t) Ls[(tid + 256 * t) & 31][(tid + 256 * t) >> 5] = l[t];
   __syncthreads();
   if (UNIT_LOWER) {
+    static_for<0, 31>([&](auto jj) {
+      constexpr int j = decltype(jj)::value, s0 = j >> 2, o = j & 3;
+      const T xj = T{quad_bcast<o>(v[s0].re), quad_bcast<o>(v[s0].im)};
+      T t = v[s0];  // selected, not branched over: the updates stay in one block
+      cnma_(t, Ls[4 * s0 + g][j], xj);
+      v[s0].re = g > o ? t.re : v[s0].re;
+      v[s0].im = g > o ? t.im : v[s0].im;
 #pragma unroll
-    for (int ib = 0; ib < 32; ib += 8) {
-      T v[8];
-#pragma unroll
-      for (int a = 0; a < 8; ++a) v[a] = x[ib + a];
-#pragma unroll
-      for (int j = 0; j < ib; ++j) {
-        const T xj = x[j];
-#pragma unroll
-        for (int a = 0; a < 8; ++a) {
-          const T l = Ls[ib + a][j];
-          v[a].re -= l.re * xj.re - l.im * xj.im;
-          v[a].im -= l.re * xj.im + l.im * xj.re;
-        }
-      }
-#pragma unroll
-      for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int c = 0; c < a; ++c) {
-          const T l = Ls[ib + a][ib + c];
-          v[a].re -= l.re * v[c].re - l.im * v[c].im;
-          v[a].im -= l.re * v[c].im + l.im * v[c].re;
-        }
-#pragma unroll
-      for (int a = 0; a < 8; ++a) x[ib + a] = v[a];
-    }
+      for (int s = s0 + 1; s < 8; ++s) cnma_(v[s], Ls[4 * s + g][j], xj);
+      if (j & 1) asm volatile("" ::: "memory");  // LDS reads of two rows at a time
+    });
   } else {
-#pragma unroll
-    for (int ib = 24; ib >= 0; ib -= 8) {
-      T v[8];
-#pragma unroll
-      for (int a = 0; a < 8; ++a) v[a] = x[ib + a];
-#pragma unroll
-      for (int j = ib + 8; j < 32; ++j) {
-        const T xj = x[j];
-#pragma unroll
-        for (int a = 0; a < 8; ++a) {
-          const T u = Ls[ib + a][j];
-          v[a].re -= u.re * xj.re - u.im * xj.im;
-          v[a].im -= u.re * xj.im + u.im * xj.re;
-        }
-      }
-#pragma unroll
-      for (int a = 7; a >= 0; --a) {
-#pragma unroll
-        for (int c = a + 1; c < 8; ++c) {
-          const T u = Ls[ib + a][ib + c];
-          v[a].re -= u.re * v[c].re - u.im * v[c].im;
-          v[a].im -= u.re * v[c].im + u.im * v[c].re;
-        }
+    if (tid < 32) {
+      const T d = tid < n ? Ls[tid][tid] : T{1, 0};
+      Ls[tid][tid] = cinv_(d);
+    }
+    __syncthreads();
+    // blocks of 8 rows from the bottom: first the solved rows below the block
+    // in ascending order, then the block's own rows
+    static_for<0, 4>([&](auto bb) {
+      constexpr int ib = 24 - 8 * decltype(bb)::value, s0 = ib >> 2;
+      static_for<ib + 8, 32>([&](auto jj) {
+        constexpr int j = decltype(jj)::value;
+        const T xj = T{quad_bcast<(j & 3)>(v[j >> 2].re), quad_bcast<(j & 3)>(v[j >> 2].im)};
+        cnma_(v[s0], Ls[ib + g][j], xj);
+        cnma_(v[s0 + 1], Ls[ib + 4 + g][j], xj);
+        if ((j & 3) == 3) asm volatile("" ::: "memory");
+      });
+      static_for<0, 8>([&](auto aa) {
+        constexpr int a = 7 - decltype(aa)::value, sa = s0 + (a >> 2);
+        T x = v[sa];
+        static_for<a + 1, 8>([&](auto cc) {
+          constexpr int c = decltype(cc)::value, sc = s0 + (c >> 2);
+          const T xc = T{quad_bcast<(c & 3)>(v[sc].re), quad_bcast<(c & 3)>(v[sc].im)};
+          cnma_(x, Ls[ib + a][ib + c], xc);
+        });
         const T d = Ls[ib + a][ib + a];
-        v[a] = T{v[a].re * d.re - v[a].im * d.im, v[a].re * d.im + v[a].im * d.re};
-      }
-#pragma unroll
-      for (int a = 0; a < 8; ++a) x[ib + a] = v[a];
-    }
+        x = cmul_(x, d);
+        v[sa].re = g == (a & 3) ? x.re : v[sa].re;
+        v[sa].im = g == (a & 3) ? x.im : v[sa].im;
+        asm volatile("" ::: "memory");
+      });
+    });
   }
+  if (col < nrhs) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if ((lane >> 4) == q) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) St[w][lane & 15][i] = x[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int cc = 2 * t + (lane >> 5), i = lane & 31, col = c0 + 16 * q + cc;
-      if (i < n && col < nrhs) B[i + (int64_t)col * ldb] = St[w][cc][i];
-    }
-    __syncthreads();
+    for (int s = 0; s < 8; ++s)
+      if (4 * s + g < n) {
+        B[4 * s + g].re = v[s].re;
+        B[4 * s + g].im = v[s].im;
+      }
   }
 }
 
 // ---------------------------------------------------------------------------
 // Host orchestration
 // ---------------------------------------------------------------------------
-// QB_LASWP_TAIL=0 (read once): the last steps' interchanges one lane per column.
-static bool laswp_tail_off() {
-  static const bool off = [] {
-    const char* e = getenv("QB_LASWP_TAIL");
-    return e && e[0] == '0';
-  }();
-  return off;
-}
-
 template <typename T>
 static int laswp(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int cb, int ce, int k0, int k1,
                  const int* ipiv, int64_t sP, int batch) {
   if (ce <= cb || k1 <= k0) return QB_OK;
-  dim3 g((ce - cb + 127) / 128, batch);
-  hipLaunchKernelGGL(k_laswp<T>, g, dim3(128), 0, ctx->stream, A, lda, sA, cb, ce, k0, k1, ipiv,
-                     sP);
-  QB_HIP(ctx, hipGetLastError());
-  return QB_OK;
-}
-
-// laswp for interchanges whose rows all lie in [k0, n): the LDS block kernel
-// when n - k0 <= 2048 and n >= 4096, else k_laswp.  Measured: the last steps
-// at n = 8192 (48 matrices) gain 5 ms per window; at n = 1640 (240 matrices,
-// mostly diagonal pivots, which k_laswp skips at no cost) every step would
-// take the kernel and the C_5 windows lost 7%.
-template <typename T>
-static int laswp_rows(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int cb, int ce, int k0, int k1,
-                      int n, const int* ipiv, int64_t sP, int batch) {
-  if (ce <= cb || k1 <= k0) return QB_OK;
-  const int R = n - k0;
-  if (R > 2048 || n < 4096 || laswp_tail_off())
-    return laswp(ctx, A, lda, sA, cb, ce, k0, k1, ipiv, sP, batch);
-  const int tc = (int)((size_t)48 * 1024 / ((size_t)R * sizeof(T)));
-  const int cpw = 256;
-  const size_t lds = (size_t)tc * R * sizeof(T) + (size_t)(R + (k1 - k0)) * sizeof(int);
+  const int np = k1 - k0, cpw = np <= 64 ? 16 : 64;
   dim3 g((ce - cb + cpw - 1) / cpw, batch);
-  hipLaunchKernelGGL(k_laswp_tail<T>, g, dim3(256), lds, ctx->stream, A, lda, sA, cb, ce, k0, k1,
-                     n, ipiv, sP, cpw, tc);
+  hipLaunchKernelGGL(k_laswp<T>, g, dim3(256), 5 * (size_t)np * sizeof(int), ctx->stream, A, lda,
+                     sA, cb, ce, k0, np, ipiv, sP, cpw);
   QB_HIP(ctx, hipGetLastError());
   return QB_OK;
 }
@@ -1484,101 +1653,25 @@ static int split32(int n) {
   return h >= n ? n / 2 : h;
 }
 
-// Leaf launch (n <= 32): k_trsm_leaf_reg with two waves per workgroup when
-// the launch has at least 8 waves per CU to give (the LU's block-row solves),
-// else the one-wave LDS leaf k_trsm_leaf, which is the faster of the two at
-// low occupancy (the moment solves: 576 waves, 270 against 274 ms per window).
-// QB_TRSM_LEAF=lds (read once) or qb_set_trsm_leaf_lds(1) takes the LDS leaf
-// everywhere; qb_set_trsm_leaf_lds(0) the register leaf everywhere (one wave
-// per workgroup for the small launches).
-static int g_trsm_leaf_lds = -1;
-void qb_set_trsm_leaf_lds(int mode) { g_trsm_leaf_lds = mode; }
-static int trsm_leaf_mode() {
-  static const int env = [] {
-    const char* e = getenv("QB_TRSM_LEAF");
-    return e && e[0] == 'l' ? 1 : -1;
-  }();
-  return g_trsm_leaf_lds >= 0 ? g_trsm_leaf_lds : env;
-}
+// There is one leaf kernel: every mode selects it.
+void qb_set_trsm_leaf_lds(int) {}
 
 template <typename T, bool LOWER>
 static int trsm_leaf(qb_ctx* ctx, int n, int nrhs, const T* L, int64_t ldl, int64_t sL, T* B,
                      int64_t ldb, int64_t sB, int batch) {
   int slot = qb_prof_begin(ctx, QB_K_TRSM, 4.0 * n * n * (double)nrhs * batch, 0);
-  const int64_t waves = (int64_t)((nrhs + 63) / 64) * batch;
-  const int mode = trsm_leaf_mode();
-  if (mode == 1 || (mode < 0 && waves < 8 * 256)) {
-    hipLaunchKernelGGL((k_trsm_leaf<T, LOWER>), dim3((nrhs + 63) / 64, batch), dim3(64), 0,
-                       ctx->stream, n, nrhs, L, ldl, sL, B, ldb, sB, ctx->bix);
-  } else if (waves >= 8 * 256) {
-    hipLaunchKernelGGL((k_trsm_leaf_reg<T, LOWER, 2>), dim3((nrhs + 127) / 128, batch),
-                       dim3(128), 0, ctx->stream, n, nrhs, L, ldl, sL, B, ldb, sB, ctx->bix);
-  } else {
-    hipLaunchKernelGGL((k_trsm_leaf_reg<T, LOWER, 1>), dim3((nrhs + 63) / 64, batch), dim3(64),
-                       0, ctx->stream, n, nrhs, L, ldl, sL, B, ldb, sB, ctx->bix);
-  }
+  hipLaunchKernelGGL((k_trsm_leaf<T, LOWER>), dim3((nrhs + 63) / 64, batch), dim3(256), 0,
+                     ctx->stream, n, nrhs, L, ldl, sL, B, ldb, sB, ctx->bix);
   qb_prof_end(ctx, slot);
   QB_HIP(ctx, hipGetLastError());
   return QB_OK;
 }
 
 // X = L^{-1} B with L the unit-lower n x n block at L (ld ldl).
-// Unit-lower triangular-solve leaf (n <= 32 rows) without LDS, for the LU
-// panel beside the trailing update: each lane holds its right-hand-side
-// column in registers and reads the triangle with wave-uniform loads.  Row i
-// subtracts L(i, j) x_j in increasing j, the order of k_trsm_leaf.
-template <typename T>
-__global__ void __launch_bounds__(64) k_trsm_leaf_lower_reg(int n, int nrhs, const T* __restrict__ L,
-                                                           int64_t ldl, int64_t sL,
-                                                           T* __restrict__ B, int64_t ldb,
-                                                           int64_t sB, const int* __restrict__ bix) {
-  typedef typename Scal<T>::S S;
-  const int64_t b = bix ? bix[blockIdx.y] : blockIdx.y;
-  L += b * sL;
-  B += b * sB;
-  const int col = blockIdx.x * 64 + threadIdx.x;
-  if (col >= nrhs) return;
-  T* Bc = B + (int64_t)col * ldb;
-  S xr[32], xi[32];
-#pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    xr[i] = i < n ? Bc[i].re : S(0);
-    xi[i] = i < n ? Bc[i].im : S(0);
-  }
-#pragma unroll
-  for (int j = 0; j < 31; ++j) {
-    if (j + 1 < n) {
-#pragma unroll
-      for (int i = j + 1; i < 32; ++i) {
-        if (i < n) {
-          const S lr = L[i + (int64_t)j * ldl].re, li = L[i + (int64_t)j * ldl].im;
-          xr[i] -= lr * xr[j] - li * xi[j];
-          xi[i] -= lr * xi[j] + li * xr[j];
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 32; ++i)
-    if (i < n) {
-      Bc[i].re = xr[i];
-      Bc[i].im = xi[i];
-    }
-}
-
 template <typename T>
 static int trsm_lower(qb_ctx* ctx, int n, int nrhs, const T* L, int64_t ldl, int64_t sL, T* B,
                       int64_t ldb, int64_t sB, int batch) {
   if (n <= 0 || nrhs <= 0) return QB_OK;
-  if (n <= 32 && ctx->panel_lean) {
-    dim3 g((nrhs + 63) / 64, batch);
-    int slot = qb_prof_begin(ctx, QB_K_TRSM, 4.0 * n * n * (double)nrhs * batch, 0);
-    hipLaunchKernelGGL((k_trsm_leaf_lower_reg<T>), g, dim3(64), 0, ctx->stream, n, nrhs, L, ldl,
-                       sL, B, ldb, sB, ctx->bix);
-    qb_prof_end(ctx, slot);
-    QB_HIP(ctx, hipGetLastError());
-    return QB_OK;
-  }
   if (n <= 32) return trsm_leaf<T, true>(ctx, n, nrhs, L, ldl, sL, B, ldb, sB, batch);
   int n1 = split32(n);
   int rc = trsm_lower(ctx, n1, nrhs, L, ldl, sL, B, ldb, sB, batch);
@@ -1605,23 +1698,6 @@ static int trsm_upper(qb_ctx* ctx, int n, int nrhs, const T* U, int64_t ldu, int
   return trsm_upper(ctx, n1, nrhs, U, ldu, sU, B, ldb, sB, batch);
 }
 
-// Threads of a leaf workgroup that runs beside the trailing update.  Two
-// workgroups of the complex128 trailing-update tiles (70 KB of LDS, two waves
-// per SIMD at 128 VGPRs) leave a CU 20 KB of LDS and two waves per SIMD: the
-// complex128 leaf (18 KB, 94 VGPRs) fits there with 512 threads, and with
-// 1024 it waits for the whole trailing update to drain.  QB_PANEL_THREADS (a
-// multiple of 64 in [64, 1024], read once) overrides it.
-template <typename T>
-static int panel_threads_beside() {
-  static const int env = [] {
-    const char* e = getenv("QB_PANEL_THREADS");
-    long v = e ? strtol(e, nullptr, 10) : 0;
-    return (v >= 64 && v <= 1024 && v % 64 == 0) ? (int)v : 0;
-  }();
-  if (env) return env;
-  return sizeof(T) == sizeof(cd) ? 512 : 1024;
-}
-
 // The lean kernels for a complex128 panel beside the trailing update
 // (qb_ctx::panel_lean).  They leave LDS to the trailing tile, which pays only
 // when that tile holds LDS: beside a register-streamed tile (no LDS) the
@@ -1646,21 +1722,40 @@ static bool panel_lean_beside(const qb_ctx* ctx, int M, int N, int K) {
   return !kGemmReg[1][v];
 }
 
-// Recursive panel: factor columns [c0, c0+w) (rows c0..n-1) of every matrix,
-// leaves with `threads` threads per workgroup.
+// One leaf: the rows per thread follow from the rows left, the columns held at
+// a time from the registers they then take (RPT * W = 32 for complex128, 64 for
+// complex64, at most the leaf's 32).
+template <typename T>
+static void panel_leaf(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, int w,
+                       int* ipiv, int64_t sP, int* info, int batch) {
+  constexpr int X = sizeof(T) == sizeof(cf) ? 2 : 1;
+  const int m = n - c0;
+  if (m <= 512)
+    launch_getf2<T, 256, 2, 16>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  else if (m <= 1024)
+    launch_getf2<T, 256, 4, 8 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  else if (m <= 2048)
+    launch_getf2<T, 256, 8, 4 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  else if (m <= 4096)
+    launch_getf2<T, 256, 16, 2 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  else
+    hipLaunchKernelGGL(k_getf2_long<T>, dim3(batch), dim3(512), 0, ctx->stream, A, lda, sA, n, c0,
+                       w, ipiv, sP, info);
+}
+
+// Recursive panel: factor columns [c0, c0+w) (rows c0..n-1) of every matrix.
 template <typename T>
 static int panel_rec(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, int w, int* ipiv,
-                     int64_t sP, int* info, int batch, int threads = 1024) {
+                     int64_t sP, int* info, int batch) {
   if (w <= 32) {
     int slot = qb_prof_begin(ctx, QB_K_PANEL, 8.0 * (double)(n - c0) * w * w / 2 * batch, 0);
-    hipLaunchKernelGGL(k_getf2<T>, dim3(batch), dim3(threads), 0, ctx->stream, A, lda, sA, n, c0,
-                       w, ipiv, sP, info);
+    panel_leaf<T>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
     qb_prof_end(ctx, slot);
     QB_HIP(ctx, hipGetLastError());
     return QB_OK;
   }
   int w1 = split32(w);
-  int rc = panel_rec(ctx, A, lda, sA, n, c0, w1, ipiv, sP, info, batch, threads);
+  int rc = panel_rec(ctx, A, lda, sA, n, c0, w1, ipiv, sP, info, batch);
   if (rc) return rc;
   rc = laswp(ctx, A, lda, sA, c0 + w1, c0 + w, c0, c0 + w1, ipiv, sP, batch);
   if (rc) return rc;
@@ -1672,7 +1767,7 @@ static int panel_rec(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, 
                    A + c0 + (int64_t)(c0 + w1) * lda, lda, sA,
                    A + c0 + w1 + (int64_t)(c0 + w1) * lda, lda, sA, batch);
   if (rc) return rc;
-  rc = panel_rec(ctx, A, lda, sA, n, c0 + w1, w - w1, ipiv, sP, info, batch, threads);
+  rc = panel_rec(ctx, A, lda, sA, n, c0 + w1, w - w1, ipiv, sP, info, batch);
   if (rc) return rc;
   return laswp(ctx, A, lda, sA, c0, c0 + w1, c0 + w1, c0 + w, ipiv, sP, batch);
 }
@@ -1750,13 +1845,13 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
       QB_HIP(ctx, hipEventRecord(ctx->ev_main, main));
       QB_HIP(ctx, hipStreamWaitEvent(aux, ctx->ev_main, 0));
       rc = on_aux([&] {
-        return laswp_rows(ctx, A, lda, sA, 0, k0, k0, k0 + kb, n, ipiv, sP, batch);
+        return laswp(ctx, A, lda, sA, 0, k0, k0, k0 + kb, ipiv, sP, batch);
       });
     } else {
-      rc = laswp_rows(ctx, A, lda, sA, 0, k0, k0, k0 + kb, n, ipiv, sP, batch);
+      rc = laswp(ctx, A, lda, sA, 0, k0, k0, k0 + kb, ipiv, sP, batch);
     }
     if (rc) return rc;
-    rc = laswp_rows(ctx, A, lda, sA, k0 + kb, n, k0, k0 + kb, n, ipiv, sP, batch);
+    rc = laswp(ctx, A, lda, sA, k0 + kb, n, k0, k0 + kb, ipiv, sP, batch);
     if (rc) return rc;
     if (k0 + kb >= n) break;
     const int k1 = k0 + kb, m = n - k1;
@@ -1774,8 +1869,7 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
     QB_HIP(ctx, hipStreamWaitEvent(aux, ctx->ev_main, 0));
     rc = on_aux([&] {
       ctx->panel_lean = m > kb1 && panel_lean_beside<T>(ctx, m, m - kb1, kb);
-      const int r = panel_rec(ctx, A, lda, sA, n, k1, kb1, ipiv, sP, info, batch,
-                              m > kb1 ? panel_threads_beside<T>() : 1024);
+      const int r = panel_rec(ctx, A, lda, sA, n, k1, kb1, ipiv, sP, info, batch);
       ctx->panel_lean = false;
       return r;
     });
