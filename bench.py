@@ -35,8 +35,9 @@ import numpy as np  # noqa: E402
 PEAK = {"c64": 157.3, "c128": 78.6, "i8": 5000.0}  # dense MFMA TFLOP/s (fp32, fp64), int8 TOPS
 # HBM bytes per GEMM launch over the windows of the default workload, from
 # FETCH_SIZE / WRITE_SIZE counter runs scaled by a copy kernel of known size
-# (profiles/beyn_window_star_N8192_pmc_traffic.txt)
-TRAFFIC_PER_LAUNCH = {"c128": 1664.7e6, "c64": 467.3e6}
+# (profiles/beyn_window_star_N8192_pmc_traffic.txt; its c128 figure is of the
+# launches before the LU's trailing updates left for the int8 matrix cores)
+TRAFFIC_PER_LAUNCH = {"c64": 467.3e6}
 
 
 def parse():
@@ -833,8 +834,9 @@ def main():
                           if len(sums) == 2 else None),
         "kernels": hs["kernels"],
         "gemm_autotune": [l for l in rep.splitlines() if l],
-        "roofline": {"kernel": ("k_gemm_sub<complex128>, every launch of the window (LU "
-                                "updates, triangular solves, QR; FP64 MFMA)"
+        "roofline": {"kernel": ("k_gemm_sub<complex128>, every launch of the window "
+                                "(panels, triangular solves, QR; FP64 MFMA; the LU's "
+                                "int8 updates are kernels.gemm_c128_i8)"
                                 if best == "fp64" else
                                 "k_gemm_sub<complex64> + k_gemm_bf6, every launch of the "
                                 "window (LU updates, triangular solves; MFMA)"),

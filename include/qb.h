@@ -106,6 +106,13 @@ int64_t qb_ctx_device_bytes(const qb_ctx* ctx);
  * Off by default.  No reference counterpart. */
 int qb_ctx_set_graphs(qb_ctx* ctx, int32_t on);
 
+/* Let large FP64 factorisations take residue buffers for the time of the LU
+ * (on by default): their trailing updates then run on the int8 matrix cores,
+ * at FP64 accuracy and about 1.4 times the speed of the FP64 ones.  Off, or
+ * where the buffers do not fit, they run on the FP64 matrix cores.  No
+ * reference counterpart. */
+int qb_ctx_set_residue_buffers(qb_ctx* ctx, int32_t on);
+
 /* Free and total device memory of the context's GPU (hipMemGetInfo); the
  * serving loop sizes its admission budget from it.  No reference
  * counterpart. */
@@ -130,7 +137,8 @@ enum {
   QB_K_OTHER = 6,     /* swaps, gathers, norms, moments        */
   QB_K_OZAKI = 7,     /* int8 products of the refinement residual (MFMA) */
   QB_K_GEMM_C64_BF16 = 8, /* complex64 C -= A*B on bf16 MFMA (split operands) */
-  QB_K_COUNT = 9
+  QB_K_GEMM_C128_I8 = 9,  /* complex128 C -= A*B on int8 MFMA (residues) */
+  QB_K_COUNT = 10
 };
 /* Enable (1) / disable (0) recording a pair of HIP events on the context's
  * stream around every launch, and clear the counters.  No counterpart in the
@@ -148,7 +156,9 @@ int qb_ctx_kernel_stats(qb_ctx* ctx, int32_t kind, double* total_ms, int64_t* la
  * three-product (Gauss) tiles and 8 M N K otherwise (the algorithmic count
  * of qb_ctx_kernel_stats is always 8 M N K); for QB_K_OZAKI the int8
  * operations of the padded products as launched; for QB_K_GEMM_C64_BF16 the
- * bf16 operations (48 M N K: 4 real products of 6 split products each).  No
+ * bf16 operations (48 M N K: 4 real products of 6 split products each); for
+ * QB_K_GEMM_C128_I8 the int8 operations (64 M N K: 2 products for each of 16
+ * moduli).  No
  * reference counterpart. */
 int qb_ctx_kernel_issued(qb_ctx* ctx, int32_t kind, double* issued);
 
@@ -284,9 +294,12 @@ int32_t qb_window_blocks(const qb_window* w);
 int qb_window_matrix_cols(qb_window* w, int32_t node, int64_t j0, int64_t ncols, double* out);
 void qb_window_destroy(qb_window* w);
 /* Device bytes a window of this size would hold (the admission footprint):
- * matrices, pivots, solve buffers for r probes, and up to 32 MiB of tables
- * per node. */
+ * matrices, pivots, solve buffers for r probes or the residue buffers of the
+ * LU before them (the larger), and up to 32 MiB of tables per node. */
 int64_t qb_window_footprint(int64_t N, int32_t nq, int32_t precision, int32_t r);
+/* The part of it that a context without residue buffers
+ * (qb_ctx_set_residue_buffers) does not need. */
+int64_t qb_window_residue_extra(int64_t N, int32_t nq, int32_t precision, int32_t r);
 
 /* The moment loop of construct_B_matrix (beyn.jl:278-285): X_j = T(z_j)^{-1} V,
  * A0 = sum_j w_j X_j, A1 = sum_j w_j z_j X_j, w_j = (R/nq) e^{i 2pi j/nq}.

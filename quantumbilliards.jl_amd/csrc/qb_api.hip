@@ -261,6 +261,12 @@ int qb_ctx_set_cache_limit(qb_ctx* ctx, int64_t bytes) {
   return QB_OK;
 }
 
+int qb_ctx_set_residue_buffers(qb_ctx* ctx, int32_t on) {
+  if (!ctx) return QB_E_ARG;
+  ctx->residues = on != 0;
+  return QB_OK;
+}
+
 int qb_ctx_set_profiling(qb_ctx* ctx, int32_t enable) {
   if (!ctx) return QB_E_ARG;
   (void)hipSetDevice(ctx->device);
@@ -1035,18 +1041,30 @@ static size_t win_bytes_core(int64_t N, int nq, int precision) {
   return b;
 }
 
-extern "C" int64_t qb_window_footprint(int64_t N, int32_t nq, int32_t precision, int32_t r) {
-  size_t b = win_bytes_core(N, nq, precision);
-  size_t nv = (size_t)N * r;
-  // moment work buffers: X and R (complex128) per node, a complex64 copy
-  // per node in mixed mode, V, A0, A1, and the QR block [A0 | A1] that
-  // qb_window_moments_qr keeps
-  b += 2 * (size_t)nq * nv * sizeof(cd) + 5 * nv * sizeof(cd);
+// moment work buffers: X and R (complex128) per node, a complex64 copy
+// per node in mixed mode, V, A0, A1, and the QR block [A0 | A1] that
+// qb_window_moments_qr keeps
+static size_t win_bytes_moments(int64_t N, int nq, int precision, int r) {
+  const size_t nv = (size_t)N * r;
+  size_t b = 2 * (size_t)nq * nv * sizeof(cd) + 5 * nv * sizeof(cd);
   if (precision == QB_MIXED || precision == QB_MIXED_INT8RES) {
     b += (size_t)nq * nv * sizeof(cf);
     if (oz_enabled(precision, N))
       b += qb_oz_step_bytes(N, r, nq < QB_OZ_SLOTS ? nq : QB_OZ_SLOTS);
   }
+  return b;
+}
+
+extern "C" int64_t qb_window_residue_extra(int64_t N, int32_t nq, int32_t precision, int32_t r) {
+  // the LU has given its residue buffers back when the moments begin
+  if (precision != QB_FP64) return 0;
+  const int64_t e = qb_getrf_rns_bytes(N, nq) - (int64_t)win_bytes_moments(N, nq, precision, r);
+  return e > 0 ? e : 0;
+}
+
+extern "C" int64_t qb_window_footprint(int64_t N, int32_t nq, int32_t precision, int32_t r) {
+  size_t b = win_bytes_core(N, nq, precision) + win_bytes_moments(N, nq, precision, r) +
+             (size_t)qb_window_residue_extra(N, nq, precision, r);
   // Chebyshev tables, bounded by 1.2e5 panels of degree 7 per node
   b += (size_t)nq * (32u << 20);
   return (int64_t)b;

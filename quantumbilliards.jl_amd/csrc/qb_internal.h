@@ -87,6 +87,7 @@ struct qb_ctx {
   // keyed by operand type, buffers and shape; gemm_epoch changes whenever the
   // autotuner changes a tile pick, so stale captures are not replayed.
   bool graphs = false;
+  bool residues = true;  // LUs may take residue buffers (qb_ctx_set_residue_buffers)
   uint64_t gemm_epoch = 0;
   struct GraphRec {
     int ty;

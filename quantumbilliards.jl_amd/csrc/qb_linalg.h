@@ -26,6 +26,8 @@ template <typename T>
 int qb_getrf_first_panel(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipiv,
                          int64_t sP, int* info, int batch);
 int qb_lu_nb(int n);
+// Residue buffers that qb_getrf_batched<cd> takes for the time of its call.
+int64_t qb_getrf_rns_bytes(int64_t n, int batch);
 // qb_getrf_batched through a cached hipGraph when ctx->graphs is set and
 // launch accounting is off: the first call with given buffers captures the
 // launch sequence (both streams) and instantiates it, later calls replay it.
@@ -42,6 +44,26 @@ void qb_set_trsm_leaf_lds(int mode);
 template <typename T>
 int qb_trsm_lu_batched(qb_ctx* ctx, const T* LU, int n, int64_t lda, int64_t sA, T* B, int nrhs,
                        int64_t ldb, int64_t sB, int batch);
+
+// complex128 C[b] -= A[b] B[b] on the int8 matrix cores (qb_rns.hip) for inner
+// dimension 512.  qb_rns_open takes the residue buffers for up to M x 512 and 512 x N
+// operands of `batch` matrices (QB_E_NOMEM: no room, nothing changed);
+// qb_rns_set_a slices the A operands (of ctx->bix's matrices when set), after
+// which qb_rns_sub subtracts their products with any number of B's.  All on
+// ctx->stream.
+struct QbRns {
+  signed char *mem = nullptr, *A = nullptr, *B = nullptr;
+  double *scA = nullptr, *scB = nullptr;
+  int64_t strideA = 0, strideB = 0, maxM = 0, maxN = 0;
+  size_t bytes = 0;
+  int batch = 0, nb = 0, M = 0;
+};
+int64_t qb_rns_bytes(int64_t M, int64_t N, int batch);
+int qb_rns_open(qb_ctx* ctx, QbRns* h, int64_t M, int64_t N, int batch);
+int qb_rns_set_a(qb_ctx* ctx, QbRns* h, int M, const cd* A, int64_t lda, int64_t sA);
+int qb_rns_sub(qb_ctx* ctx, QbRns* h, int N, const cd* B, int64_t ldb, int64_t sB, cd* C,
+               int64_t ldc, int64_t sC);
+void qb_rns_close(qb_ctx* ctx, QbRns* h);
 
 int qb_perm_from_ipiv(qb_ctx* ctx, const int* ipiv, int* perm, int n, int batch);
 // dst[b][i + c*n] = src[(b*sb)][perm[b][i] + c*n] for a permuted broadcast /

@@ -1063,10 +1063,12 @@ __device__ __forceinline__ int swap_source(int x, int k0, const int* p, int kb, 
 // a trailing-update workgroup that ends; eight waited for both of a CU's.  The leaf that this one replaces kept its columns in
 // global memory (one workgroup too) and took, on average over the leaves of an
 // N = 530 and an N = 1792 window (32 matrices), 172 and 254 us; this one takes 90
-// and 93 (up to 512 rows), 106 (1024) and 185 us (2048).  From 4096 rows on it
-// would hold one column at a time, read as much as the leaf in global memory does
-// with fewer loads in flight, and lose to it (5.6 against 1.25 ms beside the
-// trailing update of 8192 x 8192): k_getf2_long takes those.
+// and 93 (up to 512 rows), 106 (1024) and 185 us (2048).  Up to 8192 rows eight
+// waves hold two complex128 columns at a time; beside the residue updates
+// (qb_rns.hip), whose workgroups end every 74 us, they take 0.99 ms per leaf of an
+// N = 8192 window (48 matrices), k_getf2_long 2.56 ms there (window: 1019 against
+// 1043 ms).  k_getf2_long takes longer columns, and complex64 ones above 4096 rows,
+// which run beside the FP32 tiles: there the eight waves wait for room.
 // ---------------------------------------------------------------------------
 template <typename T, int NT, int RPT, int W>
 __global__ void __launch_bounds__(NT) k_getf2(T* __restrict__ A, int64_t lda, int64_t sA, int n,
@@ -1738,6 +1740,8 @@ static void panel_leaf(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0
     launch_getf2<T, 256, 8, 4 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
   else if (m <= 4096)
     launch_getf2<T, 256, 16, 2 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  else if (m <= 8192 && sizeof(T) == sizeof(cd))
+    launch_getf2<T, 512, 16, 2 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
   else
     hipLaunchKernelGGL(k_getf2_long<T>, dim3(batch), dim3(512), 0, ctx->stream, A, lda, sA, n, c0,
                        w, ipiv, sP, info);
@@ -1812,6 +1816,19 @@ int qb_getrf_first_panel(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int*
   return QB_OK;
 }
 
+// The complex128 trailing updates that run on the int8 matrix cores (qb_rns.hip):
+// steps of the full panel width of 512 with at least kRnsMin rows left.  An
+// update takes 33 to 36 ps per entry there against 48.8 ps, and its slices 12.5
+// ps for each of 512 (M + N) elements: at 1024 rows the two meet.  Matrices
+// below 4096 rows have panels of 256 columns, where the residues gain nothing,
+// and panels of 512 cost them what the updates would win (1141 rows: 12.8 ms for
+// a window of 32 matrices against 12.4, 1792 rows: 24.6 against 24.1).
+static const int kRnsMin = 1024;
+static bool lu_rns(int n) { return qb_lu_nb(n) == 512 && n - 512 >= kRnsMin; }
+int64_t qb_getrf_rns_bytes(int64_t n, int batch) {
+  return lu_rns((int)n) ? qb_rns_bytes(n - 512, n - 512, batch) : 0;
+}
+
 template <typename T>
 int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipiv, int64_t sP,
                      int* info, int batch, bool first_done) {
@@ -1834,6 +1851,18 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
   else
     rc = panel_rec(ctx, A, lda, sA, n, 0, n < NB ? n : NB, ipiv, sP, info, batch);
   if (rc) return rc;
+  // Residue buffers of the complex128 trailing updates; without room for them,
+  // and under capture (no allocation there), every update takes the FP64 tiles.
+  QbRns rns;
+  bool use_rns = false;
+  if constexpr (sizeof(T) == sizeof(cd))
+    use_rns = lu_rns(n) && ctx->residues && !ctx->graphs &&
+              qb_rns_open(ctx, &rns, n - NB, n - NB, batch) == QB_OK;
+  struct Close {  // on every way out
+    qb_ctx* ctx;
+    QbRns* h;
+    ~Close() { qb_rns_close(ctx, h); }
+  } close_rns{ctx, &rns};
   // The interchanges of step s in the columns left of its panel (the L part
   // of earlier panels) run on the auxiliary stream, ahead of the next panel:
   // nothing on the main stream touches those columns any more once the
@@ -1862,8 +1891,17 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
     rc = trsm_lower(ctx, kb, m, A11, lda, sA, A12, lda, sA, batch);
     if (rc) return rc;
     // next panel's columns first
-    rc = gemm_sub<T>(ctx, m, kb1, kb, A21, lda, sA, A12, lda, sA, A + k1 + (int64_t)k1 * lda, lda,
-                     sA, batch);
+    const bool rns_step = use_rns && kb == NB && m >= kRnsMin;
+    if constexpr (sizeof(T) == sizeof(cd)) {
+      if (rns_step) {
+        rc = qb_rns_set_a(ctx, &rns, m, A21, lda, sA);
+        if (!rc)
+          rc = qb_rns_sub(ctx, &rns, kb1, A12, lda, sA, A + k1 + (int64_t)k1 * lda, lda, sA);
+      }
+    }
+    if (!rns_step)
+      rc = gemm_sub<T>(ctx, m, kb1, kb, A21, lda, sA, A12, lda, sA, A + k1 + (int64_t)k1 * lda,
+                       lda, sA, batch);
     if (rc) return rc;
     QB_HIP(ctx, hipEventRecord(ctx->ev_main, main));
     QB_HIP(ctx, hipStreamWaitEvent(aux, ctx->ev_main, 0));
@@ -1877,8 +1915,14 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
     QB_HIP(ctx, hipEventRecord(ctx->ev_aux, aux));
     if (m > kb1) {
       ctx->gemm_conc = true;  // beside the panel on the second stream
-      rc = gemm_sub<T>(ctx, m, m - kb1, kb, A21, lda, sA, A12 + (int64_t)kb1 * lda, lda, sA,
-                       A + k1 + (int64_t)(k1 + kb1) * lda, lda, sA, batch);
+      if constexpr (sizeof(T) == sizeof(cd)) {
+        if (rns_step)
+          rc = qb_rns_sub(ctx, &rns, m - kb1, A12 + (int64_t)kb1 * lda, lda, sA,
+                          A + k1 + (int64_t)(k1 + kb1) * lda, lda, sA);
+      }
+      if (!rns_step)
+        rc = gemm_sub<T>(ctx, m, m - kb1, kb, A21, lda, sA, A12 + (int64_t)kb1 * lda, lda, sA,
+                         A + k1 + (int64_t)(k1 + kb1) * lda, lda, sA, batch);
       ctx->gemm_conc = false;
       if (rc) return rc;
     }

@@ -30,10 +30,11 @@ EXPORTS = (
     "qb_geom_set_orbits", "qb_geom_dim", "qb_host_alloc", "qb_host_free",
     "qb_geom_set_orbits_multi", "qb_geom_irreps", "qb_window_basis_irrep",
     "qb_window_create_multi", "qb_window_blocks", "qb_window_matrix_cols",
-    "qb_ctx_kernel_issued", "qb_assemble_noalloc",
+    "qb_ctx_kernel_issued", "qb_assemble_noalloc", "qb_ctx_set_residue_buffers",
+    "qb_window_residue_extra",
 )
 KERNEL_CLASSES = ("tables", "assemble", "gemm_c64", "gemm_c128", "panel", "trsm", "other",
-                  "ozaki", "gemm_c64_bf16")
+                  "ozaki", "gemm_c64_bf16", "gemm_c128_i8")
 
 
 class QBError(RuntimeError):
@@ -115,6 +116,8 @@ def lib():
         "qb_ctx_set_profiling": (C.c_int, [P, I32]),
         "qb_ctx_autotune": (C.c_int, [P, I64, I32, I32, I32, C.c_char_p, I64]),
         "qb_ctx_set_cache_limit": (C.c_int, [P, I64]),
+        "qb_ctx_set_residue_buffers": (C.c_int, [P, I32]),
+        "qb_window_residue_extra": (I64, [I64, I32, I32, I32]),
         "qb_ctx_mem_info": (C.c_int, [P, C.POINTER(I64), C.POINTER(I64)]),
         "qb_ctx_set_graphs": (C.c_int, [P, I32]),
         "qb_residuals": (C.c_int, [P, P, I32, P, I64, C.POINTER(ChebParams), P, I32, P, P, P, P,

@@ -164,9 +164,13 @@ class Window:
             pass
 
 
-def footprint(N: int, nq: int, precision: str = "fp64", r: int = 64) -> int:
-    """Device bytes of one window (the admission footprint of the serving loop)."""
-    return int(_lib.lib().qb_window_footprint(int(N), int(nq), _PREC[precision], int(r)))
+def footprint(N: int, nq: int, precision: str = "fp64", r: int = 64,
+              residues: bool = True) -> int:
+    """Device bytes of one window (the admission footprint of the serving loop);
+    residues=False: on a context whose LUs take no residue buffers."""
+    a = (int(N), int(nq), _PREC[precision], int(r))
+    b = int(_lib.lib().qb_window_footprint(*a))
+    return b if residues else b - int(_lib.lib().qb_window_residue_extra(*a))
 
 
 def _svd_B(A0, A1, svd_tol):

@@ -55,6 +55,10 @@ class Context:
         """Bytes of freed device buffers kept for reuse (0 disables caching)."""
         _lib.check(self.ptr, _lib.lib().qb_ctx_set_cache_limit(self.ptr, int(nbytes)))
 
+    def set_residue_buffers(self, on: bool):
+        """Whether large FP64 LUs may take residue buffers (int8 matrix cores)."""
+        _lib.check(self.ptr, _lib.lib().qb_ctx_set_residue_buffers(self.ptr, 1 if on else 0))
+
     def autotune(self, N: int, nq: int, r: int, precision: str = "mixed") -> str:
         """Pick GEMM tile variants for the shapes of an (N, nq, r) window
         (qb_ctx_autotune); returns the report."""

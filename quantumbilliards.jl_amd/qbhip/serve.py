@@ -340,6 +340,13 @@ class Server:
                 if fa <= self.budget:
                     prec, fp = alt, fa
                     break
+        if fp > self.budget:
+            # an FP64 window then factors on the FP64 matrix cores alone
+            for alt in (prec, "fp64"):
+                fa = footprint(N, nm, alt, r, residues=False)
+                if fa <= self.budget:
+                    prec, fp = alt, fa
+                    break
         return b, Ns, N, r, fp, prec
 
     def _dispatch(self):
@@ -447,6 +454,7 @@ class Server:
             # assembled and factored (the C calls release the interpreter)
             vf = self.host_pool.submit(probe_block, np.random.default_rng(req.seed), N, r)
             tw = time.perf_counter()
+            ctx.set_residue_buffers(fp >= footprint(N, req.nq * nirr * len(reqs), prec, r))
             if len(reqs) == 1:
                 win = Window(solver, pts, req.k0, req.R, req.nq, precision=prec, geom=geom,
                              **cheb)
@@ -472,7 +480,8 @@ class Server:
                 if r2 > GROW_LIMIT * max(r, 64):
                     saturated = True
                     break
-                extra = footprint(N, req.nq * nirr * len(reqs), prec, r2) - fp
+                extra = max(0, footprint(N, req.nq * nirr * len(reqs), prec, r2,
+                                         residues=False) - fp)
                 if r2 == r_used or not self._reserve(extra):
                     saturated = True
                     break
