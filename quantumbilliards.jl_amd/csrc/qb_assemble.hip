@@ -486,8 +486,7 @@ int qb_assemble_conj_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host
 #define QB_ENV_PMAX 128  // 32 octaves
 
 struct EnvLob {
-  double t[QB_ENV_NC];                 // cospi(j / M)
-  double C[QB_ENV_NC * QB_ENV_NC];     // C[m (M+1) + j] = cospi(j m / M)
+  double t[QB_ENV_NC];  // cospi(j / M)
 };
 
 // Quarter-octave panel p (0-based from octave o0) and local coordinate t of r.
@@ -502,23 +501,31 @@ __device__ __forceinline__ void env_panel(double r, int o0, int P, int* p, doubl
   *t = 8.0 * m - (9.0 + 2.0 * q);
 }
 
-// Envelope tables: one thread per (wavenumber, panel); coefficients of the
-// interpolant at the M+1 Lobatto points (DCT-I with c_0 and c_M halved),
-// E_0 and E_1 interleaved: env[((q P + p) (M+1) + m) 2 + {0, 1}].
+// Envelope tables: coefficients of the interpolant at the M+1 Lobatto points
+// (DCT-I with c_0 and c_M halved), E_0 and E_1 interleaved:
+// env[((q P + p) (M+1) + m) 2 + {0, 1}].  A lane evaluates one point, a wave
+// four panels, and turns from its point to its coefficient through LDS.  What
+// bounds it: one evaluation's serial arithmetic; one thread per panel did 13 in
+// a row (ellipse of 530 nodes, 32 wavenumbers: 355 -> 23 us).
+#define QB_ENV_PPW (64 / QB_ENV_NC)  // panels per wave
+
 __global__ __launch_bounds__(64) void k_env_tables(const cd* __restrict__ zk, int64_t nz, int o0,
                                                    int P, EnvLob lc, cd* __restrict__ env) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= nz * (int64_t)P) return;
-  const int64_t q = gid / P;
-  const int p = (int)(gid - q * P);
-  const int oct = o0 + p / 4, qq = p % 4;
-  const double a = ldexp(1.0 + 0.25 * qq, oct), b = ldexp(1.25 + 0.25 * qq, oct);
-  const double c = 0.5 * (a + b), h = 0.5 * (b - a);
-  const cd k = zk[q];
-  cd f0[QB_ENV_NC], f1[QB_ENV_NC];
-#pragma unroll
-  for (int j = 0; j < QB_ENV_NC; ++j) {
-    const double r = fma(h, lc.t[j], c);
+  __shared__ cd f0[64], f1[64];
+  __shared__ double ct[QB_ENV_NC];
+  const int lane = threadIdx.x, pl = lane / QB_ENV_NC, j = lane - pl * QB_ENV_NC;
+  const int64_t gid = (int64_t)blockIdx.x * QB_ENV_PPW + pl;
+  const bool on = pl < QB_ENV_PPW && gid < nz * (int64_t)P;
+  if (lane < QB_ENV_NC) ct[lane] = lc.t[lane];
+  __syncthreads();
+  if (on) {
+    const int64_t q = gid / P;
+    const int p = (int)(gid - q * P);
+    const int oct = o0 + p / 4, qq = p % 4;
+    const double a = ldexp(1.0 + 0.25 * qq, oct), b = ldexp(1.25 + 0.25 * qq, oct);
+    const double c = 0.5 * (a + b), h = 0.5 * (b - a);
+    const double r = fma(h, ct[j], c);
+    const cd k = zk[q];
     const cd z = mk(k.re * r, k.im * r);
     cd h0, h1;
     qb_hankel1_01(z, &h0, &h1);
@@ -526,25 +533,27 @@ __global__ __launch_bounds__(64) void k_env_tables(const cd* __restrict__ zk, in
     sincos(z.re, &sn, &cs);
     const double g = exp(z.im);
     const cd e = mk(cs * g, -sn * g);  // e^{-i z}
-    f0[j] = h0 * e;
-    f1[j] = h1 * e;
+    f0[lane] = h0 * e;
+    f1[lane] = h1 * e;
   }
-  cd* o = env + (q * P + p) * (int64_t)(2 * QB_ENV_NC);
-  const double s2 = 2.0 / QB_ENV_M;
+  __syncthreads();
+  if (!on) return;
+  const int m = j, base = pl * QB_ENV_NC;
+  const double sg = (m & 1) ? -1.0 : 1.0;
+  cd s0 = 0.5 * f0[base] + 0.5 * (sg * f0[base + QB_ENV_M]);
+  cd s1 = 0.5 * f1[base] + 0.5 * (sg * f1[base + QB_ENV_M]);
 #pragma unroll
-  for (int m = 0; m <= QB_ENV_M; ++m) {
-    const double sg = (m & 1) ? -1.0 : 1.0;
-    cd s0 = 0.5 * f0[0] + 0.5 * (sg * f0[QB_ENV_M]);
-    cd s1 = 0.5 * f1[0] + 0.5 * (sg * f1[QB_ENV_M]);
-    for (int j = 1; j < QB_ENV_M; ++j) {
-      const double cc = lc.C[m * QB_ENV_NC + j];
-      s0 = s0 + f0[j] * cc;
-      s1 = s1 + f1[j] * cc;
-    }
-    const double w = (m == 0 || m == QB_ENV_M) ? 0.5 * s2 : s2;
-    o[2 * m] = w * s0;
-    o[2 * m + 1] = w * s1;
+  for (int i = 1; i < QB_ENV_M; ++i) {
+    int x = (i * m) % (2 * QB_ENV_M);  // cospi(i m / M) from the nodes
+    x = x > QB_ENV_M ? 2 * QB_ENV_M - x : x;
+    s0 = s0 + f0[base + i] * ct[x];
+    s1 = s1 + f1[base + i] * ct[x];
   }
+  const double s2 = 2.0 / QB_ENV_M;
+  const double w = (m == 0 || m == QB_ENV_M) ? 0.5 * s2 : s2;
+  cd* o = env + gid * (int64_t)(2 * QB_ENV_NC);
+  o[2 * m] = w * s0;
+  o[2 * m + 1] = w * s1;
 }
 
 // MW: columns of the mirror tile staged through LDS at a time (16, or 4 for
@@ -742,11 +751,11 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
     return rc;
   }
   EnvLob lc;
-  qb_lobatto_host(QB_ENV_M, lc.t, lc.C);
+  qb_lobatto_host(QB_ENV_M, lc.t);
   const int64_t nt = nz * (int64_t)P;
   int slot = qb_prof_begin(ctx, QB_K_TABLES, 0.0, (double)ebytes);
-  hipLaunchKernelGGL(k_env_tables, dim3((unsigned)((nt + 63) / 64)), dim3(64), 0, ctx->stream,
-                     z_dev, nz, o0, P, lc, env);
+  hipLaunchKernelGGL(k_env_tables, dim3((unsigned)((nt + QB_ENV_PPW - 1) / QB_ENV_PPW)),
+                     dim3(64), 0, ctx->stream, z_dev, nz, o0, P, lc, env);
   qb_prof_end(ctx, slot);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)

@@ -179,7 +179,7 @@ size_t qb_tables_bytes(int64_t nz, const qb_cheb_params& cp, size_t* hbytes);
 // H first, J after it.  Allocates nothing; the tables are not freed.
 int qb_tables_build_in(qb_ctx* ctx, const double* z_dev, int64_t nz, double rmin_h, double rmax,
                        const qb_cheb_params& cp, void* mem, size_t mem_bytes, DevTables* t);
-void qb_lobatto_host(int M, double* t, double* C);  // nodes cospi(j/M), DCT matrix
+void qb_lobatto_host(int M, double* t);  // nodes cospi(j/M)
 
 // assembly (qb_assemble.hip) -------------------------------------------------
 // Writes T(z_q) for q in [0, nz) into out64 (ld = N, stride N*N), and, if

@@ -4,9 +4,9 @@
 // uniform breaks (chebyshev_core.jl:95-103), samples at the M+1 Lobatto
 // nodes r_j = ((b+a) + (b-a) cospi(j/M)) / 2 of every panel
 // (_build_table_h! / _build_table_j!, bessels:331-372) and the DCT-I fit of
-// _chebfit! (chebyshev_core.jl:67-80).  One thread builds one panel of one
-// wavenumber for both orders (H0 and H1, or J0 and J1), so the two series of
-// a panel are stored interleaved and read together by the assembly.
+// _chebfit! (chebyshev_core.jl:67-80).  Both orders (H0 and H1, or J0 and J1)
+// are built together: the two series of a panel are stored interleaved and
+// read together by the assembly.
 #include <math.h>
 #include <string.h>
 
@@ -15,12 +15,6 @@
 #include "qb_internal.h"
 
 #define QB_MMAX 16
-
-struct LobCoef {
-  int M;
-  double t[QB_MMAX + 1];                    // cospi(j/M)
-  double C[(QB_MMAX + 1) * (QB_MMAX + 1)];  // C[m*(M+1)+j] = cospi(j*m/M)
-};
 
 static double cospi_host(double x) {
   x = fmod(fabs(x), 2.0);
@@ -32,66 +26,90 @@ static double cospi_host(double x) {
   return (double)cosl(3.14159265358979323846264338327950288L * (long double)x);
 }
 
-void qb_lobatto_host(int M, double* t, double* C) {
+void qb_lobatto_host(int M, double* t) {
   for (int j = 0; j <= M; ++j) t[j] = cospi_host((double)j / (double)M);
-  for (int m = 0; m <= M; ++m)
-    for (int j = 0; j <= M; ++j) C[m * (M + 1) + j] = cospi_host((double)(j * m) / (double)M);
 }
 
-// kind 0: Hankel H0/H1 on [rmin, rmax]; kind 1: J0/J1 on [0, rmax].
+// Tables of both kinds in one launch: the first bh workgroups build the Hankel
+// panels (H0/H1 on [rmin, rmax]), the others those of J0/J1 on [0, rmax].
+//
+// A lane evaluates one Lobatto node of one panel, a wave as many whole panels as
+// it holds (10 of degree 5), and turns from its node j to the coefficient m = j
+// through LDS.  What bounds it: an evaluation's serial arithmetic (series,
+// recurrences: 15 to 30 us), once per lane; one thread per panel took M + 1 of
+// them in a row, kept its samples in scratch memory and left most SIMDs without
+// a wave.  One wavenumber of a star with 128 nodes: 178 (two launches) -> 25 us;
+// 24 of 1562 nodes: 391 -> 228 us; 16 of 4096 nodes: 544 -> 275 us.
+struct TabArgs {
+  int M, np;
+  double rmin;
+  cd* out;
+  double t[QB_MMAX + 1];  // cospi(j / M)
+};
+
 template <int KIND>
-__global__ void __launch_bounds__(64) k_build_tables(const cd* __restrict__ zk, int64_t nz,
-                                                     double rmin, double rmax, int np,
-                                                     LobCoef lc, cd* __restrict__ out) {
-  int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= nz * (int64_t)np) return;
-  int64_t q = gid / np;
-  int p = (int)(gid - q * np);
-  const int M = lc.M;
-  double h = (rmax - rmin) / (double)np;
-  double a = fma((double)p, h, rmin);
-  double b = (p == np - 1) ? rmax : fma((double)(p + 1), h, rmin);
-  cd k = zk[q];
-  cd f0[QB_MMAX + 1], f1[QB_MMAX + 1];
-  for (int j = 0; j <= M; ++j) {
-    double r = ((b + a) + (b - a) * lc.t[j]) / 2.0;
-    cd z = mk(k.re * r, k.im * r);
+__device__ __forceinline__ void build_panels(const TabArgs& a, const cd* __restrict__ zk,
+                                             int64_t nz, double rmax, int64_t block) {
+  __shared__ cd f0[64], f1[64];
+  __shared__ double ct[QB_MMAX + 1];
+  const int M = a.M, n1 = M + 1, np = a.np, lane = threadIdx.x;
+  const int pl = lane / n1, j = lane - pl * n1;
+  const int64_t gid = block * (64 / n1) + pl;
+  const bool on = pl < 64 / n1 && gid < nz * (int64_t)np;
+  if (lane <= M) ct[lane] = a.t[lane];
+  __syncthreads();
+  if (on) {
+    const int64_t q = gid / np;
+    const int p = (int)(gid - q * np);
+    const double h = (rmax - a.rmin) / (double)np;
+    const double lo = fma((double)p, h, a.rmin);
+    const double hi = (p == np - 1) ? rmax : fma((double)(p + 1), h, a.rmin);
+    const double r = ((hi + lo) + (hi - lo) * ct[j]) / 2.0;
+    const cd k = zk[q];
+    const cd z = mk(k.re * r, k.im * r);
+    cd v0, v1;
     if (KIND == 0)
-      qb_hankel1_01(z, &f0[j], &f1[j]);
+      qb_hankel1_01(z, &v0, &v1);
     else
-      qb_bessel_j01(z, &f0[j], &f1[j]);
+      qb_bessel_j01(z, &v0, &v1);
+    f0[lane] = v0;
+    f1[lane] = v1;
   }
-  cd* o = out + (q * (int64_t)np + p) * (int64_t)(2 * (M + 1));
-  double s2 = 2.0 / (double)M;
-  for (int m = 0; m <= M; ++m) {
-    double sg = (m & 1) ? -1.0 : 1.0;
-    cd s0 = 0.5 * f0[0];
-    cd s1 = 0.5 * f1[0];
-    s0 = s0 + 0.5 * (sg * f0[M]);
-    s1 = s1 + 0.5 * (sg * f1[M]);
-    for (int j = 1; j < M; ++j) {
-      double c = lc.C[m * (M + 1) + j];
-      s0 = s0 + f0[j] * c;
-      s1 = s1 + f1[j] * c;
-    }
-    cd c0 = s2 * s0, c1 = s2 * s1;
-    if (m == 0) {
-      c0 = 0.5 * c0;
-      c1 = 0.5 * c1;
-    }
-    o[2 * m] = c0;
-    o[2 * m + 1] = c1;
+  __syncthreads();
+  if (!on) return;
+  const int m = j, base = pl * n1;
+  const double sg = (m & 1) ? -1.0 : 1.0;
+  cd s0 = 0.5 * f0[base] + 0.5 * (sg * f0[base + M]);
+  cd s1 = 0.5 * f1[base] + 0.5 * (sg * f1[base + M]);
+  for (int i = 1; i < M; ++i) {
+    int x = (i * m) % (2 * M);  // cospi(i m / M) from the nodes
+    x = x > M ? 2 * M - x : x;
+    s0 = s0 + f0[base + i] * ct[x];
+    s1 = s1 + f1[base + i] * ct[x];
   }
+  const double w = (m == 0 ? 0.5 : 1.0) * (2.0 / (double)M);
+  cd* o = a.out + gid * (int64_t)(2 * n1);
+  o[2 * m] = w * s0;
+  o[2 * m + 1] = w * s1;
 }
 
-static LobCoef make_lob(int M) {
-  LobCoef lc{};
-  lc.M = M;
-  double t[QB_MMAX + 1], C[(QB_MMAX + 1) * (QB_MMAX + 1)];
-  qb_lobatto_host(M, t, C);
-  for (int j = 0; j <= M; ++j) lc.t[j] = t[j];
-  for (int i = 0; i < (M + 1) * (M + 1); ++i) lc.C[i] = C[i];
-  return lc;
+__global__ void __launch_bounds__(64) k_build_tables(const cd* __restrict__ zk, int64_t nz,
+                                                     double rmax, TabArgs h, TabArgs j,
+                                                     unsigned bh) {
+  if (blockIdx.x < bh)
+    build_panels<0>(h, zk, nz, rmax, blockIdx.x);
+  else
+    build_panels<1>(j, zk, nz, rmax, blockIdx.x - bh);
+}
+
+static TabArgs tab_args(int M, int np, double rmin, cd* out) {
+  TabArgs a{};
+  a.M = M;
+  a.np = np;
+  a.rmin = rmin;
+  a.out = out;
+  qb_lobatto_host(M, a.t);
+  return a;
 }
 
 size_t qb_tables_bytes(int64_t nz, const qb_cheb_params& cp, size_t* hbytes) {
@@ -115,15 +133,17 @@ static int tables_launch(qb_ctx* ctx, const double* z_dev, int64_t nz, double rm
                          double rmax, const qb_cheb_params& cp, DevTables* t) {
   size_t hb;
   const size_t tb = qb_tables_bytes(nz, cp, &hb);
-  LobCoef lh = make_lob(cp.M_h), lj = make_lob(cp.M_j);
   const cd* zk = (const cd*)z_dev;
-  int64_t nh = nz * (int64_t)cp.n_panels_h, nj = nz * (int64_t)cp.n_panels_j;
+  auto blocks = [&](int np, int M) {
+    const int64_t per = 64 / (M + 1);
+    return (nz * np + per - 1) / per;
+  };
+  const int64_t bh = blocks(cp.n_panels_h, cp.M_h), bj = blocks(cp.n_panels_j, cp.M_j);
+  if (bh + bj >= (int64_t)1 << 31) return qb_fail(ctx, QB_E_ARG, "too many table panels");
   int slot = qb_prof_begin(ctx, QB_K_TABLES, 0.0, (double)tb);
-  hipLaunchKernelGGL(k_build_tables<0>, dim3((unsigned)((nh + 63) / 64)), dim3(64), 0, ctx->stream,
-                     zk, nz, rmin_h, rmax, cp.n_panels_h, lh, t->H);
-  QB_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL(k_build_tables<1>, dim3((unsigned)((nj + 63) / 64)), dim3(64), 0, ctx->stream,
-                     zk, nz, 0.0, rmax, cp.n_panels_j, lj, t->J);
+  hipLaunchKernelGGL(k_build_tables, dim3((unsigned)(bh + bj)), dim3(64), 0, ctx->stream, zk, nz,
+                     rmax, tab_args(cp.M_h, cp.n_panels_h, rmin_h, t->H),
+                     tab_args(cp.M_j, cp.n_panels_j, 0.0, t->J), (unsigned)bh);
   qb_prof_end(ctx, slot);
   QB_HIP(ctx, hipGetLastError());
   return QB_OK;
