@@ -1,20 +1,13 @@
 """Chebyshev tables of every degree and of panel counts around the number that a wave
 builds at once, seen through the matrices assembled from them: the oracle builds the
 same tables (coarse ones too: both interpolate, neither needs to be accurate)."""
-import os
-import sys
-
 import numpy as np
 import pytest
 import scipy.special as sp
 
+from oracle import oracle as O
+
 pytestmark = pytest.mark.gpu
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
-
-
-def _oracle():
-    import oracle
-    return oracle
 
 
 def _case(op, kind, Ns, k0):
@@ -37,7 +30,6 @@ def test_matrices_from_tables(op, kind, Ns, k0, cp):
     17 coefficients of 17 samples each and a Clenshaw sum round to below
     17 * 17 * 4 u = 1.3e-13 of max |H_1(z rmin)|; weights and k r are at most 1 and
     k0 times rmax = 3 in the entries."""
-    O = _oracle()
     q, solver, pts = _case(op, kind, Ns, k0)
     z = np.array([k0 + 0.4j, k0 - 0.3j, k0])
     T = q.assemble(solver, pts, z, n_panels_h=cp[0], M_h=cp[1], n_panels_j=cp[2], M_j=cp[3])
