@@ -734,7 +734,10 @@ extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const doub
   // its own (QB_ASM_TABLES=1: the uniform Hankel tables, as the windows then)
   const bool pairs = (flags & QB_ASM_CONJ_PAIRS) != 0;
   const bool env = pairs && getenv("QB_ASM_TABLES") == nullptr;
-  if (!rc && !env) rc = qb_tables_build(ctx, (const double*)zd, nz, rmin, rmax, *cheb, true, &t);
+  const bool fine = !pairs && g->sym.m == 0 &&
+                    qb_env_stands_in(op == QB_CFIE_KRESS, (const cd*)z, nz, rmin, rmax, *cheb);
+  if (!rc && !env && !fine)
+    rc = qb_tables_build(ctx, (const double*)zd, nz, rmin, rmax, *cheb, true, &t);
   if (!rc) {
     if (on_dev)
       od = (cd*)out;
@@ -749,6 +752,8 @@ extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const doub
         rc = qb_fail(ctx, QB_E_ARG,
                      "QB_ASM_CONJ_PAIRS needs nodes closed under conjugation and no symmetry "
                      "orbits (with QB_ASM_TABLES: tables with M_h = M_j in {5, 7})");
+    } else if (fine) {
+      rc = qb_assemble_env_list(ctx, g, op, (const cd*)z, nz, rmin, rmax, od);
     } else {
       rc = qb_assemble_dev(ctx, g, op, zd, nz, t, od, nullptr);
     }
@@ -853,16 +858,21 @@ extern "C" int qb_assemble_deriv(qb_ctx* ctx, const qb_geom* g, int32_t op, cons
   if (!rc && hipMemcpyAsync(zd, z, nz * sizeof(cd), hipMemcpyHostToDevice, ctx->stream) !=
                  hipSuccess)
     rc = qb_fail(ctx, QB_E_HIP, "upload failed");
-  if (!rc) rc = qb_tables_build(ctx, (const double*)zd, nz, rmin, rmax, *cheb, true, &t);
+  const bool fine =
+      g->sym.m == 0 && qb_env_stands_in(true, (const cd*)z, nz, rmin, rmax, *cheb);
+  if (!rc && !fine)
+    rc = qb_tables_build(ctx, (const double*)zd, nz, rmin, rmax, *cheb, true, &t);
   for (int m = 0; m < 3 && !rc; ++m) {
     if (on_dev)
       od[m] = (cd*)host[m];
     else
       rc = qb_dev_alloc(ctx, (void**)&od[m], obytes);
   }
+  const bool ref_sign = (flags & QB_DERIV_MATRIX_SIGN) == 0;
   if (!rc)
-    rc = qb_assemble_deriv_dev(ctx, g, op, zd, nz, t, od[0], od[1], od[2],
-                               (flags & QB_DERIV_MATRIX_SIGN) == 0);
+    rc = fine ? qb_assemble_deriv_env(ctx, g, op, (const cd*)z, nz, rmin, rmax, od[0], od[1], od[2],
+                                      ref_sign)
+              : qb_assemble_deriv_dev(ctx, g, op, zd, nz, t, od[0], od[1], od[2], ref_sign);
   for (int m = 0; m < 3 && !rc && !on_dev; ++m)
     if (hipMemcpyAsync(host[m], od[m], obytes, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
       rc = qb_fail(ctx, QB_E_HIP, "download failed");
@@ -926,8 +936,13 @@ extern "C" int qb_residuals(qb_ctx* ctx, const qb_geom* g, int32_t op, const dou
       break;
     }
     DevTables t;
-    rc = qb_tables_build(ctx, (const double*)zd, nb, rmin, rmax, *cheb, true, &t);
-    if (!rc) rc = qb_assemble_dev(ctx, g, op, zd, nb, t, Td, nullptr);
+    const cd* lz = (const cd*)lam + q0;
+    if (g->sym.m == 0 && qb_env_stands_in(op == QB_CFIE_KRESS, lz, nb, rmin, rmax, *cheb)) {
+      rc = qb_assemble_env_list(ctx, g, op, lz, nb, rmin, rmax, Td);
+    } else {
+      rc = qb_tables_build(ctx, (const double*)zd, nb, rmin, rmax, *cheb, true, &t);
+      if (!rc) rc = qb_assemble_dev(ctx, g, op, zd, nb, t, Td, nullptr);
+    }
     if (!rc) rc = qb_gemv_norms(ctx, Td, phid, N, (int)nb, nsplit, part, rowabs, colsum);
     part_h.resize((size_t)nsplit * nb * N);
     row_h.resize((size_t)nsplit * nb * N);
@@ -1226,6 +1241,9 @@ static int win_create(qb_ctx* ctx, const qb_geom* g, int32_t op, int32_t nwin, c
       crc = qb_assemble_env_dev(ctx, g, op, w->zj.data(), w->z_dev, nz, rmin, rmax, w->T64, o32,
                                 ahead ? nb : 0,
                                 ahead ? std::function<int()>(first_panel) : std::function<int()>());
+    if (crc == 1 && !no_conj &&
+        qb_env_stands_in(op == QB_CFIE_KRESS, w->zj.data(), nz, rmin, rmax, *cheb))
+      crc = qb_assemble_red_env(ctx, g, op, w->zj.data(), nz, rmin, rmax, w->T64, o32);
     if (crc == 1) {
       QB_TRY(qb_tables_build(ctx, (const double*)w->z_dev, nz, rmin, rmax, *cheb, true, &tab));
       crc = no_conj ? 1 : qb_assemble_conj_dev(ctx, g, op, w->zj.data(), w->z_dev, nz, tab,

@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(256) k_assemble(DevGeom g, const cd* __restric
       if (same) {
         int64_t o = g.off[ci];
         int64_t nc = g.off[ci + 1] - o;
-        int64_t dd = (i - j) % nc;
+        int64_t dd = i - j;  // both in [o, o + nc)
         if (dd < 0) dd += nc;
         Rij = g.rk[o + dd];
         lt = g.lt[o + dd];  // both circulant columns are even in (i - j)
@@ -300,7 +300,7 @@ k_assemble_conj(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ H, 
         if (same) {
           const int64_t o = g.off[ci];
           const int64_t nc = g.off[ci + 1] - o;
-          int64_t dd = (i - j) % nc;
+          int64_t dd = i - j;  // both in [o, o + nc)
           if (dd < 0) dd += nc;
           Rij = g.rk[o + dd];
           lt = g.lt[o + dd];  // both circulant columns are even in (i - j)
@@ -562,8 +562,8 @@ __global__ __launch_bounds__(64) void k_env_tables(const cd* __restrict__ zk, in
 template <int OP, int MW, int OCC>
 __global__ void __launch_bounds__(256, OCC)
 k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env, int o0, int P,
-               const int* __restrict__ pairs, int T, int J0, int first, cd* __restrict__ out64,
-               cf* __restrict__ out32) {
+               const int* __restrict__ pairs, int nout, int T, int J0, int first,
+               cd* __restrict__ out64, cf* __restrict__ out32) {
   static_assert(MW == 4 || MW == 8 || MW == 16, "mirror width");
   extern __shared__ __align__(16) cd smem[];
   const int tsz = P * 2 * QB_ENV_NC;  // complex coefficients per node
@@ -573,6 +573,7 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
   const int64_t N = g.N;
   const int qa = pairs[2 * blockIdx.z], qb = pairs[2 * blockIdx.z + 1];
   const bool two = qa != qb;
+  const bool both = two && qb < nout;  // node b is an output too
   for (int e = threadIdx.x; e < tsz; e += 256) {
     Ta[e] = env[(int64_t)qa * tsz + e];
     Tb[e] = env[(int64_t)qb * tsz + e];
@@ -622,7 +623,7 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
       cd va, vb, wa = mk(0, 0), wb = mk(0, 0);  // (i, j) and (j, i) of nodes a and b
       if (i == j) {
         va = diag_entry<OP>(g, j, ka);
-        vb = two ? diag_entry<OP>(g, j, kb) : va;
+        vb = both ? diag_entry<OP>(g, j, kb) : va;
       } else {
         const double dx = xi - g.x[j], dy = yi - g.y[j];
         const double r = hypot(dx, dy);
@@ -632,7 +633,7 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
         if (same) {
           const int64_t o = g.off[ci];
           const int64_t nc = g.off[ci + 1] - o;
-          int64_t dd = (i - j) % nc;
+          int64_t dd = i - j;  // both in [o, o + nc)
           if (dd < 0) dd += nc;
           Rij = g.rk[o + dd];
           lt = g.lt[o + dd];  // both circulant columns are even in (i - j)
@@ -678,24 +679,24 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
         sb.j0 = cconj(sa.j0);
         sb.j1 = cconj(sa.j1);
         va = offdiag_entry<OP>(g, i, j, dx, dy, invr, same, Rij, lt, ka, sa);
-        vb = two ? offdiag_entry<OP>(g, i, j, dx, dy, invr, same, Rij, lt, kb, sb) : va;
+        vb = both ? offdiag_entry<OP>(g, i, j, dx, dy, invr, same, Rij, lt, kb, sb) : va;
         if (!diag_tile) {
           wa = offdiag_entry<OP>(g, j, i, -dx, -dy, invr, same, Rij, lt, ka, sa);
-          wb = two ? offdiag_entry<OP>(g, j, i, -dx, -dy, invr, same, Rij, lt, kb, sb) : wa;
+          wb = both ? offdiag_entry<OP>(g, j, i, -dx, -dy, invr, same, Rij, lt, kb, sb) : wa;
         }
       }
       const int64_t e1 = i + j * N;
       if (out64) {
         out64[ba + e1] = va;
-        if (two) out64[bb + e1] = vb;
+        if (both) out64[bb + e1] = vb;
       }
       if (out32) {
         out32[ba + e1] = to_cf(va);
-        if (two) out32[bb + e1] = to_cf(vb);
+        if (both) out32[bb + e1] = to_cf(vb);
       }
       if (!diag_tile) {
         mir[0][il][jl - MW * h] = wa;
-        mir[1][il][jl - MW * h] = wb;
+        if (both) mir[1][il][jl - MW * h] = wb;
       }
     }
     if (diag_tile) continue;  // uniform over the block
@@ -712,7 +713,7 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
       const cd xa = mir[0][il2][jl2];
       if (out64) out64[ba + e2] = xa;
       if (out32) out32[ba + e2] = to_cf(xa);
-      if (two) {
+      if (both) {
         const cd xb = mir[1][il2][jl2];
         if (out64) out64[bb + e2] = xb;
         if (out32) out32[bb + e2] = to_cf(xb);
@@ -726,6 +727,29 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
 // (three workgroups per CU for DLP, whose registers fit without spilling).
 static bool env_occ3_default(int op) { return op == QB_DLP_KRESS; }
 
+// Panels of the envelope tables for distances in [rmin, rmax]: the first octave
+// and the panel count, or false when there are too many.
+static bool env_range(double rmin, double rmax, int* o0, int* P) {
+  if (!(rmin > 0.0) || !(rmax > rmin)) return false;
+  *o0 = ilogb(rmin);
+  *P = 4 * (ilogb(rmax) - *o0 + 1);
+  return *P <= QB_ENV_PMAX;
+}
+static size_t env_bytes(int64_t nz, int P) { return (size_t)nz * P * 2 * QB_ENV_NC * sizeof(cd); }
+static void env_launch_tables(qb_ctx* ctx, const cd* z_dev, int64_t nz, int o0, int P, cd* env) {
+  EnvLob lc;
+  qb_lobatto_host(QB_ENV_M, lc.t);
+  const int64_t nt = nz * (int64_t)P;
+  int slot = qb_prof_begin(ctx, QB_K_TABLES, 0.0, (double)env_bytes(nz, P));
+  hipLaunchKernelGGL(k_env_tables, dim3((unsigned)((nt + QB_ENV_PPW - 1) / QB_ENV_PPW)),
+                     dim3(64), 0, ctx->stream, z_dev, nz, o0, P, lc, env);
+  qb_prof_end(ctx, slot);
+}
+
+static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
+                              int64_t nout, const std::vector<int>& pr, int o0, int P, cd* out64,
+                              cf* out32, int cols_first, const std::function<int()>& between);
+
 int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
                         const cd* z_dev, int64_t nz, double rmin, double rmax, cd* out64,
                         cf* out32, int cols_first, const std::function<int()>& between) {
@@ -734,14 +758,19 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
   if (g->sym.m > 0) return 1;
   if (op != QB_CFIE_KRESS && op != QB_DLP_KRESS) return 1;
   if (op == QB_DLP_KRESS && g->d.ncomp != 1) return 1;
-  if (!(rmin > 0.0) || !(rmax > rmin)) return 1;
   std::vector<int> pr;
-  if (!qb_conj_pairs(z_host, nz, &pr)) return 1;
-  const int o0 = ilogb(rmin), o1 = ilogb(rmax);
-  const int P = 4 * (o1 - o0 + 1);
-  if (P > QB_ENV_PMAX) return 1;
+  int o0, P;
+  if (!env_range(rmin, rmax, &o0, &P) || !qb_conj_pairs(z_host, nz, &pr)) return 1;
+  return assemble_env_pairs(ctx, g, op, z_dev, nz, nz, pr, o0, P, out64, out32, cols_first,
+                            between);
+}
+
+// The pairs `pr` of the nz nodes z_dev; only nodes below nout have a matrix.
+static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
+                              int64_t nout, const std::vector<int>& pr, int o0, int P, cd* out64,
+                              cf* out32, int cols_first, const std::function<int()>& between) {
   const int npair = (int)pr.size() / 2;
-  const size_t ebytes = (size_t)nz * P * 2 * QB_ENV_NC * sizeof(cd);
+  const size_t ebytes = env_bytes(nz, P);
   cd* env = nullptr;
   int* pd = nullptr;
   int rc = qb_dev_alloc(ctx, (void**)&env, ebytes);
@@ -750,13 +779,8 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
     qb_dev_free(ctx, env, ebytes);
     return rc;
   }
-  EnvLob lc;
-  qb_lobatto_host(QB_ENV_M, lc.t);
-  const int64_t nt = nz * (int64_t)P;
-  int slot = qb_prof_begin(ctx, QB_K_TABLES, 0.0, (double)ebytes);
-  hipLaunchKernelGGL(k_env_tables, dim3((unsigned)((nt + QB_ENV_PPW - 1) / QB_ENV_PPW)),
-                     dim3(64), 0, ctx->stream, z_dev, nz, o0, P, lc, env);
-  qb_prof_end(ctx, slot);
+  env_launch_tables(ctx, z_dev, nz, o0, P, env);
+  int slot;
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
     e = hipMemcpyAsync(pd, pr.data(), pr.size() * sizeof(int), hipMemcpyHostToDevice,
@@ -779,14 +803,15 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
     if (const char* e = getenv("QB_ASM_ENV_OCC"))
       occ3 = e[0] == '3' && lds4 <= (size_t)(160 * 1024) / 3;
     const size_t lds = occ3 ? lds4 : lds16;
-    const double ent = (double)N * N * nz;
+    const double ent = (double)N * N * nout;
     slot = qb_prof_begin(ctx, QB_K_ASSEMBLE, 0.0,
                          ent * ((out64 ? sizeof(cd) : 0) + (out32 ? sizeof(cf) : 0)));
     auto launch = [&](auto kern, int64_t npairs, int first) {
       (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds);
       hipLaunchKernelGGL(kern, dim3((unsigned)npairs, 1, (unsigned)npair), dim3(256), lds,
-                         ctx->stream, g->d, z_dev, env, o0, P, pd, T, J0, first, out64, out32);
+                         ctx->stream, g->d, z_dev, env, o0, P, pd, (int)nout, T, J0, first, out64,
+                         out32);
     };
     auto launch_all = [&](int64_t npairs, int first) {
       if (op == QB_CFIE_KRESS) {
@@ -828,6 +853,98 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
   return QB_OK;
 }
 
+// Whether uniform tables of the sizes cp would give the Hankel and Bessel values
+// of these wavenumbers so exactly (tables tuned to an absolute error of 1e-12)
+// that the envelope tables may stand in for them: they are within 1e-14 of the
+// functions, built in 25 us and read from LDS.  Coarser tables are interpolated
+// as the caller asked.  The error of a panel of
+// half-width d is about its last coefficient (entering whole, as in the
+// reference): for the pole of H_1, at the first distance that the operator reads
+// from the table, 2 rho^-M / (s^2 - 1)^(1/2) with s the pole's distance in
+// half-widths, for e^{ikr} 2 (|k| d / 2)^M / M!.  Against the actual errors of
+// tables of 500 to 75000 panels the estimate is 1.5 to 10 times them, hence the
+// bound 1.2e-11.  Both routes, tables included: 16 DLP matrices of N = 4096 6.55
+// (uniform) and 2.00 ms, 24 CFIE ones of 1562 1.34 and 0.78 ms, 32 near-real ones
+// of 2050 6.15 and 2.05 ms, one of 128 98 and 75 us, six of 1500 with both
+// derivatives 0.74 and 0.42 ms: what bounds the uniform route is the L1 request
+// per lane and coefficient.
+bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double rmax,
+                      const qb_cheb_params& cp) {
+  int o0, P;
+  if (getenv("QB_ASM_TABLES") || !env_range(rmin, rmax, &o0, &P)) return false;
+  const double dh = (rmax - rmin) / (2.0 * cp.n_panels_h), dj = rmax / (2.0 * cp.n_panels_j);
+  auto osc = [](double q, int M) {  // 2 q^M / M!, geometric tail
+    double v = 2.0;
+    for (int n = 1; n <= M; ++n) v *= q / n;
+    return q < 0.5 * (M + 1) ? v / (1.0 - q / (M + 1)) : INFINITY;
+  };
+  for (int64_t i = 0; i < nz; ++i) {
+    const double ak = hypot(z[i].re, z[i].im);
+    if (!(z[i].re > 0.0) || !(fabs(z[i].im) * rmax < 50.0) || !(ak < 1e12)) return false;
+    const double grow = exp(fabs(z[i].im) * rmax);
+    const double r1 = direct && 0.2 / ak > rmin ? 0.2 / ak : rmin;  // first distance read
+    const double c = fmax(rmin + dh, r1 - dh), s = c / dh;
+    if (!(s > 1.0)) return false;
+    const double w = sqrt(s * s - 1.0), rho = s + w;
+    const double pole = 2.0 * s / w * pow(rho, -cp.M_h) * rho / (rho - 1.0);
+    const double amp = 2.0 / (QB_PI * ak * c) + sqrt(2.0 / (QB_PI * ak * c));
+    const double eh = grow * amp * (pole + osc(0.5 * ak * dh, cp.M_h));
+    const double ej = grow * osc(0.5 * ak * dj, cp.M_j);
+    if (!(eh < 1.2e-11) || !(ej < 1.2e-11)) return false;
+  }
+  return true;
+}
+
+// The wavenumbers z on the device, followed by the conjugates `extra` of some.
+static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd** zd) {
+  int rc = qb_dev_alloc(ctx, (void**)zd, zs.size() * sizeof(cd));
+  if (!rc && hipMemcpyAsync(*zd, zs.data(), zs.size() * sizeof(cd), hipMemcpyHostToDevice,
+                            ctx->stream) != hipSuccess)
+    rc = qb_fail(ctx, QB_E_HIP, "wavenumber upload failed");
+  return rc;
+}
+
+// Matrices of any wavenumbers (Re z > 0) of a plain geometry from envelope
+// tables.  A wavenumber whose conjugate is in the list to rounding (equal real
+// parts, imaginary parts that differ by less than an ulp of k r) is assembled
+// with it; for the others the conjugate's table is built beside their own
+// (J_n = (H_n(k r) + conj H_n(conj(k) r)) / 2) and only their matrix is written.
+int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
+                         double rmin, double rmax, cd* out64) {
+  int o0, P;
+  if (!env_range(rmin, rmax, &o0, &P)) return qb_fail(ctx, QB_E_ARG, "distance range");
+  const int64_t N = g->d.N;
+  const double eps = 1.1e-16 / rmax;
+  for (int64_t q0 = 0; q0 < nz; q0 += 1024) {
+    const int64_t n = nz - q0 < 1024 ? nz - q0 : 1024;
+    std::vector<cd> zs(z_host + q0, z_host + q0 + n);
+    std::vector<int> pr;
+    std::vector<char> used(n, 0);
+    for (int64_t a = 0; a < n; ++a) {
+      if (used[a]) continue;
+      int64_t b = fabs(zs[a].im) <= eps ? a : -1;
+      for (int64_t c = a + 1; b < 0 && c < n; ++c)
+        if (!used[c] && zs[c].re == zs[a].re && fabs(zs[c].im + zs[a].im) <= eps) b = c;
+      if (b < 0) {
+        b = (int64_t)zs.size();
+        zs.push_back(mk(zs[a].re, -zs[a].im));
+      } else {
+        used[b] = 1;
+      }
+      pr.push_back((int)a);
+      pr.push_back((int)b);
+    }
+    cd* zd = nullptr;
+    int rc = env_upload_z(ctx, zs, &zd);
+    if (!rc)
+      rc = assemble_env_pairs(ctx, g, op, zd, (int64_t)zs.size(), n, pr, o0, P,
+                              out64 + q0 * N * N, nullptr, 0, std::function<int()>());
+    qb_dev_free(ctx, zd, zs.size() * sizeof(cd));
+    if (rc) return rc;
+  }
+  return QB_OK;
+}
+
 int qb_assemble_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
                     const DevTables& t, cd* out64, cf* out32) {
   if (op != QB_CFIE_KRESS && op != QB_DLP_KRESS)
@@ -864,6 +981,85 @@ int qb_assemble_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int6
   return QB_OK;
 }
 
+// One wavenumber's envelope tables in LDS: its own (Ta) and its conjugate's (Tb).
+struct EnvView {
+  const cd *Ta, *Tb;
+  int o0, P;
+};
+// Tables of a launch: the uniform ones (t), or the envelope tables env
+// [2 nz][P][13][2] (the conjugates' from nz on) for the kernels with MH = -1.
+struct AsmTabs {
+  DevTables t;
+  const cd* env;
+  int o0, P;
+  int64_t nz;
+};
+// The view of wavenumber q.  Envelope tables are copied to `smem` by the whole
+// workgroup (a barrier follows).
+template <int MH>
+__device__ __forceinline__ auto tab_view(const AsmTabs& tb, int64_t q, cd* smem) {
+  if constexpr (MH < 0) {
+    const int tsz = tb.P * 2 * QB_ENV_NC;
+    for (int e = threadIdx.x; e < tsz; e += blockDim.x) {
+      smem[e] = tb.env[q * tsz + e];
+      smem[tsz + e] = tb.env[(tb.nz + q) * tsz + e];
+    }
+    __syncthreads();
+    return EnvView{smem, smem + tsz, tb.o0, tb.P};
+  } else {
+    TabView tv;
+    tv.H = tb.t.H + q * (int64_t)tb.t.np_h * (2 * (tb.t.M_h + 1));
+    tv.J = tb.t.J ? tb.t.J + q * (int64_t)tb.t.np_j * (2 * (tb.t.M_j + 1)) : nullptr;
+    tv.np_h = tb.t.np_h;
+    tv.M_h = tb.t.M_h;
+    tv.np_j = tb.t.np_j;
+    tv.M_j = tb.t.M_j;
+    tv.rmin_h = tb.t.rmin_h;
+    tv.rmax = tb.t.rmax;
+    return tv;
+  }
+}
+
+// The specials from envelope tables: H_n(k r) = E_n e^{ikr} with the node's own
+// table, J_n = (H_n(k r) + conj H_n(conj(k) r)) / 2 with the conjugate's; one
+// sincos and one exp serve both.  Below |k r| = 0.2 (direct) the functions
+// themselves.
+__device__ __forceinline__ Spec specials_env(const EnvView& ev, double r, cd k, bool direct,
+                                             bool want_j) {
+  Spec s;
+  s.j0 = mk(0, 0);
+  s.j1 = mk(0, 0);
+  const cd z = mk(k.re * r, k.im * r);
+  if (direct && cabsd(z) < 0.2) {
+    qb_hankel1_01(z, &s.h0, &s.h1);
+    if (want_j) qb_bessel_j01(z, &s.j0, &s.j1);
+    return s;
+  }
+  int pp;
+  double t, sn, cs;
+  env_panel(r, ev.o0, ev.P, &pp, &t);
+  sincos(z.re, &sn, &cs);
+  const double ga = exp(-z.im);
+  cd e0, e1;
+  qb_clenshaw2<QB_ENV_M>(ev.Ta + pp * (2 * QB_ENV_NC), t, &e0, &e1);
+  const cd ea = mk(cs * ga, sn * ga);
+  s.h0 = e0 * ea;
+  s.h1 = e1 * ea;
+  if (want_j) {
+    qb_clenshaw2<QB_ENV_M>(ev.Tb + pp * (2 * QB_ENV_NC), t, &e0, &e1);
+    const double gb = 1.0 / ga;
+    const cd eb = mk(cs * gb, sn * gb);
+    const cd g0 = e0 * eb, g1 = e1 * eb;
+    s.j0 = 0.5 * (s.h0 + cconj(g0));
+    s.j1 = 0.5 * (s.h1 + cconj(g1));
+  }
+  return s;
+}
+template <int OP, int MH, int MJ>
+__device__ __forceinline__ Spec specials(const EnvView& ev, double r, cd k, bool same) {
+  return specials_env(ev, r, k, OP == QB_CFIE_KRESS, same);
+}
+
 // ---------------------------------------------------------------------------
 // Assembly with the first and second wavenumber derivatives, T, dT/dk and
 // d2T/dk2, for the expanded boundary integral method:
@@ -890,6 +1086,11 @@ __device__ __forceinline__ Spec specials_all(const TabView& tv, double r, cd k, 
     s.j1 = mk(0, 0);
   }
   return s;
+}
+
+template <int MH, int MJ>
+__device__ __forceinline__ Spec specials_all(const EnvView& ev, double r, cd k, bool want_j) {
+  return specials_env(ev, r, k, true, want_j);
 }
 
 // Off-diagonal entry (target i, source j) of T, T', T''.
@@ -993,18 +1194,18 @@ __device__ __forceinline__ D3 diag_deriv(const DevGeom& g, int64_t j, cd k) {
 }
 
 // Tile pairs as in k_assemble; the mirrored tile of each of the three
-// outputs is staged in LDS 16 source columns at a time (3 x 16 x 65 complex
-// = 50 KB) and written 16 contiguous rows per column.
+// outputs is staged in LDS CW source columns at a time (3 x 16 x 65 complex
+// = 50 KB; 8 beside envelope tables, so that two workgroups fit in a CU) and
+// written CW contiguous rows per column.
 template <int OP, int MH, int MJ>
-__global__ void __launch_bounds__(256) k_assemble_deriv(DevGeom g, const cd* __restrict__ zk,
-                                                        const cd* __restrict__ H,
-                                                        const cd* __restrict__ J, int np_h,
-                                                        int M_h, int np_j, int M_j,
-                                                        double rmin_h, double rmax, int64_t q0,
+__global__ void __launch_bounds__(256, MH < 0 ? 2 : 1) k_assemble_deriv(DevGeom g, const cd* __restrict__ zk,
+                                                        AsmTabs tb, int64_t q0,
                                                         int T, cd* __restrict__ o0,
                                                         cd* __restrict__ o1,
                                                         cd* __restrict__ o2, double off_sign) {
-  __shared__ cd mir[3][16][65];  // mir[out][j_local - 16 ch][i_local] = A[j, i]
+  constexpr int CW = MH < 0 ? 8 : 16;
+  __shared__ cd mir[3][CW][65];  // mir[out][j_local - CW ch][i_local] = A[j, i]
+  extern __shared__ __align__(16) cd smem[];
   const int64_t N = g.N;
   const int64_t q = q0 + blockIdx.z;
   int64_t p = blockIdx.x;
@@ -1014,15 +1215,7 @@ __global__ void __launch_bounds__(256) k_assemble_deriv(DevGeom g, const cd* __r
     ++d;
   }
   const int Jt = (int)p, It = Jt + d;
-  TabView tv;
-  tv.H = H + q * (int64_t)np_h * (2 * (M_h + 1));
-  tv.J = J + q * (int64_t)np_j * (2 * (M_j + 1));
-  tv.np_h = np_h;
-  tv.M_h = M_h;
-  tv.np_j = np_j;
-  tv.M_j = M_j;
-  tv.rmin_h = rmin_h;
-  tv.rmax = rmax;
+  const auto tv = tab_view<MH>(tb, q, smem);
   const cd k = zk[q];
   const int il = threadIdx.x & 63, jl0 = threadIdx.x >> 6;
   const int64_t i = (int64_t)It * 64 + il;
@@ -1037,11 +1230,11 @@ __global__ void __launch_bounds__(256) k_assemble_deriv(DevGeom g, const cd* __r
     ci = g.comp[i];
   }
 #pragma unroll 1
-  for (int ch = 0; ch < 4; ++ch) {
+  for (int ch = 0; ch < 64 / CW; ++ch) {
 #pragma unroll 1
-    for (int c = 0; c < 4; ++c) {
-      const int jc = jl0 + 4 * c;  // 0..15 inside the chunk
-      const int64_t j = (int64_t)Jt * 64 + 16 * ch + jc;
+    for (int c = 0; c < CW / 4; ++c) {
+      const int jc = jl0 + 4 * c;  // 0..CW-1 inside the chunk
+      const int64_t j = (int64_t)Jt * 64 + CW * ch + jc;
       if (!iok || j >= N) continue;
       D3 vij, vji;
       if (i == j) {
@@ -1056,7 +1249,7 @@ __global__ void __launch_bounds__(256) k_assemble_deriv(DevGeom g, const cd* __r
         if (same) {
           const int64_t o = g.off[ci];
           const int64_t nc = g.off[ci + 1] - o;
-          int64_t dd = (i - j) % nc;
+          int64_t dd = i - j;  // both in [o, o + nc)
           if (dd < 0) dd += nc;
           Rij = g.rk[o + dd];
           lt = g.lt[o + dd];
@@ -1078,9 +1271,9 @@ __global__ void __launch_bounds__(256) k_assemble_deriv(DevGeom g, const cd* __r
     }
     if (diag_tile) continue;  // uniform over the workgroup
     __syncthreads();
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      const int jr = e & 15, il2 = e >> 4;
-      const int64_t ii = (int64_t)It * 64 + il2, jj = (int64_t)Jt * 64 + 16 * ch + jr;
+    for (int e = threadIdx.x; e < CW * 64; e += 256) {
+      const int jr = e % CW, il2 = e / CW;
+      const int64_t ii = (int64_t)It * 64 + il2, jj = (int64_t)Jt * 64 + CW * ch + jr;
       if (ii >= N || jj >= N) continue;
       const int64_t idx = base + jj + ii * N;
       o0[idx] = mir[0][jr][il2];
@@ -1093,15 +1286,18 @@ __global__ void __launch_bounds__(256) k_assemble_deriv(DevGeom g, const cd* __r
 
 template <int OP, int MH, int MJ>
 static void launch_asm_deriv(qb_ctx* ctx, const qb_geom* g, const cd* z, int64_t q0, int64_t nzc,
-                             const DevTables& t, cd* o0, cd* o1, cd* o2, double off_sign) {
+                             const AsmTabs& tb, cd* o0, cd* o1, cd* o2, double off_sign) {
   int64_t N = g->d.N;
   int T = (int)((N + 63) / 64);
   int64_t pairs = (int64_t)T * (T + 1) / 2;
   dim3 grid((unsigned)pairs, 1, (unsigned)nzc);
   int slot = qb_prof_begin(ctx, QB_K_ASSEMBLE, 0.0, 3.0 * (double)N * N * nzc * sizeof(cd));
-  hipLaunchKernelGGL((k_assemble_deriv<OP, MH, MJ>), grid, dim3(256), 0, ctx->stream, g->d, z,
-                     t.H, t.J, t.np_h, t.M_h, t.np_j, t.M_j, t.rmin_h, t.rmax, q0, T, o0, o1, o2,
-                     off_sign);
+  const size_t lds = MH < 0 ? 2 * env_bytes(1, tb.P) : 0;
+  if (MH < 0)
+    (void)hipFuncSetAttribute((const void*)k_assemble_deriv<OP, MH, MJ>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL((k_assemble_deriv<OP, MH, MJ>), grid, dim3(256), lds, ctx->stream, g->d, z,
+                     tb, q0, T, o0, o1, o2, off_sign);
   qb_prof_end(ctx, slot);
 }
 
@@ -1118,26 +1314,85 @@ int qb_assemble_deriv_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev
   if (g->sym.m > 0)
     return qb_assemble_red_deriv_dev(ctx, g, op, z_dev, nz, t, out, dout, ddout, off_sign);
   int64_t N = g->d.N;
+  const AsmTabs tb{t, nullptr, 0, 0, nz};
   for (int64_t q0 = 0; q0 < nz; q0 += 1024) {
     int64_t nzc = nz - q0 < 1024 ? nz - q0 : 1024;
     const int64_t o = q0 * N * N;
     const int mh = t.M_h, mj = t.M_j;
     if (op == QB_CFIE_KRESS) {
       if (mh == 7 && mj == 7)
-        launch_asm_deriv<QB_CFIE_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, t, out + o, dout + o,
+        launch_asm_deriv<QB_CFIE_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, tb, out + o, dout + o,
                                               ddout + o, off_sign);
       else
-        launch_asm_deriv<QB_CFIE_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, t, out + o, dout + o,
+        launch_asm_deriv<QB_CFIE_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, tb, out + o, dout + o,
                                               ddout + o, off_sign);
     } else {
       if (mh == 7 && mj == 7)
-        launch_asm_deriv<QB_DLP_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, t, out + o, dout + o,
+        launch_asm_deriv<QB_DLP_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, tb, out + o, dout + o,
                                              ddout + o, off_sign);
       else
-        launch_asm_deriv<QB_DLP_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, t, out + o, dout + o,
+        launch_asm_deriv<QB_DLP_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, tb, out + o, dout + o,
                                              ddout + o, off_sign);
     }
     QB_HIP(ctx, hipGetLastError());
+  }
+  return QB_OK;
+}
+
+// Envelope tables of the wavenumbers zs and then of their conjugates, in memory
+// for env_free.
+struct EnvTabs {
+  cd *z = nullptr, *env = nullptr;
+  size_t zb = 0, eb = 0;
+};
+static void env_free(qb_ctx* ctx, EnvTabs* e) {
+  qb_dev_free(ctx, e->env, e->eb);
+  qb_dev_free(ctx, e->z, e->zb);
+  *e = EnvTabs();
+}
+static int env_build(qb_ctx* ctx, const cd* z_host, int64_t nz, double rmin, double rmax,
+                     EnvTabs* e, AsmTabs* tb) {
+  tb->nz = nz;
+  if (!env_range(rmin, rmax, &tb->o0, &tb->P)) return qb_fail(ctx, QB_E_ARG, "distance range");
+  std::vector<cd> zs(z_host, z_host + nz);
+  for (int64_t i = 0; i < nz; ++i) zs.push_back(mk(z_host[i].re, -z_host[i].im));
+  e->zb = zs.size() * sizeof(cd);
+  e->eb = env_bytes(2 * nz, tb->P);
+  int rc = env_upload_z(ctx, zs, &e->z);
+  if (!rc) rc = qb_dev_alloc(ctx, (void**)&e->env, e->eb);
+  if (!rc) {
+    env_launch_tables(ctx, e->z, 2 * nz, tb->o0, tb->P, e->env);
+    if (hipGetLastError() != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, "table launch failed");
+  }
+  // the host copies are read before the call returns
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess && !rc)
+    rc = qb_fail(ctx, QB_E_HIP, "tables failed");
+  tb->env = e->env;
+  if (rc) env_free(ctx, e);
+  return rc;
+}
+
+// T, T', T'' of a plain geometry from envelope tables (qb_env_stands_in).
+int qb_assemble_deriv_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
+                          double rmin, double rmax, cd* out, cd* dout, cd* ddout, bool ref_sign) {
+  const double off_sign = ref_sign ? -1.0 : 1.0;
+  const int64_t N = g->d.N;
+  for (int64_t q0 = 0; q0 < nz; q0 += 1024) {
+    const int64_t nzc = nz - q0 < 1024 ? nz - q0 : 1024, o = q0 * N * N;
+    EnvTabs e;
+    AsmTabs tb{};
+    int rc = env_build(ctx, z_host + q0, nzc, rmin, rmax, &e, &tb);
+    if (rc) return rc;
+    if (op == QB_CFIE_KRESS)
+      launch_asm_deriv<QB_CFIE_KRESS, -1, -1>(ctx, g, e.z, 0, nzc, tb, out + o, dout + o, ddout + o,
+                                              off_sign);
+    else
+      launch_asm_deriv<QB_DLP_KRESS, -1, -1>(ctx, g, e.z, 0, nzc, tb, out + o, dout + o, ddout + o,
+                                             off_sign);
+    const hipError_t le = hipGetLastError(), se = hipStreamSynchronize(ctx->stream);
+    env_free(ctx, &e);
+    if (le != hipSuccess) return qb_fail(ctx, QB_E_HIP, hipGetErrorString(le));
+    if (se != hipSuccess) return qb_fail(ctx, QB_E_HIP, hipGetErrorString(se));
   }
   return QB_OK;
 }
@@ -1175,7 +1430,7 @@ __device__ __forceinline__ PairGeo pair_geo(const DevGeom& g, int64_t i, int64_t
   if (p.same) {
     const int64_t o = g.off[ci];
     const int64_t nc = g.off[ci + 1] - o;
-    int64_t dd = (i - j) % nc;
+    int64_t dd = i - j;  // both in [o, o + nc)
     if (dd < 0) dd += nc;
     p.Rij = g.rk[o + dd];
     p.lt = g.lt[o + dd];
@@ -1473,9 +1728,9 @@ __global__ void __launch_bounds__(256) k_assemble_red_deriv(
 template <int OP, int MH, int MJ, int MAXI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
-                          const cd* __restrict__ H, const cd* __restrict__ J, int np_h, int M_h,
-                          int np_j, int M_j, double rmin_h, double rmax, int64_t q0, int64_t nz,
+                          AsmTabs tb, int64_t q0, int64_t nz,
                           int T, cd* __restrict__ out64, cf* __restrict__ out32) {
+  extern __shared__ __align__(16) cd smem[];
   const int64_t m = s.m;
   const int G = s.G;
   const int nirr = s.nirr;
@@ -1487,11 +1742,11 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
     ++d;
   }
   const int Jt = (int)p, It = Jt + d;
-  const TabView tv = tab_view(H, J, q, np_h, M_h, np_j, M_j, rmin_h, rmax);
+  const auto tv = tab_view<MH>(tb, q, smem);
   const cd k = zk[q];
   const int il = threadIdx.x & 63, jl0 = threadIdx.x >> 6;
   const int64_t a = (int64_t)It * 64 + il;
-  if (a >= m) return;  // no barrier in this kernel
+  if (a >= m) return;  // no barrier from here on
   const bool diag_tile = (It == Jt);
   const int64_t mm = m * m;
   const int64_t i = s.img[a * G];
@@ -1585,8 +1840,7 @@ static void launch_red(qb_ctx* ctx, const qb_geom* g, const cd* z, int64_t q0, i
     const int64_t pairs = (int64_t)Tm * (Tm + 1) / 2;
     hipLaunchKernelGGL((k_assemble_red_pair_multi<OP, MH, MJ, 8>),
                        dim3((unsigned)pairs, 1, (unsigned)nzc), dim3(256), 0, ctx->stream, g->d,
-                       g->sym, z, t.H, t.J, t.np_h, t.M_h, t.np_j, t.M_j, t.rmin_h, t.rmax, q0,
-                       nz, (int)Tm, o64, o32);
+                       g->sym, z, AsmTabs{t, nullptr, 0, 0, nz}, q0, nz, (int)Tm, o64, o32);
   } else if (nirr <= 8) {
     hipLaunchKernelGGL((k_assemble_red<OP, MH, MJ, 8>), grid, dim3(256), 0, ctx->stream, g->d,
                        g->sym, z, t.H, t.J, t.np_h, t.M_h, t.np_j, t.M_j, t.rmin_h, t.rmax, q0,
@@ -1610,6 +1864,51 @@ static void launch_red_deriv(qb_ctx* ctx, const qb_geom* g, const cd* z, int64_t
                      0, ctx->stream, g->d, g->sym, z, t.H, t.J, t.np_h, t.M_h, t.np_j, t.M_j,
                      t.rmin_h, t.rmax, q0, o0, o1, o2, off_sign);
   qb_prof_end(ctx, slot);
+}
+
+template <int OP>
+struct RedPairMulti {
+  template <int MAXI>
+  auto operator()() const {
+    return k_assemble_red_pair_multi<OP, -1, -1, MAXI>;
+  }
+};
+
+// Reduced matrices of 2 to 8 irreps with pair sharing, from envelope tables;
+// other geometries return 1.
+int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
+                        double rmin, double rmax, cd* out64, cf* out32) {
+  const int64_t m = g->sym.m;
+  const int nirr = g->sym.nirr;
+  if (m <= 0 || !g->sym.pair || nirr < 2 || nirr > 8 || nz > 1024) return 1;
+  EnvTabs e;
+  AsmTabs tb{};
+  int rc = env_build(ctx, z_host, nz, rmin, rmax, &e, &tb);
+  if (rc) return rc;
+  const unsigned Tm = (unsigned)((m + 63) / 64);
+  const double ent = (double)m * m * nz * nirr;
+  const size_t lds = 2 * env_bytes(1, tb.P);
+  int slot = qb_prof_begin(ctx, QB_K_ASSEMBLE, 0.0,
+                           ent * ((out64 ? sizeof(cd) : 0) + (out32 ? sizeof(cf) : 0)));
+  auto launch = [&](auto k) {
+    // accumulators for the number of irreps: with room for eight the kernel spills
+    auto kern = nirr <= 4 ? k.template operator()<4>() : nirr <= 6 ? k.template operator()<6>()
+                                                                   : k.template operator()<8>();
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
+    hipLaunchKernelGGL(kern, dim3(Tm * (Tm + 1) / 2, 1, (unsigned)nz), dim3(256), lds, ctx->stream,
+                       g->d, g->sym, e.z, tb, (int64_t)0, nz, (int)Tm, out64, out32);
+  };
+  if (op == QB_CFIE_KRESS)
+    launch(RedPairMulti<QB_CFIE_KRESS>());
+  else
+    launch(RedPairMulti<QB_DLP_KRESS>());
+  qb_prof_end(ctx, slot);
+  const hipError_t le = hipGetLastError(), se = hipStreamSynchronize(ctx->stream);
+  env_free(ctx, &e);
+  if (le != hipSuccess) return qb_fail(ctx, QB_E_HIP, hipGetErrorString(le));
+  if (se != hipSuccess) return qb_fail(ctx, QB_E_HIP, hipGetErrorString(se));
+  return QB_OK;
 }
 
 int qb_assemble_red_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,

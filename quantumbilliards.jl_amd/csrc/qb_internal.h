@@ -212,6 +212,16 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
                         const cd* z_dev, int64_t nz, double rmin, double rmax, cd* out64,
                         cf* out32, int cols_first = 0,
                         const std::function<int()>& between = std::function<int()>());
+// Envelope tables in the place of uniform ones of the sizes cp (direct: the
+// operator evaluates below |k r| = 0.2 directly), and the assemblies from them.
+bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double rmax,
+                      const qb_cheb_params& cp);
+int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
+                         double rmin, double rmax, cd* out64);
+int qb_assemble_deriv_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
+                          double rmin, double rmax, cd* out, cd* dout, cd* ddout, bool ref_sign);
+int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
+                        double rmin, double rmax, cd* out64, cf* out32);
 // Pairs (a, b) of wavenumbers with z_b = conj(z_a) (a real one with itself),
 // flattened; false when some wavenumber has no partner.
 bool qb_conj_pairs(const cd* z_host, int64_t nz, std::vector<int>* pr);
