@@ -614,7 +614,7 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
   __syncthreads();
   constexpr int CPS = MW / 4;  // column groups (4 columns each) per mirror stage
 #pragma unroll 1
-  for (int h = 0; h < 64 / MW; ++h) {
+  for (int h = blockIdx.y; h < 64 / MW; h += gridDim.y) {
 #pragma unroll 1
     for (int c = CPS * h; c < CPS * h + CPS; ++c) {
       const int jl = jl0 + 4 * c;
@@ -746,6 +746,15 @@ static void env_launch_tables(qb_ctx* ctx, const cd* z_dev, int64_t nz, int o0, 
   qb_prof_end(ctx, slot);
 }
 
+// Workgroups that share the column stages of a tile pair when the tile pairs alone
+// are fewer than two rounds of the chip's 512 places (one matrix of N = 128, three
+// tile pairs: 53 -> 18 us).
+static unsigned env_split(int64_t tiles, unsigned stages) {
+  unsigned n = 1;
+  while (n < stages && tiles * n < 1024) n *= 2;
+  return n;
+}
+
 static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
                               int64_t nout, const std::vector<int>& pr, int o0, int P, cd* out64,
                               cf* out32, int cols_first, const std::function<int()>& between);
@@ -809,8 +818,9 @@ static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z
     auto launch = [&](auto kern, int64_t npairs, int first) {
       (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds);
-      hipLaunchKernelGGL(kern, dim3((unsigned)npairs, 1, (unsigned)npair), dim3(256), lds,
-                         ctx->stream, g->d, z_dev, env, o0, P, pd, (int)nout, T, J0, first, out64,
+      hipLaunchKernelGGL(kern, dim3((unsigned)npairs, env_split(npairs * npair, occ3 ? 16 : 4),
+                                    (unsigned)npair),
+                         dim3(256), lds, ctx->stream, g->d, z_dev, env, o0, P, pd, (int)nout, T, J0, first, out64,
                          out32);
     };
     auto launch_all = [&](int64_t npairs, int first) {
@@ -864,9 +874,9 @@ static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z
 // half-widths, for e^{ikr} 2 (|k| d / 2)^M / M!.  Against the actual errors of
 // tables of 500 to 75000 panels the estimate is 1.5 to 10 times them, hence the
 // bound 1.2e-11.  Both routes, tables included: 16 DLP matrices of N = 4096 6.55
-// (uniform) and 2.00 ms, 24 CFIE ones of 1562 1.34 and 0.78 ms, 32 near-real ones
-// of 2050 6.15 and 2.05 ms, one of 128 98 and 75 us, six of 1500 with both
-// derivatives 0.74 and 0.42 ms: what bounds the uniform route is the L1 request
+// (uniform) and 1.45 ms, 24 CFIE ones of 1562 1.34 and 0.51 ms, 32 near-real ones
+// of 2050 6.15 and 2.05 ms, one of 128 98 and 38 us, six of 1500 with both
+// derivatives 0.74 and 0.37 ms: what bounds the uniform route is the L1 request
 // per lane and coefficient.
 bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double rmax,
                       const qb_cheb_params& cp) {
@@ -906,15 +916,14 @@ static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd** zd) {
 
 // Matrices of any wavenumbers (Re z > 0) of a plain geometry from envelope
 // tables.  A wavenumber whose conjugate is in the list to rounding (equal real
-// parts, imaginary parts that differ by less than an ulp of k r) is assembled
-// with it; for the others the conjugate's table is built beside their own
+// parts, imaginary parts within u |k| of opposite: less than the rounding of k r
+// moves the argument at every r) is assembled with it; for the others the conjugate's table is built beside their own
 // (J_n = (H_n(k r) + conj H_n(conj(k) r)) / 2) and only their matrix is written.
 int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
                          double rmin, double rmax, cd* out64) {
   int o0, P;
   if (!env_range(rmin, rmax, &o0, &P)) return qb_fail(ctx, QB_E_ARG, "distance range");
   const int64_t N = g->d.N;
-  const double eps = 1.1e-16 / rmax;
   for (int64_t q0 = 0; q0 < nz; q0 += 1024) {
     const int64_t n = nz - q0 < 1024 ? nz - q0 : 1024;
     std::vector<cd> zs(z_host + q0, z_host + q0 + n);
@@ -922,6 +931,7 @@ int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host
     std::vector<char> used(n, 0);
     for (int64_t a = 0; a < n; ++a) {
       if (used[a]) continue;
+      const double eps = 1.1e-16 * zs[a].re;
       int64_t b = fabs(zs[a].im) <= eps ? a : -1;
       for (int64_t c = a + 1; b < 0 && c < n; ++c)
         if (!used[c] && zs[c].re == zs[a].re && fabs(zs[c].im + zs[a].im) <= eps) b = c;
@@ -1230,7 +1240,7 @@ __global__ void __launch_bounds__(256, MH < 0 ? 2 : 1) k_assemble_deriv(DevGeom 
     ci = g.comp[i];
   }
 #pragma unroll 1
-  for (int ch = 0; ch < 64 / CW; ++ch) {
+  for (int ch = blockIdx.y; ch < 64 / CW; ch += gridDim.y) {
 #pragma unroll 1
     for (int c = 0; c < CW / 4; ++c) {
       const int jc = jl0 + 4 * c;  // 0..CW-1 inside the chunk
@@ -1290,7 +1300,7 @@ static void launch_asm_deriv(qb_ctx* ctx, const qb_geom* g, const cd* z, int64_t
   int64_t N = g->d.N;
   int T = (int)((N + 63) / 64);
   int64_t pairs = (int64_t)T * (T + 1) / 2;
-  dim3 grid((unsigned)pairs, 1, (unsigned)nzc);
+  dim3 grid((unsigned)pairs, env_split(pairs * nzc, MH < 0 ? 8 : 4), (unsigned)nzc);
   int slot = qb_prof_begin(ctx, QB_K_ASSEMBLE, 0.0, 3.0 * (double)N * N * nzc * sizeof(cd));
   const size_t lds = MH < 0 ? 2 * env_bytes(1, tb.P) : 0;
   if (MH < 0)
@@ -1720,10 +1730,8 @@ __global__ void __launch_bounds__(256) k_assemble_red_deriv(
 
 // Multi-irrep twin of k_assemble_red_pair: one specials evaluation per image
 // term serves entry (a, b) and entry (b, a) of all nirr irreps at once.  The
-// nirr mirror values of a thread are written directly as rows of the mirror
-// tiles: 64 lanes store 64 scattered 16-byte values per instruction, and the
-// L2 cache merges the 64 rows of every mirror column that the 4 waves of the
-// block write into whole lines.  Diagonal tiles are assembled entry by entry.
+// nirr mirror values of a thread are staged in LDS four columns at a time and
+// written as four contiguous rows.  Diagonal tiles are assembled entry by entry.
 // Outputs indexed as in k_assemble_red (matrix e * nz + q from the base).
 template <int OP, int MH, int MJ, int MAXI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -1746,20 +1754,22 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
   const cd k = zk[q];
   const int il = threadIdx.x & 63, jl0 = threadIdx.x >> 6;
   const int64_t a = (int64_t)It * 64 + il;
-  if (a >= m) return;  // no barrier from here on
+  __shared__ cd mir[MAXI][64][5];  // mir[e][a_local][b_local % 4] = A_red[b, a]
+  const bool aok = a < m;
   const bool diag_tile = (It == Jt);
   const int64_t mm = m * m;
-  const int64_t i = s.img[a * G];
+  const int64_t i = s.img[(aok ? a : m - 1) * G];
   const double xi = g.x[i], yi = g.y[i];
   const int ci = g.comp[i];
 #pragma unroll 1
   for (int c = 0; c < 16; ++c) {
     const int64_t b = (int64_t)Jt * 64 + jl0 + 4 * c;
-    if (b >= m) break;
+    const bool ok = aok && b < m;
     cd acc[MAXI], accm[MAXI];
 #pragma unroll
     for (int e = 0; e < MAXI; ++e) acc[e] = accm[e] = mk(0, 0);
-    if (diag_tile) {
+    if (!ok) {
+    } else if (diag_tile) {
 #pragma unroll 1
       for (int l = 0; l < G; ++l) {
         const int64_t j = s.img[b * G + l];
@@ -1802,16 +1812,26 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
     }
 #pragma unroll
     for (int e = 0; e < MAXI; ++e) {
-      if (e >= nirr) break;
+      if (e >= nirr || !ok) break;
       const int64_t idx = ((int64_t)e * nz + q) * mm + a + b * m;
       if (out64) out64[idx] = acc[e];
       if (out32) out32[idx] = to_cf(acc[e]);
-      if (!diag_tile) {
-        const int64_t idt = ((int64_t)e * nz + q) * mm + b + a * m;
-        if (out64) out64[idt] = accm[e];
-        if (out32) out32[idt] = to_cf(accm[e]);
-      }
+      if (!diag_tile) mir[e][il][jl0] = accm[e];
     }
+    if (diag_tile) continue;  // uniform over the workgroup
+    __syncthreads();
+    {
+      const int il2 = threadIdx.x >> 2, jr = threadIdx.x & 3;
+      const int64_t a2 = (int64_t)It * 64 + il2, b2 = (int64_t)Jt * 64 + 4 * c + jr;
+      if (a2 < m && b2 < m)
+        for (int e = 0; e < nirr; ++e) {
+          const int64_t idt = ((int64_t)e * nz + q) * mm + b2 + a2 * m;
+          const cd v = mir[e][il2][jr];
+          if (out64) out64[idt] = v;
+          if (out32) out32[idt] = to_cf(v);
+        }
+    }
+    __syncthreads();
   }
 }
 
