@@ -226,7 +226,11 @@ int64_t qb_geom_dim(const qb_geom* g);
  * (cheb-DLP:1110-1124).  Writes nz dense N x N complex128 matrices
  * out[q*N*N + i + j*N] = T(z_q)[i,j] (overwrites, like the reference).  With
  * flags & QB_OUT_DEVICE, out is a device pointer; otherwise host memory.
- * rminmax (may be NULL) receives the padded table range [rmin, rmax]. */
+ * rminmax (may be NULL) receives the padded table range [rmin, rmax].
+ * Where tables of the given sizes would resolve H and J to about 1e-12 (the
+ * estimate of qb_env_stands_in), on a plain geometry, the values come from
+ * envelope tables instead (1e-14), also in qb_assemble_deriv and
+ * qb_residuals; coarser tables are interpolated as the reference does. */
 int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const double* z,
                 int64_t nz, const qb_cheb_params* cheb, double* out,
                 int32_t flags, double* rminmax);
@@ -239,7 +243,8 @@ int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const double* z,
  * kernel; no conjugate pairing).  The Chebyshev tables, the only memory
  * beyond the inputs and outputs, are built in a fixed device array of
  * QB_NOALLOC_SCRATCH_BYTES that the library holds on every GPU it runs on
- * until the process ends.  They take
+ * until the process ends (in the place of tables tuned to 1e-12 or finer, the
+ * envelope tables that qb_assemble takes then).  The tables of the sizes given take
  *   nz * (n_panels_h * (M_h + 1) + n_panels_j * (M_j + 1)) * 32 bytes;
  * a call that needs more is rejected with QB_E_ARG (assemble fewer
  * wavenumbers per call).  Every call on one GPU shares that GPU's array and

@@ -815,10 +815,22 @@ extern "C" int qb_assemble_noalloc(qb_ctx* ctx, const qb_geom* g, int32_t op,
   }
   if (nz == 0) return QB_OK;
   (void)hipSetDevice(ctx->device);
-  DevTables t;
-  rc = qb_tables_build_in(ctx, z_dev, nz, rmin, rmax, *cheb, mem,
-                          (size_t)QB_NOALLOC_SCRATCH_BYTES, &t);
-  if (!rc) rc = qb_assemble_dev(ctx, g, op, (const cd*)z_dev, nz, t, (cd*)out_dev, nullptr);
+  // the route, and so the bits, of qb_assemble, which knows the wavenumbers
+  std::vector<cd> zh(nz);
+  if (hipMemcpyAsync(zh.data(), z_dev, nz * sizeof(cd), hipMemcpyDeviceToHost, ctx->stream) !=
+          hipSuccess ||
+      hipStreamSynchronize(ctx->stream) != hipSuccess)
+    return qb_fail(ctx, QB_E_HIP, "wavenumber download failed");
+  rc = 1;
+  if (g->sym.m == 0 && qb_env_stands_in(op == QB_CFIE_KRESS, zh.data(), nz, rmin, rmax, *cheb))
+    rc = qb_assemble_env_list(ctx, g, op, zh.data(), nz, rmin, rmax, (cd*)out_dev, mem,
+                              (size_t)QB_NOALLOC_SCRATCH_BYTES);
+  if (rc == 1) {
+    DevTables t;
+    rc = qb_tables_build_in(ctx, z_dev, nz, rmin, rmax, *cheb, mem,
+                            (size_t)QB_NOALLOC_SCRATCH_BYTES, &t);
+    if (!rc) rc = qb_assemble_dev(ctx, g, op, (const cd*)z_dev, nz, t, (cd*)out_dev, nullptr);
+  }
   // complete on return, as qb_assemble is
   const hipError_t e = hipStreamSynchronize(ctx->stream);
   if (!rc && e != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));

@@ -25,6 +25,15 @@ struct TabView {
   double rmin_h, rmax;
 };
 
+// H0, H1 (and J0, J1) below |z| = 0.2: qb_hankel1_01's series alone, without the
+// code and the registers of its other regions.
+__device__ __forceinline__ void hank_series(cd z, cd* h0, cd* h1, cd* j0, cd* j1) {
+  cd y0, y1;
+  qb_bessel_series(z, true, j0, j1, &y0, &y1);
+  *h0 = *j0 + mk(-y0.im, y0.re);
+  *h1 = *j1 + mk(-y1.im, y1.re);
+}
+
 template <int MH, int MJ>
 __device__ __forceinline__ void hank(const TabView& tv, double r, cd k, bool cutoff, cd* h0,
                                      cd* h1) {
@@ -603,7 +612,7 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
     It = Jt + d;
   }
   const cd ka = zk[qa], kb = zk[qb];
-  const int il = threadIdx.x & 63, jl0 = threadIdx.x >> 6;
+  const int il = threadIdx.x & 63, jl0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t i = (int64_t)It * 64 + il;
   const bool iok = i < N;
   const int64_t ba = (int64_t)qa * N * N, bb = (int64_t)qb * N * N;
@@ -642,9 +651,10 @@ k_assemble_env(DevGeom g, const cd* __restrict__ zk, const cd* __restrict__ env,
         const cd za = mk(ka.re * r, ka.im * r);
         if (OP == QB_CFIE_KRESS && cabsd(za) < 0.2) {
           // h0_h1_multi_ks_at_r! (bessels:1190-1206): |kr| < 0.2 directly
-          qb_hankel1_01(za, &sa.h0, &sa.h1);
+          cd j0, j1;  // formed below, as elsewhere
+          hank_series(za, &sa.h0, &sa.h1, &j0, &j1);
           if (two)
-            qb_hankel1_01(mk(kb.re * r, kb.im * r), &sb.h0, &sb.h1);
+            hank_series(mk(kb.re * r, kb.im * r), &sb.h0, &sb.h1, &j0, &j1);
           else
             sb = sa;
         } else {
@@ -757,7 +767,8 @@ static unsigned env_split(int64_t tiles, unsigned stages) {
 
 static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
                               int64_t nout, const std::vector<int>& pr, int o0, int P, cd* out64,
-                              cf* out32, int cols_first, const std::function<int()>& between);
+                              cf* out32, int cols_first, const std::function<int()>& between,
+                              void* mem = nullptr);
 
 int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
                         const cd* z_dev, int64_t nz, double rmin, double rmax, cd* out64,
@@ -774,20 +785,29 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
                             between);
 }
 
-// The pairs `pr` of the nz nodes z_dev; only nodes below nout have a matrix.
+// The pairs `pr` of the nz nodes z_dev; only nodes below nout have a matrix.  mem:
+// the caller's device memory for the tables and the pairs, or null.
 static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
                               int64_t nout, const std::vector<int>& pr, int o0, int P, cd* out64,
-                              cf* out32, int cols_first, const std::function<int()>& between) {
+                              cf* out32, int cols_first, const std::function<int()>& between,
+                              void* mem) {
   const int npair = (int)pr.size() / 2;
   const size_t ebytes = env_bytes(nz, P);
-  cd* env = nullptr;
-  int* pd = nullptr;
-  int rc = qb_dev_alloc(ctx, (void**)&env, ebytes);
-  if (!rc) rc = qb_dev_alloc(ctx, (void**)&pd, pr.size() * sizeof(int));
-  if (rc) {
-    qb_dev_free(ctx, env, ebytes);
-    return rc;
+  cd* env = (cd*)mem;
+  int* pd = mem ? (int*)((char*)mem + ebytes) : nullptr;
+  if (!mem) {
+    int rc = qb_dev_alloc(ctx, (void**)&env, ebytes);
+    if (!rc) rc = qb_dev_alloc(ctx, (void**)&pd, pr.size() * sizeof(int));
+    if (rc) {
+      qb_dev_free(ctx, env, ebytes);
+      return rc;
+    }
   }
+  auto release = [&] {
+    if (mem) return;
+    qb_dev_free(ctx, pd, pr.size() * sizeof(int));
+    qb_dev_free(ctx, env, ebytes);
+  };
   env_launch_tables(ctx, z_dev, nz, o0, P, env);
   int slot;
   hipError_t e = hipGetLastError();
@@ -849,16 +869,14 @@ static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess && brc != 0) {
       (void)hipStreamSynchronize(ctx->stream);
-      qb_dev_free(ctx, pd, pr.size() * sizeof(int));
-      qb_dev_free(ctx, env, ebytes);
+      release();
       return brc;
     }
   }
   // the tables and the pair list must outlive the launch
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   else (void)hipStreamSynchronize(ctx->stream);
-  qb_dev_free(ctx, pd, pr.size() * sizeof(int));
-  qb_dev_free(ctx, env, ebytes);
+  release();
   if (e != hipSuccess) return qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));
   return QB_OK;
 }
@@ -905,13 +923,11 @@ bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double 
   return true;
 }
 
-// The wavenumbers z on the device, followed by the conjugates `extra` of some.
-static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd** zd) {
-  int rc = qb_dev_alloc(ctx, (void**)zd, zs.size() * sizeof(cd));
-  if (!rc && hipMemcpyAsync(*zd, zs.data(), zs.size() * sizeof(cd), hipMemcpyHostToDevice,
-                            ctx->stream) != hipSuccess)
-    rc = qb_fail(ctx, QB_E_HIP, "wavenumber upload failed");
-  return rc;
+static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd* zd) {
+  if (hipMemcpyAsync(zd, zs.data(), zs.size() * sizeof(cd), hipMemcpyHostToDevice, ctx->stream) !=
+      hipSuccess)
+    return qb_fail(ctx, QB_E_HIP, "wavenumber upload failed");
+  return QB_OK;
 }
 
 // Matrices of any wavenumbers (Re z > 0) of a plain geometry from envelope
@@ -919,10 +935,14 @@ static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd** zd) {
 // parts, imaginary parts within u |k| of opposite: less than the rounding of k r
 // moves the argument at every r) is assembled with it; for the others the conjugate's table is built beside their own
 // (J_n = (H_n(k r) + conj H_n(conj(k) r)) / 2) and only their matrix is written.
+// mem: mem_bytes of device memory to work in, or null; 1 when too few.
 int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
-                         double rmin, double rmax, cd* out64) {
+                         double rmin, double rmax, cd* out64, void* mem, size_t mem_bytes) {
   int o0, P;
   if (!env_range(rmin, rmax, &o0, &P)) return qb_fail(ctx, QB_E_ARG, "distance range");
+  // a wavenumber and its partner take a node's tables, z and two pair indices each
+  const size_t most = (size_t)(nz < 1024 ? nz : 1024) * 2 * (env_bytes(1, P) + sizeof(cd) + 8);
+  if (mem && most > mem_bytes) return 1;
   const int64_t N = g->d.N;
   for (int64_t q0 = 0; q0 < nz; q0 += 1024) {
     const int64_t n = nz - q0 < 1024 ? nz - q0 : 1024;
@@ -944,12 +964,15 @@ int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host
       pr.push_back((int)a);
       pr.push_back((int)b);
     }
-    cd* zd = nullptr;
-    int rc = env_upload_z(ctx, zs, &zd);
+    const size_t zb = zs.size() * sizeof(cd);
+    cd* zd = (cd*)mem;
+    int rc = mem ? QB_OK : qb_dev_alloc(ctx, (void**)&zd, zb);
+    if (!rc) rc = env_upload_z(ctx, zs, zd);
     if (!rc)
       rc = assemble_env_pairs(ctx, g, op, zd, (int64_t)zs.size(), n, pr, o0, P,
-                              out64 + q0 * N * N, nullptr, 0, std::function<int()>());
-    qb_dev_free(ctx, zd, zs.size() * sizeof(cd));
+                              out64 + q0 * N * N, nullptr, 0, std::function<int()>(),
+                              mem ? (char*)mem + zb : nullptr);
+    if (!mem) qb_dev_free(ctx, zd, zb);
     if (rc) return rc;
   }
   return QB_OK;
@@ -1041,8 +1064,7 @@ __device__ __forceinline__ Spec specials_env(const EnvView& ev, double r, cd k, 
   s.j1 = mk(0, 0);
   const cd z = mk(k.re * r, k.im * r);
   if (direct && cabsd(z) < 0.2) {
-    qb_hankel1_01(z, &s.h0, &s.h1);
-    if (want_j) qb_bessel_j01(z, &s.j0, &s.j1);
+    hank_series(z, &s.h0, &s.h1, &s.j0, &s.j1);
     return s;
   }
   int pp;
@@ -1227,7 +1249,7 @@ __global__ void __launch_bounds__(256, MH < 0 ? 2 : 1) k_assemble_deriv(DevGeom 
   const int Jt = (int)p, It = Jt + d;
   const auto tv = tab_view<MH>(tb, q, smem);
   const cd k = zk[q];
-  const int il = threadIdx.x & 63, jl0 = threadIdx.x >> 6;
+  const int il = threadIdx.x & 63, jl0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t i = (int64_t)It * 64 + il;
   const int64_t base = (q - q0) * N * N;
   const bool diag_tile = (It == Jt);
@@ -1368,8 +1390,9 @@ static int env_build(qb_ctx* ctx, const cd* z_host, int64_t nz, double rmin, dou
   for (int64_t i = 0; i < nz; ++i) zs.push_back(mk(z_host[i].re, -z_host[i].im));
   e->zb = zs.size() * sizeof(cd);
   e->eb = env_bytes(2 * nz, tb->P);
-  int rc = env_upload_z(ctx, zs, &e->z);
+  int rc = qb_dev_alloc(ctx, (void**)&e->z, e->zb);
   if (!rc) rc = qb_dev_alloc(ctx, (void**)&e->env, e->eb);
+  if (!rc) rc = env_upload_z(ctx, zs, e->z);
   if (!rc) {
     env_launch_tables(ctx, e->z, 2 * nz, tb->o0, tb->P, e->env);
     if (hipGetLastError() != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, "table launch failed");
@@ -1730,8 +1753,10 @@ __global__ void __launch_bounds__(256) k_assemble_red_deriv(
 
 // Multi-irrep twin of k_assemble_red_pair: one specials evaluation per image
 // term serves entry (a, b) and entry (b, a) of all nirr irreps at once.  The
-// nirr mirror values of a thread are staged in LDS four columns at a time and
-// written as four contiguous rows.  Diagonal tiles are assembled entry by entry.
+// nirr mirror values of a thread are summed in LDS four columns at a time (24
+// registers fewer) and written as four contiguous rows.  What bounds it is
+// the registers: with envelope tables, five irreps of 1640 and 48 nodes took 30 ms
+// while 85 of them were spilled, 17.4 ms with 30.  Diagonal tiles are assembled entry by entry.
 // Outputs indexed as in k_assemble_red (matrix e * nz + q from the base).
 template <int OP, int MH, int MJ, int MAXI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -1752,7 +1777,9 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
   const int Jt = (int)p, It = Jt + d;
   const auto tv = tab_view<MH>(tb, q, smem);
   const cd k = zk[q];
-  const int il = threadIdx.x & 63, jl0 = threadIdx.x >> 6;
+  const int il = threadIdx.x & 63;
+  // the wave's column: uniform, so its node, images and weights are scalar loads
+  const int jl0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t a = (int64_t)It * 64 + il;
   __shared__ cd mir[MAXI][64][5];  // mir[e][a_local][b_local % 4] = A_red[b, a]
   const bool aok = a < m;
@@ -1765,9 +1792,9 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
   for (int c = 0; c < 16; ++c) {
     const int64_t b = (int64_t)Jt * 64 + jl0 + 4 * c;
     const bool ok = aok && b < m;
-    cd acc[MAXI], accm[MAXI];
+    cd acc[MAXI];
 #pragma unroll
-    for (int e = 0; e < MAXI; ++e) acc[e] = accm[e] = mk(0, 0);
+    for (int e = 0; e < MAXI; ++e) acc[e] = mir[e][il][jl0] = mk(0, 0);
     if (!ok) {
     } else if (diag_tile) {
 #pragma unroll 1
@@ -1783,7 +1810,7 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
         }
 #pragma unroll
         for (int e = 0; e < MAXI; ++e)
-          if (e < nirr) acc[e] = acc[e] + s.scale[((int64_t)e * m + b) * G + l] * v;
+          acc[e] = acc[e] + s.scale[((int64_t)(e < nirr ? e : 0) * m + b) * G + l] * v;
       }
     } else {
       const int64_t ib = s.img[b * G];
@@ -1802,12 +1829,14 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
                                         k, sp);
         const cd v2 = offdiag_entry<OP>(g, ib, jm, p2.dx, p2.dy, p1.invr, p2.same, p2.Rij,
                                         p2.lt, k, sp);
+        // weights without a condition: behind branches on nirr their loads stood in
+        // a row, ten waits per image
 #pragma unroll
-        for (int e = 0; e < MAXI; ++e)
-          if (e < nirr) {
-            acc[e] = acc[e] + s.scale[((int64_t)e * m + b) * G + l] * v1;
-            accm[e] = accm[e] + s.scale[((int64_t)e * m + a) * G + ls] * v2;
-          }
+        for (int e = 0; e < MAXI; ++e) {
+          const int64_t em = (int64_t)(e < nirr ? e : 0) * m;
+          acc[e] = acc[e] + s.scale[(em + b) * G + l] * v1;
+          mir[e][il][jl0] = mir[e][il][jl0] + s.scale[(em + a) * G + ls] * v2;
+        }
       }
     }
 #pragma unroll
@@ -1816,7 +1845,6 @@ k_assemble_red_pair_multi(DevGeom g, DevSym s, const cd* __restrict__ zk,
       const int64_t idx = ((int64_t)e * nz + q) * mm + a + b * m;
       if (out64) out64[idx] = acc[e];
       if (out32) out32[idx] = to_cf(acc[e]);
-      if (!diag_tile) mir[e][il][jl0] = accm[e];
     }
     if (diag_tile) continue;  // uniform over the workgroup
     __syncthreads();

@@ -217,7 +217,8 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
 bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double rmax,
                       const qb_cheb_params& cp);
 int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
-                         double rmin, double rmax, cd* out64);
+                         double rmin, double rmax, cd* out64, void* mem = nullptr,
+                         size_t mem_bytes = 0);
 int qb_assemble_deriv_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
                           double rmin, double rmax, cd* out, cd* dout, cd* ddout, bool ref_sign);
 int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
