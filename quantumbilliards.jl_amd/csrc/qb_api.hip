@@ -923,19 +923,17 @@ extern "C" int qb_residuals(qb_ctx* ctx, const qb_geom* g, int32_t op, const dou
   int64_t G = batch > 0 ? batch : (int64_t)std::max<size_t>(1, ((size_t)8 << 30) / per);
   G = std::min<int64_t>(G, nl);
   const int nsplit = 8;
-  cd *zd = nullptr, *Td = nullptr, *phid = nullptr, *part = nullptr;
-  double *rowabs = nullptr, *colsum = nullptr;
+  cd *zd = nullptr, *Td = nullptr, *phid = nullptr;
+  void* work = nullptr;
+  double* nrm = nullptr;
   const size_t b_z = G * sizeof(cd), b_T = G * per, b_phi = (size_t)G * N * sizeof(cd);
-  const size_t b_part = (size_t)nsplit * G * N * sizeof(cd);
-  const size_t b_row = (size_t)nsplit * G * N * sizeof(double), b_col = (size_t)G * N * sizeof(double);
+  const size_t b_work = qb_gemv_norms_bytes(N, (int)G, nsplit), b_nrm = 5 * G * sizeof(double);
   rc = qb_dev_alloc(ctx, (void**)&zd, b_z);
   if (!rc) rc = qb_dev_alloc(ctx, (void**)&Td, b_T);
   if (!rc) rc = qb_dev_alloc(ctx, (void**)&phid, b_phi);
-  if (!rc) rc = qb_dev_alloc(ctx, (void**)&part, b_part);
-  if (!rc) rc = qb_dev_alloc(ctx, (void**)&rowabs, b_row);
-  if (!rc) rc = qb_dev_alloc(ctx, (void**)&colsum, b_col);
-  std::vector<cd> part_h;
-  std::vector<double> row_h, col_h;
+  if (!rc) rc = qb_dev_alloc(ctx, &work, b_work);
+  if (!rc) rc = qb_dev_alloc(ctx, (void**)&nrm, b_nrm);
+  std::vector<double> nrm_h(5 * G);
   for (int64_t q0 = 0; !rc && q0 < nl; q0 += G) {
     const int64_t nb = std::min<int64_t>(G, nl - q0);
     hipError_t e = hipMemcpyAsync(zd, lam + 2 * q0, nb * sizeof(cd), hipMemcpyHostToDevice,
@@ -955,53 +953,21 @@ extern "C" int qb_residuals(qb_ctx* ctx, const qb_geom* g, int32_t op, const dou
       rc = qb_tables_build(ctx, (const double*)zd, nb, rmin, rmax, *cheb, true, &t);
       if (!rc) rc = qb_assemble_dev(ctx, g, op, zd, nb, t, Td, nullptr);
     }
-    if (!rc) rc = qb_gemv_norms(ctx, Td, phid, N, (int)nb, nsplit, part, rowabs, colsum);
-    part_h.resize((size_t)nsplit * nb * N);
-    row_h.resize((size_t)nsplit * nb * N);
-    col_h.resize((size_t)nb * N);
-    if (!rc) {
-      e = hipMemcpyAsync(part_h.data(), part, part_h.size() * sizeof(cd), hipMemcpyDeviceToHost,
-                         ctx->stream);
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(row_h.data(), rowabs, row_h.size() * sizeof(double),
-                           hipMemcpyDeviceToHost, ctx->stream);
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(col_h.data(), colsum, col_h.size() * sizeof(double),
-                           hipMemcpyDeviceToHost, ctx->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-      if (e != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));
-    } else {
-      (void)hipStreamSynchronize(ctx->stream);
-    }
+    if (!rc) rc = qb_gemv_norms(ctx, Td, phid, N, (int)nb, nsplit, work, nrm);
+    if (!rc && hipMemcpyAsync(nrm_h.data(), nrm, 5 * nb * sizeof(double), hipMemcpyDeviceToHost,
+                              ctx->stream) != hipSuccess)
+      rc = qb_fail(ctx, QB_E_HIP, "norm download failed");
+    e = hipStreamSynchronize(ctx->stream);
+    if (!rc && e != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));
     qb_tables_free(ctx, &t);
     if (rc) break;
-    for (int64_t b = 0; b < nb; ++b) {
-      double s2 = 0, s1 = 0, smx = 0, rmx = 0, cmx = 0;
-      for (int64_t i = 0; i < N; ++i) {
-        double yr = 0, yi = 0, ra = 0;
-        for (int s = 0; s < nsplit; ++s) {
-          const size_t o = ((size_t)s * nb + b) * N + i;
-          yr += part_h[o].re;
-          yi += part_h[o].im;
-          ra += row_h[o];
-        }
-        const double a = hypot(yr, yi);
-        s2 += a * a;
-        s1 += a;
-        smx = std::max(smx, a);
-        rmx = std::max(rmx, ra);
-        cmx = std::max(cmx, col_h[(size_t)b * N + i]);
-      }
-      if (res2) res2[q0 + b] = sqrt(s2);
-      if (resn1) resn1[q0 + b] = s1;
-      if (resninf) resninf[q0 + b] = smx;
-      if (opn1) opn1[q0 + b] = cmx;
-      if (opninf) opninf[q0 + b] = rmx;
-    }
+    double* const res[5] = {res2, resn1, resninf, opn1, opninf};
+    for (int64_t b = 0; b < nb; ++b)
+      for (int c = 0; c < 5; ++c)
+        if (res[c]) res[c][q0 + b] = nrm_h[5 * b + c];
   }
-  qb_dev_free(ctx, colsum, b_col);
-  qb_dev_free(ctx, rowabs, b_row);
-  qb_dev_free(ctx, part, b_part);
+  qb_dev_free(ctx, nrm, b_nrm);
+  qb_dev_free(ctx, work, b_work);
   qb_dev_free(ctx, phid, b_phi);
   qb_dev_free(ctx, Td, b_T);
   qb_dev_free(ctx, zd, b_z);

@@ -97,11 +97,11 @@ int qb_gemm_tune(qb_ctx* ctx, int M, int N, int K, int batch, double* best_tflop
 const char* qb_gemm_variant_name(int ty, int v);
 
 // Residual check (qb_residual.hip): for nb matrices T (N x N, stride N*N) and
-// vectors phi (stride N), partial products part[s][b][i] and partial row
-// sums rowabs[s][b][i] of |T| over nsplit column chunks, and column sums
-// colsum[b][j] of |T|.
+// vectors phi (stride N) ||T phi||_2, _1, _inf, ||T||_1 and ||T||_inf in
+// out[5 b ..] (device); work: qb_gemv_norms_bytes.
+size_t qb_gemv_norms_bytes(int64_t N, int nb, int nsplit);
 int qb_gemv_norms(qb_ctx* ctx, const cd* T, const cd* phi, int64_t N, int nb, int nsplit,
-                  cd* part, double* rowabs, double* colsum);
+                  void* work, double* out);
 
 // Householder QR (qb_qr.hip): the first r columns of the N x ncols block A
 // (ld = N) are factored in place (R on and above the diagonal, reflectors
