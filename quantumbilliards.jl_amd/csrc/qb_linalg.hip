@@ -815,7 +815,7 @@ int qb_gemm_class(int M, int N, int K) {
 }
 
 template <typename T>
-static int gemm_default(int M, int N, int K) {
+static int gemm_default(int M, int N, int K, bool conc = false) {
   // the tile a shape gets when the autotuner has not timed its class (the
   // serving loop's windows of many sizes): for complex128 the autotuner's
   // usual picks; complex64 keeps four-product tiles (the three-product form
@@ -824,10 +824,13 @@ static int gemm_default(int M, int N, int K) {
   // shape of a window (32 matrices, 8 M N K per second against the 128 x 128 or
   // 256 x 64 tile): 2816 x 2816 x 256 112 against 85 TFLOP/s, 1536 x 352 x 1536 105
   // against 80, 64 x 352 x 64 28 against 10, 2048 x 32 x 32 25 against 20.  The
-  // bits are the same: every tile sums in the order of k.
+  // bits are the same: every tile sums in the order of k.  Beside the lookahead
+  // panel (conc) four workgroups leave its leaves no place (610 against 320 us per
+  // leaf of N = 3072): there the 128 x 64 tile, 102 TFLOP/s.  A mixed window of 3072,
+  // 32 nodes: 140 ms with the 128 x 128 tile, 113 with 64 x 64 everywhere, 107 with both.
   (void)M;
   if constexpr (sizeof(T) == sizeof(cf))
-    return 12;
+    return conc ? 3 : 12;
   else
     return (N <= 32 || K <= 32) ? QB_GEMM_LEAN_C128 : K <= 64 ? 16 : 21;  // 128x32 register tile
 }
@@ -848,6 +851,7 @@ int gemm_sub(qb_ctx* ctx, int M, int N, int K, const T* A, int64_t lda, int64_t 
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return QB_OK;
   const int ty = sizeof(T) == sizeof(cf) ? 0 : 1;
   int v = (ctx->gemm_conc ? ctx->gemm_pick_conc : ctx->gemm_pick)[ty][qb_gemm_class(M, N, K)];
+  if (v < 0) v = gemm_default<T>(M, N, K, ctx->gemm_conc);
   if (ty == 1 && ctx->panel_lean) v = QB_GEMM_LEAN_C128;
   return gemm_sub_v<T>(ctx, v, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, batch);
 }
@@ -2146,6 +2150,9 @@ __global__ void k_moments(const cd* __restrict__ X, int64_t nv, int nq, const cd
   A1[i] = a1;
 }
 // Per-node max |.|_inf of n_per entries (|re|+|im| bound not used: true modulus).
+// 64 workgroups of 256 per node, each with one atomic: with 1024 of them and one per
+// wave the atomics to a node's address took the time (32 nodes of 3072 x 352:
+// 844 -> 86 us).
 __global__ void k_node_maxabs(const cd* __restrict__ X, int64_t n_per, int64_t stride,
                               double* __restrict__ out, const int* __restrict__ bix) {
   const int64_t b = bix ? bix[blockIdx.y] : blockIdx.y;
@@ -2155,8 +2162,13 @@ __global__ void k_node_maxabs(const cd* __restrict__ X, int64_t n_per, int64_t s
        i += (int64_t)gridDim.x * blockDim.x)
     m = fmax(m, cabsd(X[i]));
   for (int off = 32; off >= 1; off >>= 1) m = fmax(m, __shfl_xor(m, off));
-  if ((threadIdx.x & 63) == 0)
+  __shared__ double red[4];
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
     atomicMax((unsigned long long*)(out + b), (unsigned long long)__double_as_longlong(m));
+  }
 }
 __global__ void k_node_maxabs32(const cf* __restrict__ X, int64_t n_per, double* __restrict__ out) {
   const int64_t b = blockIdx.y;
@@ -2169,18 +2181,32 @@ __global__ void k_node_maxabs32(const cf* __restrict__ X, int64_t n_per, double*
   if ((threadIdx.x & 63) == 0)
     atomicMax((unsigned long long*)(out + b), (unsigned long long)__double_as_longlong(m));
 }
-// Per-node infinity norm of the matrix: max_i sum_j |A_ij|.  One thread per row.
-__global__ void k_node_rownorm(const cd* __restrict__ A, int64_t n, int64_t sA,
-                               double* __restrict__ out) {
+// Per-node infinity norm of the matrix: max_i sum_j |A_ij|.  A workgroup takes 64
+// rows, each of its four waves every fourth group of four columns (one thread per row left
+// half the places of the chip empty; 32 matrices of 3072: 2.0 -> 0.95 ms, 5.1 TB/s).
+__global__ void __launch_bounds__(256) k_node_rownorm(const cd* __restrict__ A, int64_t n,
+                                                      int64_t sA, double* __restrict__ out) {
+  __shared__ double red[4][64];
   const int64_t b = blockIdx.y;
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+  const cd* a = A + b * sA + (i < n ? i : n - 1);
   double s = 0;
-  if (i < n) {
-    const cd* a = A + b * sA + i;
-    for (int64_t j = 0; j < n; ++j) s += cabsd(a[j * n]);
+  int64_t j = 4 * w;
+  for (; j + 4 <= n; j += 16) {
+    cd v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = a[(j + u) * n];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s += cabsd(v[u]);
   }
+  for (; j < n && j % 16 < 4 * w + 4; ++j) s += cabsd(a[j * n]);
+  red[w][lane] = s;
+  __syncthreads();
+  if (w) return;
+  s = i < n ? (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]) : 0.0;
   for (int off = 32; off >= 1; off >>= 1) s = fmax(s, __shfl_xor(s, off));
-  if ((threadIdx.x & 63) == 0)
+  if (lane == 0)
     atomicMax((unsigned long long*)(out + b), (unsigned long long)__double_as_longlong(s));
 }
 
@@ -2225,7 +2251,7 @@ int qb_node_maxabs(qb_ctx* ctx, const cd* X, int64_t n_per, int64_t stride, int 
   // entries are cleared first
   QB_HIP(ctx, hipMemsetAsync(out_dev, 0, (n_out > nb ? n_out : nb) * sizeof(double), ctx->stream));
   int64_t g = (n_per + 255) / 256;
-  dim3 grid((unsigned)(g > 1024 ? 1024 : g), nb);
+  dim3 grid((unsigned)(g > 64 ? 64 : g), nb);
   hipLaunchKernelGGL(k_node_maxabs, grid, dim3(256), 0, ctx->stream, X, n_per, stride, out_dev,
                      ctx->bix);
   QB_HIP(ctx, hipGetLastError());
@@ -2241,7 +2267,7 @@ int qb_node_maxabs32(qb_ctx* ctx, const cf* X, int64_t n_per, int nb, double* ou
 }
 int qb_node_rownorm(qb_ctx* ctx, const cd* A, int64_t n, int nb, double* out_dev) {
   QB_HIP(ctx, hipMemsetAsync(out_dev, 0, nb * sizeof(double), ctx->stream));
-  dim3 grid((unsigned)((n + 255) / 256), nb);
+  dim3 grid((unsigned)((n + 63) / 64), nb);
   hipLaunchKernelGGL(k_node_rownorm, grid, dim3(256), 0, ctx->stream, A, n, n * n, out_dev);
   QB_HIP(ctx, hipGetLastError());
   return QB_OK;

@@ -211,3 +211,20 @@ extern "C" double qbt_oz_bench(qb_ctx* ctx, int N, int r, int nb, int iters) {
   hipFree(Cw); hipFree(F);
   return ms / iters;
 }
+
+// Largest row sum and largest entry, by modulus, of nb host matrices n x n.
+extern "C" int qbt_node_norms(qb_ctx* ctx, int n, int nb, const cd* A, double* rows, double* mx) {
+  cd* dA;
+  double* dO;
+  const size_t a = (size_t)n * n * nb * sizeof(cd);
+  if (hipMalloc(&dA, a) || hipMalloc(&dO, 2 * nb * sizeof(double))) return -2;
+  hipMemcpy(dA, A, a, hipMemcpyHostToDevice);
+  int rc = qb_node_rownorm(ctx, dA, n, nb, dO);
+  if (!rc) rc = qb_node_maxabs(ctx, dA, (int64_t)n * n, (int64_t)n * n, nb, dO + nb, nb);
+  hipStreamSynchronize(ctx->stream);
+  hipMemcpy(rows, dO, nb * sizeof(double), hipMemcpyDeviceToHost);
+  hipMemcpy(mx, dO + nb, nb * sizeof(double), hipMemcpyDeviceToHost);
+  hipFree(dA);
+  hipFree(dO);
+  return rc;
+}

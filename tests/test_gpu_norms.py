@@ -1,7 +1,11 @@
 """Norms formed on the device, at row and column counts around the groups of 4, 16, 64
 and 256 that the kernels take."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
+
 pytestmark = pytest.mark.gpu
 
 
@@ -26,3 +30,17 @@ def test_residual_norms(N, nl, batch):
         tol = 4 * N * 1.2e-16 * (a @ np.abs(phi[:, i])).sum()
         for c in range(5):
             assert abs(got[c][i] - ref[c]) <= (tol if c < 3 else 4 * N * 1.2e-16 * ref[c])
+
+
+@pytest.mark.parametrize("n,nb", [(1, 1), (3, 2), (4, 1), (15, 2), (17, 3), (63, 1), (65, 2), (130, 2), (300, 3)])
+def test_matrix_norms(n, nb):
+    import qbhip as q
+    L = C.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "libqbt_linalg.so"))
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((nb, n, n)) + 1j * rng.standard_normal((nb, n, n))
+    rows, mx = np.zeros(nb), np.zeros(nb)
+    assert L.qbt_node_norms(C.c_void_p(q.default_context().ptr.value), n, nb, C.c_void_p(A.ctypes.data),
+                            C.c_void_p(rows.ctypes.data), C.c_void_p(mx.ctypes.data)) == 0
+    # A[b] holds the matrix column by column
+    assert np.allclose(rows, np.abs(A).sum(1).max(1), rtol=n * 2.3e-16, atol=0)
+    assert np.allclose(mx, np.abs(A).max((1, 2)), rtol=2.3e-16, atol=0)
