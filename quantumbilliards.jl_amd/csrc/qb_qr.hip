@@ -16,25 +16,20 @@
 #include "qb_internal.h"
 #include "qb_linalg.h"
 
-// zlarfg for column j: rows j..N-1.  One workgroup per block; block b =
-// blockIdx.y holds its matrix at A + b * bstride and its tau at tau + b * tstride.
-__global__ void __launch_bounds__(1024) k_house(cd* __restrict__ A, int64_t N, int64_t ld, int j,
-                                                cd* __restrict__ tau, int64_t bstride,
-                                                int64_t tstride) {
-  __shared__ double red[16];
+// zlarfg of x = A[:, j], rows j..N-1, by the NT threads of a workgroup.
+template <int NT>
+__device__ __forceinline__ void reflector(cd* __restrict__ x, int64_t N, int j, cd* __restrict__ tau) {
+  __shared__ double red[NT / 64];
   __shared__ cd s_scale;
-  A += (int64_t)blockIdx.y * bstride;
-  tau += (int64_t)blockIdx.y * tstride;
-  cd* x = A + (int64_t)j * ld;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   double s = 0;
-  for (int64_t i = j + 1 + tid; i < N; i += blockDim.x) s += x[i].re * x[i].re + x[i].im * x[i].im;
+  for (int64_t i = j + 1 + tid; i < N; i += NT) s += x[i].re * x[i].re + x[i].im * x[i].im;
   for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
   if (lane == 0) red[wv] = s;
   __syncthreads();
   if (tid == 0) {
     double sig2 = 0;
-    for (int q = 0; q < (int)(blockDim.x + 63) / 64; ++q) sig2 += red[q];
+    for (int q = 0; q < NT / 64; ++q) sig2 += red[q];
     const cd alpha = x[j];
     if (sig2 == 0.0 && alpha.im == 0.0) {
       tau[j] = mk(0.0, 0.0);
@@ -50,27 +45,42 @@ __global__ void __launch_bounds__(1024) k_house(cd* __restrict__ A, int64_t N, i
   __syncthreads();
   const cd sc = s_scale;
   if (sc.re == 0.0 && sc.im == 0.0) return;
-  for (int64_t i = j + 1 + tid; i < N; i += blockDim.x) x[i] = x[i] * sc;
+  for (int64_t i = j + 1 + tid; i < N; i += NT) x[i] = x[i] * sc;
+}
+
+// The reflector of column j.  One workgroup per block; block b = blockIdx.y holds
+// its matrix at A + b * bstride and its tau at tau + b * tstride.
+__global__ void __launch_bounds__(1024) k_house(cd* __restrict__ A, int64_t N, int64_t ld, int j,
+                                                cd* __restrict__ tau, int64_t bstride,
+                                                int64_t tstride) {
+  reflector<1024>(A + (int64_t)blockIdx.y * bstride + (int64_t)j * ld, N, j,
+                  tau + (int64_t)blockIdx.y * tstride);
 }
 
 // Columns c0 + blockIdx.x (< c1) of A: a <- a - t v (v^H a) over rows j..N-1,
 // with v the stored reflector of column j (v[j] = 1) of V and t = conj(tau_j)
 // (ADJ: applying H_j^H, the QR sweep) or tau_j (applying H_j, forming Q).
-// Block b = blockIdx.y: V, A at + b * bstride, tau at + b * tstride.
+// Block b = blockIdx.y: V, A at + b * bstride, tau at + b * tstride.  With `next`
+// (ADJ, c0 = j + 1, in place) the workgroup of column j + 1 goes on to form that
+// column's reflector: inside a panel every step is one launch of 4.7 us, not two of
+// 3.3 and 4.0 us and the gap between (a block of 530 rows).
 template <bool ADJ>
 __global__ void __launch_bounds__(256) k_house_apply(const cd* __restrict__ V, int64_t ldv,
                                                      cd* __restrict__ A, int64_t N, int64_t lda,
-                                                     int j, int c0, const cd* __restrict__ tau,
-                                                     int64_t bstride, int64_t tstride) {
+                                                     int j, int c0, cd* __restrict__ tau,
+                                                     int64_t bstride, int64_t tstride, bool next) {
   __shared__ double red_re[4], red_im[4];
   V += (int64_t)blockIdx.y * bstride;
   A += (int64_t)blockIdx.y * bstride;
   tau += (int64_t)blockIdx.y * tstride;
   const cd t = ADJ ? cconj(tau[j]) : tau[j];
-  if (t.re == 0.0 && t.im == 0.0) return;  // uniform over the workgroup
   const cd* v = V + (int64_t)j * ldv;
   cd* a = A + (int64_t)(c0 + blockIdx.x) * lda;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  if (t.re == 0.0 && t.im == 0.0) {  // uniform over the workgroup
+    if (next && blockIdx.x == 0) reflector<256>(a, N, j + 1, tau);
+    return;
+  }
   // w = v^H a
   double wr = 0, wi = 0;
   for (int64_t i = j + tid; i < N; i += 256) {
@@ -95,6 +105,9 @@ __global__ void __launch_bounds__(256) k_house_apply(const cd* __restrict__ V, i
     const cd vi = (i == j) ? mk(1.0, 0.0) : v[i];
     a[i] = a[i] - vi * tw;
   }
+  if (!next || blockIdx.x != 0) return;
+  __syncthreads();  // the column is complete
+  reflector<256>(a, N, j + 1, tau);
 }
 
 // ---------------------------------------------------------------------------
@@ -129,38 +142,58 @@ __global__ void k_qr_form_v(const cd* __restrict__ A, int64_t N, int j0, int jb,
 
 // T of the panel from tau and G = V^H V (jb x jb, ld jb): T(i,i) = tau_i,
 // T(0:i, i) = -tau_i T(0:i, 0:i) G(0:i, i); stored (jb x jb, ld jb) as
-// -T^H (ADJ, the QR sweep) or -T (forming Q).  One workgroup of jb threads
-// per block (jb <= QB_QR_NB).
+// -T^H (ADJ, the QR sweep) or -T (forming Q).  One workgroup per block
+// (jb <= QB_QR_NB), all of which reads and writes; row t of T is thread t's alone.
+// What bounds it: the 32 columns one after the other (24 us; with loads column by
+// column and one chain of sums 43).
 template <bool ADJ>
-__global__ void k_qr_form_t(const cd* __restrict__ G, const cd* __restrict__ tau, int j0, int jb,
+__global__ void __launch_bounds__(256) k_qr_form_t(const cd* __restrict__ G, const cd* __restrict__ tau, int j0, int jb,
                             cd* __restrict__ Th, int64_t gstride, int64_t tstride) {
-  __shared__ cd T[QB_QR_NB][QB_QR_NB + 1];
-  __shared__ cd z[QB_QR_NB];
+  __shared__ cd T[QB_QR_NB][QB_QR_NB + 1], Gs[QB_QR_NB][QB_QR_NB + 1];
+  __shared__ cd ts[QB_QR_NB];
   G += (int64_t)blockIdx.x * gstride;
   tau += (int64_t)blockIdx.x * tstride;
   Th += (int64_t)blockIdx.x * gstride;
   const int t = threadIdx.x;
-  for (int c = 0; c < jb; ++c) T[t][c] = mk(0.0, 0.0);
+  cd g[QB_QR_NB * QB_QR_NB / 256];
+#pragma unroll
+  for (int u = 0; u < QB_QR_NB * QB_QR_NB / 256; ++u) {
+    const int e = t + 256 * u;
+    g[u] = e < jb * jb ? G[e] : mk(0.0, 0.0);
+  }
+  if (t < jb) ts[t] = tau[j0 + t];
+#pragma unroll
+  for (int u = 0; u < QB_QR_NB * QB_QR_NB / 256; ++u) {
+    const int e = t + 256 * u;
+    if (e < jb * jb) {
+      Gs[e % jb][e / jb] = g[u];
+      T[e % jb][e / jb] = mk(0.0, 0.0);
+    }
+  }
   __syncthreads();
-  for (int i = 0; i < jb; ++i) {
-    const cd ti = tau[j0 + i];
-    if (t == 0) T[i][i] = ti;
-    if (t < i) z[t] = G[t + (int64_t)i * jb];
-    __syncthreads();
+  for (int i = 0; i < jb && t < jb; ++i) {
+    const cd ti = ts[i];
+    if (t == i) T[i][i] = ti;
     if (t < i) {
-      cd s = mk(0.0, 0.0);
-      for (int c = t; c < i; ++c) s = s + T[t][c] * z[c];
+      cd p[4] = {};  // four chains
+      int c = t;
+      for (; c + 4 <= i; c += 4)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = p[u] + T[t][c + u] * Gs[c + u][i];
+      for (; c < i; ++c) p[0] = p[0] + T[t][c] * Gs[c][i];
+      const cd s = (p[0] + p[1]) + (p[2] + p[3]);
       T[t][i] = mk(-(ti.re * s.re - ti.im * s.im), -(ti.re * s.im + ti.im * s.re));
     }
-    __syncthreads();
   }
-  for (int c = 0; c < jb; ++c) {
+  __syncthreads();
+  for (int e = t; e < jb * jb; e += 256) {
+    const int r = e % jb, c = e / jb;
     if (ADJ) {
-      const cd x = T[c][t];  // Th(t, c) = -conj(T(c, t))
-      Th[t + (int64_t)c * jb] = mk(-x.re, x.im);
+      const cd x = T[c][r];  // Th(r, c) = -conj(T(c, r))
+      Th[e] = mk(-x.re, x.im);
     } else {
-      const cd x = T[t][c];
-      Th[t + (int64_t)c * jb] = mk(-x.re, -x.im);
+      const cd x = T[r][c];
+      Th[e] = mk(-x.re, -x.im);
     }
   }
 }
@@ -228,13 +261,11 @@ int qb_house_qr(qb_ctx* ctx, cd* A, int64_t N, int r, int ncols, cd* tau, int nb
     // the panel: reflectors j0..j0+jb-1 applied within the panel's columns
     // (all trailing columns when unblocked)
     const int cend = blocked ? j0 + jb : ncols;
-    for (int j = j0; j < j0 + jb; ++j) {
-      hipLaunchKernelGGL(k_house, dim3(1, nb), dim3(1024), 0, ctx->stream, A, N, N, j, tau,
-                         bstride, tstride);
-      if (cend - j - 1 > 0)
-        hipLaunchKernelGGL(k_house_apply<true>, dim3(cend - j - 1, nb), dim3(256), 0,
-                           ctx->stream, A, N, A, N, N, j, j + 1, tau, bstride, tstride);
-    }
+    hipLaunchKernelGGL(k_house, dim3(1, nb), dim3(1024), 0, ctx->stream, A, N, N, j0, tau, bstride,
+                       tstride);
+    for (int j = j0; j < j0 + jb && j + 1 < cend; ++j)
+      hipLaunchKernelGGL(k_house_apply<true>, dim3(cend - j - 1, nb), dim3(256), 0, ctx->stream, A,
+                         N, A, N, N, j, j + 1, tau, bstride, tstride, j + 1 < j0 + jb);
     const int nc = ncols - (j0 + jb);
     if (!blocked || nc <= 0) continue;
     const int64_t m = N - j0;
@@ -250,7 +281,7 @@ int qb_house_qr(qb_ctx* ctx, cd* A, int64_t N, int r, int ncols, cd* tau, int nb
                           A + b * bstride + j0 + (int64_t)(j0 + jb) * N, N, part, W + b * wstride);
     }
     if (rc) break;
-    hipLaunchKernelGGL(k_qr_form_t<true>, dim3(nb), dim3(jb), 0, ctx->stream, G, tau, j0, jb, Th,
+    hipLaunchKernelGGL(k_qr_form_t<true>, dim3(nb), dim3(256), 0, ctx->stream, G, tau, j0, jb, Th,
                        gstride, tstride);
     // W2 = T^H W = 0 - Th W
     hipLaunchKernelGGL(k_qr_zero, dim3((unsigned)((nb * wstride + 255) / 256)), dim3(256), 0,
@@ -276,7 +307,7 @@ int qb_house_apply_q(qb_ctx* ctx, const cd* V, int64_t N, int r, const cd* tau, 
   if (r <= QB_QR_NB) {
     for (int j = r - 1; j >= 0; --j)
       hipLaunchKernelGGL(k_house_apply<false>, dim3(ncols), dim3(256), 0, ctx->stream, V, N, Y, N,
-                         N, j, 0, tau, (int64_t)0, (int64_t)0);
+                         N, j, 0, const_cast<cd*>(tau), (int64_t)0, (int64_t)0, false);
     QB_HIP(ctx, hipGetLastError());
     return QB_OK;
   }
@@ -302,7 +333,7 @@ int qb_house_apply_q(qb_ctx* ctx, const cd* V, int64_t N, int r, const cd* tau, 
     rc = qb_qr_skinny(ctx, jb, jb, (int)m, Vh, Vb, m, part, G);
     if (!rc) rc = qb_qr_skinny(ctx, jb, ncols, (int)m, Vh, Y + j0, N, part, W);
     if (rc) break;
-    hipLaunchKernelGGL(k_qr_form_t<false>, dim3(1), dim3(jb), 0, ctx->stream, G, tau, j0, jb, Tn,
+    hipLaunchKernelGGL(k_qr_form_t<false>, dim3(1), dim3(256), 0, ctx->stream, G, tau, j0, jb, Tn,
                        (int64_t)0, (int64_t)0);
     // W2 = T W = 0 - (-T) W, then Y(j0:, :) -= V W2
     hipLaunchKernelGGL(k_qr_zero, dim3((unsigned)((wn + 255) / 256)), dim3(256), 0, ctx->stream,
