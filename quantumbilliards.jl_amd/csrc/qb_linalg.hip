@@ -49,6 +49,22 @@ __device__ __forceinline__ doublex4 mfma16(double a, double b, doublex4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// Tile of this workgroup of a (gx, gy, batch) grid.  Workgroups are dispatched
+// round-robin over the 8 XCDs (each with its own L2): those of one L mod 8 of a
+// matrix run on one XCD and take a contiguous range of tile ids, which walk groups
+// of `grp` m-tiles sweeping n, so that the workgroups resident on an XCD share A and B
+// panels in its L2.  Ranges differ by one tile where the count is no multiple of 8.
+__device__ __forceinline__ void xcd_tile(unsigned grp, int* mt, int* nt) {
+  const unsigned gx = gridDim.x, gy = gridDim.y, n = gx * gy;
+  const unsigned L = blockIdx.x + gx * blockIdx.y, x = L & 7u, rem = n & 7u;
+  const unsigned t = x * (n >> 3) + (x < rem ? x : rem) + (L >> 3);
+  const unsigned first = t / (grp * gy) * grp;
+  const unsigned gm = gx - first < grp ? gx - first : grp;
+  const unsigned loc = t - first * gy;
+  *mt = (int)(first + loc % gm);
+  *nt = (int)(loc / gm);
+}
+
 // ---------------------------------------------------------------------------
 // GEMM: C[b] -= A[b] * B[b]  (A: M x K, B: K x N, C: M x N)
 // ---------------------------------------------------------------------------
@@ -99,21 +115,7 @@ __global__ void __launch_bounds__(256, OCC) k_gemm_sub(int M, int N, int K, cons
   const int wm0 = (wave % WGM) * WM, wn0 = (wave / WGM) * WN;
   int mt = blockIdx.x, ntile = blockIdx.y;
   if constexpr (XCD) {
-    // Workgroups are dispatched round-robin over the 8 XCDs (each with its
-    // own L2).  Give XCD x a contiguous range of tile ids, and order tile
-    // ids in groups of 8 m-tiles sweeping n, so the workgroups resident on
-    // one XCD share A and B panels in its L2.  Only when the tile count is a
-    // multiple of 8 (every batch entry then starts on XCD 0).
-    const unsigned gx = gridDim.x, gy = gridDim.y, ntiles = gx * gy;
-    if ((ntiles & 7u) == 0) {
-      const unsigned L = blockIdx.x + gx * blockIdx.y;
-      const unsigned t = (L & 7u) * (ntiles >> 3) + (L >> 3);
-      const unsigned grp = t / (8u * gy), first = grp * 8u;
-      const unsigned gm = gx - first < 8u ? gx - first : 8u;
-      const unsigned loc = t - first * gy;
-      mt = (int)(first + loc % gm);
-      ntile = (int)(loc / gm);
-    }
+    xcd_tile(8, &mt, &ntile);
   }
   const int m0 = mt * BM, n0 = ntile * BN;
   const int64_t b = bix ? bix[blockIdx.z] : blockIdx.z;
@@ -374,16 +376,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC)
   int mt = blockIdx.x, ntile = blockIdx.y;
   if constexpr (XCD) {
     // the XCD-aware tile order of k_gemm_sub, in groups of GRP m-tiles
-    const unsigned gx = gridDim.x, gy = gridDim.y, ntiles = gx * gy;
-    if ((ntiles & 7u) == 0) {
-      const unsigned L = blockIdx.x + gx * blockIdx.y;
-      const unsigned t = (L & 7u) * (ntiles >> 3) + (L >> 3);
-      const unsigned grp = t / ((unsigned)GRP * gy), first = grp * (unsigned)GRP;
-      const unsigned gm = gx - first < (unsigned)GRP ? gx - first : (unsigned)GRP;
-      const unsigned loc = t - first * gy;
-      mt = (int)(first + loc % gm);
-      ntile = (int)(loc / gm);
-    }
+    xcd_tile(GRP, &mt, &ntile);
   }
   const int m0 = mt * BM + (wave % WGM) * WM, n0 = ntile * BN + (wave / WGM) * WN;
   if (m0 >= M || n0 >= N) return;  // the wave has no rows or columns (no barrier follows)
@@ -606,16 +599,7 @@ __global__ void __launch_bounds__(256, 1) k_gemm_bf6(int M, int N, int K, const 
   int mt = blockIdx.x, ntile = blockIdx.y;
   if constexpr (XCD) {
     // the XCD-aware tile order of k_gemm_sub
-    const unsigned gx = gridDim.x, gy = gridDim.y, ntiles = gx * gy;
-    if ((ntiles & 7u) == 0) {
-      const unsigned L = blockIdx.x + gx * blockIdx.y;
-      const unsigned t = (L & 7u) * (ntiles >> 3) + (L >> 3);
-      const unsigned grp = t / (8u * gy), first = grp * 8u;
-      const unsigned gm = gx - first < 8u ? gx - first : 8u;
-      const unsigned loc = t - first * gy;
-      mt = (int)(first + loc % gm);
-      ntile = (int)(loc / gm);
-    }
+    xcd_tile(8, &mt, &ntile);
   }
   const int m0 = mt * BM, n0 = ntile * BN;
   const int64_t b = bix ? bix[blockIdx.z] : blockIdx.z;
