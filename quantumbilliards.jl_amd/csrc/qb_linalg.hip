@@ -1753,6 +1753,16 @@ static bool panel_lean_beside(const qb_ctx* ctx, int M, int N, int K) {
   return !kGemmReg[1][v];
 }
 
+// The complex128 trailing updates that run on the int8 matrix cores (qb_rns.hip):
+// steps of the full panel width of 512 with at least kRnsMin rows left.  An
+// update takes 33 to 36 ps per entry there against 48.8 ps, and its slices 12.5
+// ps for each of 512 (M + N) elements: at 1024 rows the two meet.  Matrices
+// below 4096 rows have panels of 256 columns, where the residues gain nothing,
+// and panels of 512 cost them what the updates would win (1141 rows: 12.8 ms for
+// a window of 32 matrices against 12.4, 1792 rows: 24.6 against 24.1).
+static const int kRnsMin = 1024;
+static bool lu_rns(int n) { return qb_lu_nb(n) == 512 && n - 512 >= kRnsMin; }
+
 // One leaf: the rows per thread follow from the rows left, the columns held at
 // a time from the registers they then take (RPT * W = 32 for complex128, 64 for
 // complex64, at most the leaf's 32).
@@ -1761,6 +1771,19 @@ static void panel_leaf(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0
                        int* ipiv, int64_t sP, int* info, int batch) {
   constexpr int X = sizeof(T) == sizeof(cf) ? 2 : 1;
   const int m = n - c0;
+  if constexpr (sizeof(T) == sizeof(cd)) {
+    // beside the residue updates, whose one workgroup per CU ends every 74 us, eight
+    // waves find room: twice the columns at a time, half the reads of L (per
+    // leaf of N = 4100, 32 matrices: 2049 to 4096 rows 484 -> 314 us, 1025 to 2048 180 ->
+    // 147; up to 1024 101 either way)
+    if (m > 1024 && m <= 4096 && lu_rns(n)) {
+      if (m <= 2048)
+        launch_getf2<T, 512, 4, 8>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+      else
+        launch_getf2<T, 512, 8, 4>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+      return;
+    }
+  }
   if (m <= 512)
     launch_getf2<T, 256, 2, 16>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
   else if (m <= 1024)
@@ -1845,15 +1868,6 @@ int qb_getrf_first_panel(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int*
   return QB_OK;
 }
 
-// The complex128 trailing updates that run on the int8 matrix cores (qb_rns.hip):
-// steps of the full panel width of 512 with at least kRnsMin rows left.  An
-// update takes 33 to 36 ps per entry there against 48.8 ps, and its slices 12.5
-// ps for each of 512 (M + N) elements: at 1024 rows the two meet.  Matrices
-// below 4096 rows have panels of 256 columns, where the residues gain nothing,
-// and panels of 512 cost them what the updates would win (1141 rows: 12.8 ms for
-// a window of 32 matrices against 12.4, 1792 rows: 24.6 against 24.1).
-static const int kRnsMin = 1024;
-static bool lu_rns(int n) { return qb_lu_nb(n) == 512 && n - 512 >= kRnsMin; }
 int64_t qb_getrf_rns_bytes(int64_t n, int batch) {
   return lu_rns((int)n) ? qb_rns_bytes(n - 512, n - 512, batch) : 0;
 }
