@@ -847,7 +847,8 @@ static int gemm_default(int M, int N, int K, bool conc = false) {
   // bits are the same: every tile sums in the order of k.  Beside the lookahead
   // panel (conc) four workgroups leave its leaves no place (610 against 320 us per
   // leaf of N = 3072): there the 128 x 64 tile, 102 TFLOP/s.  A mixed window of 3072,
-  // 32 nodes: 140 ms with the 128 x 128 tile, 113 with 64 x 64 everywhere, 107 with both.
+  // 32 nodes: 140 ms with the 128 x 128 tile, 113 with 64 x 64 everywhere, 104 with both
+  // (and with faster norms, 5 ms of the difference).
   (void)M;
   if constexpr (sizeof(T) == sizeof(cf))
     return conc ? 3 : 12;
