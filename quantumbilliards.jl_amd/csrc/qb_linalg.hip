@@ -997,11 +997,15 @@ __device__ __forceinline__ T cinv_(T a) {
   const auto den = fma_(a.re, a.re, a.im * a.im);
   return T{a.re / den, -a.im / den};
 }
-// x -= a y, four fused multiply-adds
+// x -= a y: the product first, so that a term rounds the running value once.  Four
+// multiply-adds into x would round it twice (rms backward error of a 32-row solve
+// 0.089 against 0.076 u |L||U||x|, of a 32-column LU 5.2 against 4.7 u) and save
+// 2 to 3 % of windows of 530 to 1792 nodes, 1 % of ones of 3072 and 4100.
 template <typename T>
 __device__ __forceinline__ void cnma_(T& x, const T& a, const T& y) {
-  x.re = fma_(a.im, y.im, fma_(-a.re, y.re, x.re));
-  x.im = fma_(-a.im, y.re, fma_(-a.re, y.im, x.im));
+  const T p = cmul_(a, y);
+  x.re -= p.re;
+  x.im -= p.im;
 }
 
 // A[i] when ok, else 0, loaded component by component (a conditional
@@ -1637,7 +1641,10 @@ __global__ void __launch_bounds__(256, 4) k_trsm_leaf(int n, int nrhs, const T* 
         const T xj = T{quad_bcast<(j & 3)>(v[j >> 2].re), quad_bcast<(j & 3)>(v[j >> 2].im)};
         cnma_(v[s0], Ls[ib + g][j], xj);
         cnma_(v[s0 + 1], Ls[ib + 4 + g][j], xj);
-        if ((j & 3) == 3) asm volatile("" ::: "memory");
+        // the next solved rows are broadcast after this point, not all at the start:
+        // 64 VGPRs, where 128 and 18 spilled took 10.8 instead of 9.2 us
+        if constexpr ((j & 3) == 3 && j < 31)
+          asm volatile("" : "+v"(v[(j >> 2) + 1].re), "+v"(v[(j >> 2) + 1].im)::"memory");
       });
       static_for<0, 8>([&](auto aa) {
         constexpr int a = 7 - decltype(aa)::value, sa = s0 + (a >> 2);
