@@ -26,6 +26,10 @@ template <typename T>
 int qb_getrf_first_panel(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipiv,
                          int64_t sP, int* info, int batch);
 int qb_lu_nb(int n);
+struct QbLeaf {
+  int threads, rows, cols;  // threads = 0: k_getf2_long
+};
+QbLeaf qb_panel_leaf_form(bool c128, int n, int m, bool beside_fp64);
 // Residue buffers that qb_getrf_batched<cd> takes for the time of its call.
 int64_t qb_getrf_rns_bytes(int64_t n, int batch);
 // qb_getrf_batched through a cached hipGraph when ctx->graphs is set and

@@ -71,6 +71,34 @@ int qbt_trsm_c64(qb_ctx* c, int n, const cf* LU, cf* B, int nrhs, int b) {
   return run_trsm<cf>(c, n, LU, B, nrhs, b);
 }
 void qbt_set_trsm_leaf_lds(int mode) { qb_set_trsm_leaf_lds(mode); }
+
+// The first panel (w columns) of an n x n complex128 LU: A is n x w, ipiv w.
+int qbt_first_panel_c128(qb_ctx* ctx, int n, int w, cd* A, int* ipiv) {
+  if (w != (n < qb_lu_nb(n) ? n : qb_lu_nb(n))) return QB_E_ARG;
+  cd* dA = nullptr;
+  int *dP = nullptr, *dI = nullptr;
+  const size_t a = (size_t)n * w * sizeof(cd), p = w * sizeof(int);
+  bool ok = hipMalloc(&dA, a) == hipSuccess && hipMalloc(&dP, p) == hipSuccess &&
+            hipMalloc(&dI, sizeof(int)) == hipSuccess &&
+            hipMemcpy(dA, A, a, hipMemcpyHostToDevice) == hipSuccess &&
+            hipMemset(dI, 0, sizeof(int)) == hipSuccess && hipDeviceSynchronize() == hipSuccess;
+  int rc = ok ? qb_getrf_first_panel<cd>(ctx, dA, n, n, (int64_t)n * w, dP, w, dI, 1) : QB_E_HIP;
+  ok = ok && hipDeviceSynchronize() == hipSuccess &&
+       hipMemcpy(A, dA, a, hipMemcpyDeviceToHost) == hipSuccess &&
+       hipMemcpy(ipiv, dP, p, hipMemcpyDeviceToHost) == hipSuccess;
+  hipFree(dA);
+  hipFree(dP);
+  hipFree(dI);
+  return rc ? rc : ok ? QB_OK : QB_E_HIP;
+}
+
+// threads, rows and columns of a leaf (qb_panel_leaf_form).
+void qbt_leaf_form(int c128, int n, int m, int beside_fp64, int* out) {
+  const QbLeaf f = qb_panel_leaf_form(c128 != 0, n, m, beside_fp64 != 0);
+  out[0] = f.threads;
+  out[1] = f.rows;
+  out[2] = f.cols;
+}
 }
 
 // Timing of gemm_sub at one shape: buffers filled on the device, `iters`

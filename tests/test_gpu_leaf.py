@@ -5,6 +5,7 @@ import os
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 pytestmark = pytest.mark.gpu
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -141,3 +142,35 @@ def test_solves_at_their_edges(probe, dt, lower, n, nrhs):
     x = X.transpose(0, 2, 1).astype(np.clongdouble)
     t = T.astype(np.clongdouble)
     assert np.all(np.abs(B - t @ x) <= 4 * (n + 4) * u * (np.abs(t) @ np.abs(x)))
+
+
+# one row more than the leaf of four waves takes, the most of eight waves, one row more
+@pytest.mark.parametrize("n", [4097, 8192, 8193])
+def test_long_panel(probe, n):
+    """A panel P^T L U with sparse dyadic factors, whose sums are exact and whose pivots
+    are unique: both come back bit for bit."""
+    L, ctx = probe
+    rng = np.random.default_rng(n)
+    w, unit = 512, np.array([1, -1, 1j, -1j])
+    i, j = rng.integers(0, n, 6 * n), rng.integers(0, w, 6 * n)
+    low, upp = i > j, (i < j) & (i < w)
+    Lm = np.zeros((n, w), complex)
+    Um = np.zeros((w, w), complex)
+    Lm[i[low], j[low]] = rng.choice([0.5, 0.25], low.sum()) * rng.choice(unit, low.sum())
+    Um[i[upp], j[upp]] = rng.choice([1.0, 2.0], upp.sum()) * rng.choice(unit, upp.sum())
+    d = np.arange(w)
+    Lm[d, d] = 1
+    Um[d, d] = rng.choice([4.0, 8.0], w) * rng.choice(unit, w)
+    perm = rng.permutation(n)
+    A = np.empty((w, n), complex)  # [column][row]; row perm[i] is row i of L U
+    A[:, perm] = (sp.csr_matrix(Lm) @ sp.csr_matrix(Um)).toarray().T
+    ipiv = np.zeros(w, np.int32)
+    assert L.qbt_first_panel_c128(ctx, n, w, _p(A), _p(ipiv)) == 0
+    order = np.arange(n)
+    for s, q in enumerate(ipiv):
+        order[s], order[q] = order[q], order[s]
+    assert np.array_equal(order[:w], perm[:w])
+    inv = np.argsort(perm)
+    ref = Lm[inv[order]]
+    ref[:w] = np.tril(ref[:w], -1) + Um
+    assert np.array_equal(A.T, ref)
