@@ -1094,15 +1094,10 @@ __device__ __forceinline__ int swap_source(int x, int k0, const int* p, int kb, 
 // What bounds it: the latency of 32 column steps (one LDS barrier each) and of
 // 32/W changes of sub-block, and with many rows the L2 bandwidth of one CU, which
 // reads 32/W * 16 columns.  Four waves of 256 VGPRs (half a CU) find room beside
-// a trailing-update workgroup that ends; eight waited for both of a CU's.  The leaf that this one replaces kept its columns in
-// global memory (one workgroup too) and took, on average over the leaves of an
-// N = 530 and an N = 1792 window (32 matrices), 172 and 254 us; this one takes 90
-// and 93 (up to 512 rows), 106 (1024) and 185 us (2048).  Up to 8192 rows eight
-// waves hold two complex128 columns at a time; beside the residue updates
-// (qb_rns.hip), whose workgroups end every 74 us, they take 0.99 ms per leaf of an
-// N = 8192 window (48 matrices), k_getf2_long 2.56 ms there (window: 1019 against
-// 1043 ms).  k_getf2_long takes longer columns, and complex64 ones above 4096 rows,
-// which run beside the FP32 tiles: there the eight waves wait for room.
+// a trailing-update workgroup that ends; eight wait for both of a CU's, unless the
+// update leaves places often (qb_panel_leaf_form).  Per leaf of N = 530 and N = 1792
+// windows (32 matrices), on average: 94 and 96 us (up to 512 rows), 110 (1024) and 193
+// (2048); with the columns in global memory (k_getf2_long's order) 172 and 254 us.
 // ---------------------------------------------------------------------------
 template <typename T, int NT, int RPT, int W>
 __global__ void __launch_bounds__(NT) k_getf2(T* __restrict__ A, int64_t lda, int64_t sA, int n,
@@ -1340,11 +1335,11 @@ static void launch_getf2(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int 
                      c0, w, ipiv, sP, info);
 }
 
-// The same leaf for more than 4096 rows: left-looking (Crout) order with the columns in global memory.  Step
-// c forms the U part of column c by forward substitution with the unit-lower
-// top block kept in LDS, updates the rest of column c with all previous L
-// columns at once, picks the pivot, swaps the pivot row into place across the
-// w columns and scales the column.
+// The same leaf for columns too long for registers: left-looking (Crout) order with
+// the columns in global memory.  Step c forms the U part of column c by forward
+// substitution with the unit-lower top block kept in LDS, updates the rest of
+// column c with all previous L columns at once, picks the pivot, swaps the pivot row
+// into place across the w columns and scales the column.
 template <typename T>
 __global__ void __launch_bounds__(512) k_getf2_long(T* __restrict__ A, int64_t lda, int64_t sA,
                                                     int n, int c0, int w, int* __restrict__ ipiv,
@@ -1771,55 +1766,68 @@ static bool panel_lean_beside(const qb_ctx* ctx, int M, int N, int K) {
 static const int kRnsMin = 1024;
 static bool lu_rns(int n) { return qb_lu_nb(n) == 512 && n - 512 >= kRnsMin; }
 
-// One leaf: the rows per thread follow from the rows left, the columns held at
-// a time from the registers they then take (RPT * W = 32 for complex128, 64 for
-// complex64, at most the leaf's 32).
+// The form of a leaf of m rows of an n x n matrix: threads, rows per thread and columns
+// held at a time of k_getf2 (rows x columns per thread: 32 for complex128, 64 for
+// complex64, at most the leaf's 32 columns), or zeros for k_getf2_long.  beside_fp64:
+// the panel runs beside an FP64 trailing update.
+//   complex128 with 512-wide panels, 1025 to 4096 rows: eight waves, twice the columns
+//   at a time and half the reads of L.  Per leaf of N = 4100 (32 matrices) beside the
+//   residue updates, 2049 to 4096 rows: 314 us, four waves 484; 1025 to 2048: 147 and
+//   180; up to 1024 101 either way.  Beside FP64 updates a window of 4100 takes 155 ms,
+//   with four waves 161.
+//   complex128, 4097 to 8192 rows: 0.99 ms per leaf beside the residue updates (N =
+//   8192, 48 matrices), k_getf2_long 2.56; beside FP64 updates k_getf2_long, whose
+//   registers leave room for their waves: windows of 6000 and 8192 394 ms and 1.245 s,
+//   against 417 ms and 1.30 s.
+//   complex64 above 4096 rows: k_getf2_long, beside the FP32 tiles.
+QbLeaf qb_panel_leaf_form(bool c128, int n, int m, bool beside_fp64) {
+  const int x = c128 ? 1 : 2;
+  if (c128 && lu_rns(n) && m > 1024 && m <= 4096)
+    return m <= 2048 ? QbLeaf{512, 4, 8} : QbLeaf{512, 8, 4};
+  if (m <= 512) return {256, 2, 16};
+  if (m <= 1024) return {256, 4, 8 * x};
+  if (m <= 2048) return {256, 8, 4 * x};
+  if (m <= 4096) return {256, 16, 2 * x};
+  if (c128 && m <= 8192 && !beside_fp64) return {512, 16, 2};
+  return {0, 0, 0};
+}
+
 template <typename T>
 static void panel_leaf(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, int w,
-                       int* ipiv, int64_t sP, int* info, int batch) {
-  constexpr int X = sizeof(T) == sizeof(cf) ? 2 : 1;
-  const int m = n - c0;
-  if constexpr (sizeof(T) == sizeof(cd)) {
-    // beside the residue updates, whose one workgroup per CU ends every 74 us, eight
-    // waves find room: twice the columns at a time, half the reads of L (per
-    // leaf of N = 4100, 32 matrices: 2049 to 4096 rows 484 -> 314 us, 1025 to 2048 180 ->
-    // 147; up to 1024 101 either way)
-    if (m > 1024 && m <= 4096 && lu_rns(n)) {
-      if (m <= 2048)
-        launch_getf2<T, 512, 4, 8>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-      else
-        launch_getf2<T, 512, 8, 4>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-      return;
-    }
-  }
-  if (m <= 512)
-    launch_getf2<T, 256, 2, 16>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-  else if (m <= 1024)
-    launch_getf2<T, 256, 4, 8 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-  else if (m <= 2048)
-    launch_getf2<T, 256, 8, 4 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-  else if (m <= 4096)
-    launch_getf2<T, 256, 16, 2 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-  else if (m <= 8192 && sizeof(T) == sizeof(cd))
-    launch_getf2<T, 512, 16, 2 * X>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
-  else
+                       int* ipiv, int64_t sP, int* info, int batch, bool beside_fp64) {
+  constexpr bool C128 = sizeof(T) == sizeof(cd);
+  constexpr int X = C128 ? 1 : 2;
+  const QbLeaf f = qb_panel_leaf_form(C128, n, n - c0, beside_fp64);
+  if (f.threads == 0) {
     hipLaunchKernelGGL(k_getf2_long<T>, dim3(batch), dim3(512), 0, ctx->stream, A, lda, sA, n, c0,
                        w, ipiv, sP, info);
+  } else if (f.threads == 256) {
+    auto* k = f.rows == 2   ? &launch_getf2<T, 256, 2, 16>
+              : f.rows == 4 ? &launch_getf2<T, 256, 4, 8 * X>
+              : f.rows == 8 ? &launch_getf2<T, 256, 8, 4 * X>
+                            : &launch_getf2<T, 256, 16, 2 * X>;
+    k(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  } else if constexpr (C128) {
+    auto* k = f.rows == 4   ? &launch_getf2<T, 512, 4, 8>
+              : f.rows == 8 ? &launch_getf2<T, 512, 8, 4>
+                            : &launch_getf2<T, 512, 16, 2>;
+    k(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+  }
 }
 
 // Recursive panel: factor columns [c0, c0+w) (rows c0..n-1) of every matrix.
 template <typename T>
 static int panel_rec(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, int w, int* ipiv,
-                     int64_t sP, int* info, int batch) {
+                     int64_t sP, int* info, int batch, bool beside_fp64) {
   if (w <= 32) {
     int slot = qb_prof_begin(ctx, QB_K_PANEL, 8.0 * (double)(n - c0) * w * w / 2 * batch, 0);
-    panel_leaf<T>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch);
+    panel_leaf<T>(ctx, A, lda, sA, n, c0, w, ipiv, sP, info, batch, beside_fp64);
     qb_prof_end(ctx, slot);
     QB_HIP(ctx, hipGetLastError());
     return QB_OK;
   }
   int w1 = split32(w);
-  int rc = panel_rec(ctx, A, lda, sA, n, c0, w1, ipiv, sP, info, batch);
+  int rc = panel_rec(ctx, A, lda, sA, n, c0, w1, ipiv, sP, info, batch, beside_fp64);
   if (rc) return rc;
   rc = laswp(ctx, A, lda, sA, c0 + w1, c0 + w, c0, c0 + w1, ipiv, sP, batch);
   if (rc) return rc;
@@ -1831,7 +1839,8 @@ static int panel_rec(qb_ctx* ctx, T* A, int64_t lda, int64_t sA, int n, int c0, 
                    A + c0 + (int64_t)(c0 + w1) * lda, lda, sA,
                    A + c0 + w1 + (int64_t)(c0 + w1) * lda, lda, sA, batch);
   if (rc) return rc;
-  rc = panel_rec(ctx, A, lda, sA, n, c0 + w1, w - w1, ipiv, sP, info, batch);
+  rc = panel_rec(ctx, A, lda, sA, n, c0 + w1, w - w1, ipiv, sP, info, batch,
+                 beside_fp64);
   if (rc) return rc;
   return laswp(ctx, A, lda, sA, c0, c0 + w1, c0 + w1, c0 + w, ipiv, sP, batch);
 }
@@ -1869,7 +1878,7 @@ int qb_getrf_first_panel(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int*
   QB_HIP(ctx, hipEventRecord(ctx->ev_main, main));
   QB_HIP(ctx, hipStreamWaitEvent(aux, ctx->ev_main, 0));
   ctx->stream = aux;
-  const int rc = panel_rec(ctx, A, lda, sA, n, 0, n < NB ? n : NB, ipiv, sP, info, batch);
+  const int rc = panel_rec(ctx, A, lda, sA, n, 0, n < NB ? n : NB, ipiv, sP, info, batch, false);
   ctx->stream = main;
   if (rc) return rc;
   QB_HIP(ctx, hipEventRecord(ctx->ev_first, aux));
@@ -1900,7 +1909,7 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
   if (first_done)
     QB_HIP(ctx, hipStreamWaitEvent(main, ctx->ev_first, 0));
   else
-    rc = panel_rec(ctx, A, lda, sA, n, 0, n < NB ? n : NB, ipiv, sP, info, batch);
+    rc = panel_rec(ctx, A, lda, sA, n, 0, n < NB ? n : NB, ipiv, sP, info, batch, false);
   if (rc) return rc;
   // Residue buffers of the complex128 trailing updates; without room for them,
   // and under capture (no allocation there), every update takes the FP64 tiles.
@@ -1958,7 +1967,8 @@ int qb_getrf_batched(qb_ctx* ctx, T* A, int n, int64_t lda, int64_t sA, int* ipi
     QB_HIP(ctx, hipStreamWaitEvent(aux, ctx->ev_main, 0));
     rc = on_aux([&] {
       ctx->panel_lean = m > kb1 && panel_lean_beside<T>(ctx, m, m - kb1, kb);
-      const int r = panel_rec(ctx, A, lda, sA, n, k1, kb1, ipiv, sP, info, batch);
+      const int r = panel_rec(ctx, A, lda, sA, n, k1, kb1, ipiv, sP, info, batch,
+                              m > kb1 && !rns_step);
       ctx->panel_lean = false;
       return r;
     });
