@@ -998,12 +998,25 @@ __device__ __forceinline__ T cinv_(T a) {
   return T{a.re / den, -a.im / den};
 }
 // x -= a y: the product first, so that a term rounds the running value once.  Four
-// multiply-adds into x would round it twice (rms backward error of a 32-row solve
-// 0.089 against 0.076 u |L||U||x|, of a 32-column LU 5.2 against 4.7 u) and save
-// 2 to 3 % of windows of 530 to 1792 nodes, 1 % of ones of 3072 and 4100.
+// multiply-adds into x would round it twice: rms backward error of a 32-row solve
+// 0.089 against 0.076 u |L||U||x|, of a 32-column LU 5.2 against 4.7 u.
 template <typename T>
 __device__ __forceinline__ void cnma_(T& x, const T& a, const T& y) {
   const T p = cmul_(a, y);
+  x.re -= p.re;
+  x.im -= p.im;
+}
+// x -= sum a[u] y[u] of U terms, summed first: x rounds once for all of them, and the
+// terms take 4 U + 2 operations instead of 6 U (0.070 and 4.6 u where the leaves use it;
+// windows of 530 to 1792 nodes 1 to 2 % faster than with every term by itself).
+template <int U, typename T>
+__device__ __forceinline__ void cnma_sum_(T& x, const T* a, const T* y) {
+  T p = cmul_(a[0], y[0]);
+#pragma unroll
+  for (int u = 1; u < U; ++u) {
+    p.re = fma_(-a[u].im, y[u].im, fma_(a[u].re, y[u].re, p.re));
+    p.im = fma_(a[u].im, y[u].re, fma_(a[u].re, y[u].im, p.im));
+  }
   x.re -= p.re;
   x.im -= p.im;
 }
@@ -1096,7 +1109,7 @@ __device__ __forceinline__ int swap_source(int x, int k0, const int* p, int kb, 
 // reads 32/W * 16 columns.  Four waves of 256 VGPRs (half a CU) find room beside
 // a trailing-update workgroup that ends; eight wait for both of a CU's, unless the
 // update leaves places often (qb_panel_leaf_form).  Per leaf of N = 530 and N = 1792
-// windows (32 matrices), on average: 94 and 96 us (up to 512 rows), 110 (1024) and 193
+// windows (32 matrices), on average: 91 and 95 us (up to 512 rows), 113 (1024) and 179
 // (2048); with the columns in global memory (k_getf2_long's order) 172 and 254 us.
 // ---------------------------------------------------------------------------
 template <typename T, int NT, int RPT, int W>
@@ -1155,30 +1168,31 @@ __global__ void __launch_bounds__(NT) k_getf2(T* __restrict__ A, int64_t lda, in
       }
       lds_barrier();
       // rows below: a -= L(:, 0..s-1) U
-      constexpr int QC = RPT < 4 ? RPT : 4, UN = RPT == 1 ? 8 : 16 / (2 * QC);
+      // UN terms summed before they reach a, QC rows at a time: as many as registers allow
+      constexpr int UN = W >= 8 || (W == 4 && NT == 256) ? 4 : 2;
+      constexpr int QC = W >= 8 && sizeof(S) == 8 ? 2 : RPT < 4 ? RPT : 4;
 #pragma unroll
       for (int q0 = 0; q0 < RPT; q0 += QC) {
         int i = 0;
         for (; i + UN <= s; i += UN) {
-          T l[UN][QC];
+          T l[QC][UN];
 #pragma unroll
           for (int u = 0; u < UN; ++u)
 #pragma unroll
             for (int q = 0; q < QC; ++q) {
               const T* p = A + (int64_t)(i + u) * lda + ro[q0 + q];
-              l[u][q].re = p->re;
-              l[u][q].im = p->im;
+              l[q][u].re = p->re;
+              l[q][u].im = p->im;
             }
 #pragma unroll
-          for (int u = 0; u < UN; ++u) {
+          for (int k = 0; k < W; ++k) {
+            // U read a column at a time: few registers
+            if (k * UN % 4 == 0) asm volatile("" ::: "memory");
+            T uk[UN];
 #pragma unroll
-            for (int k = 0; k < W; ++k) {
-              // U read a few columns at a time: few registers
-              if ((k & 3) == 0) asm volatile("" ::: "memory");
-              const T uk = Us[i + u][k];
+            for (int u = 0; u < UN; ++u) uk[u] = Us[i + u][k];
 #pragma unroll
-              for (int q = 0; q < QC; ++q) cnma_(a[q0 + q][k], l[u][q], uk);
-            }
+            for (int q = 0; q < QC; ++q) cnma_sum_<UN>(a[q0 + q][k], l[q], uk);
           }
         }
         for (; i < s; ++i)
@@ -1575,18 +1589,16 @@ __device__ __forceinline__ float quad_bcast(float x) {
 }
 
 // ---------------------------------------------------------------------------
-// Triangular-solve leaf, n <= 32 rows: X = L^{-1} B (unit lower) or
-// X = U^{-1} B (upper).  Four lanes per
-// column (64 columns per workgroup of 256 threads): lane g holds the rows
-// 4 s + g, s < 8, in registers, a solved row reaches the other three by a DPP
-// quad broadcast, and the triangle stands in LDS (17 KB).  All loads of a
-// lane are issued before the first is used.  What bounds it is latency: one
-// load, the chain of 32 rows, one store.  It takes 6 us for the 32 x 64 leaves of
-// an N = 530 window's solves and 8 us for the panel's, where the one-lane-per-column
-// leaf that it replaces (staged through LDS load by load) took 28 us; with
-// thousands of right-hand sides (the LU's block rows) it beats the leaf that held
-// a whole column per lane as well (LU of 240 matrices of 1640: 113.3 against
-// 115.6 ms per window, of 48 of 8192: 1.228 against 1.238 s).
+// Triangular-solve leaf, n <= 32 rows: X = L^{-1} B (unit lower) or X = U^{-1} B
+// (upper).  Four lanes per column (64 columns per workgroup of 256 threads): lane g
+// holds the rows 4 s + g, s < 8, in registers, a solved row reaches the other three by
+// a DPP quad broadcast, and the triangle stands in LDS (17 KB).  All loads of a lane
+// are issued before the first is used.  What bounds it is latency: one load, the chain
+// of 32 rows, one store: 6.2 us for the 32 x 64 leaves of an N = 530 window's solves, 8
+// us for the upper ones (a lane per column, staged through LDS: 28 us).  With thousands
+// of right-hand sides (the LU's block rows) it beats a whole column per lane as well
+// (LU of 240 matrices of 1640: 113.3 against 115.6 ms per window, of 48 of 8192: 1.228
+// against 1.238 s).
 // ---------------------------------------------------------------------------
 template <typename T, bool UNIT_LOWER>
 __global__ void __launch_bounds__(256, 4) k_trsm_leaf(int n, int nrhs, const T* __restrict__ L,
@@ -1610,16 +1622,27 @@ __global__ void __launch_bounds__(256, 4) k_trsm_leaf(int n, int nrhs, const T* 
   for (int t = 0; t < 4; ++t) Ls[(tid + 256 * t) & 31][(tid + 256 * t) >> 5] = l[t];
   __syncthreads();
   if (UNIT_LOWER) {
-    static_for<0, 31>([&](auto jj) {
-      constexpr int j = decltype(jj)::value, s0 = j >> 2, o = j & 3;
-      const T xj = T{quad_bcast<o>(v[s0].re), quad_bcast<o>(v[s0].im)};
-      T t = v[s0];  // selected, not branched over: the updates stay in one block
-      cnma_(t, Ls[4 * s0 + g][j], xj);
-      v[s0].re = g > o ? t.re : v[s0].re;
-      v[s0].im = g > o ? t.im : v[s0].im;
+    // four rows at a time: among themselves, then in the rows below at once
+    static_for<0, 8>([&](auto ss) {
+      constexpr int s0 = decltype(ss)::value;
+      T x[4];
+      static_for<0, 4>([&](auto oo) {
+        constexpr int o = decltype(oo)::value;
+        x[o] = T{quad_bcast<o>(v[s0].re), quad_bcast<o>(v[s0].im)};
+        if constexpr (o < 3) {
+          T t = v[s0];  // selected, not branched over: the updates stay in one block
+          cnma_(t, Ls[4 * s0 + g][4 * s0 + o], x[o]);
+          v[s0].re = g > o ? t.re : v[s0].re;
+          v[s0].im = g > o ? t.im : v[s0].im;
+        }
+      });
 #pragma unroll
-      for (int s = s0 + 1; s < 8; ++s) cnma_(v[s], Ls[4 * s + g][j], xj);
-      if (j & 1) asm volatile("" ::: "memory");  // LDS reads of two rows at a time
+      for (int s = s0 + 1; s < 8; ++s) {
+        const T l[4] = {Ls[4 * s + g][4 * s0], Ls[4 * s + g][4 * s0 + 1], Ls[4 * s + g][4 * s0 + 2],
+                        Ls[4 * s + g][4 * s0 + 3]};
+        cnma_sum_<4>(v[s], l, x);
+        if (s & 1) asm volatile("" ::: "memory");  // LDS reads of two slots at a time
+      }
     });
   } else {
     if (tid < 32) {
@@ -1631,24 +1654,33 @@ __global__ void __launch_bounds__(256, 4) k_trsm_leaf(int n, int nrhs, const T* 
     // in ascending order, then the block's own rows
     static_for<0, 4>([&](auto bb) {
       constexpr int ib = 24 - 8 * decltype(bb)::value, s0 = ib >> 2;
-      static_for<ib + 8, 32>([&](auto jj) {
-        constexpr int j = decltype(jj)::value;
-        const T xj = T{quad_bcast<(j & 3)>(v[j >> 2].re), quad_bcast<(j & 3)>(v[j >> 2].im)};
-        cnma_(v[s0], Ls[ib + g][j], xj);
-        cnma_(v[s0 + 1], Ls[ib + 4 + g][j], xj);
-        // the next solved rows are broadcast after this point, not all at the start:
-        // 64 VGPRs, where 128 and 18 spilled took 10.8 instead of 9.2 us
-        if constexpr ((j & 3) == 3 && j < 31)
-          asm volatile("" : "+v"(v[(j >> 2) + 1].re), "+v"(v[(j >> 2) + 1].im)::"memory");
+      static_for<s0 + 2, 8>([&](auto ss) {
+        constexpr int s = decltype(ss)::value;
+        const T x[4] = {T{quad_bcast<0>(v[s].re), quad_bcast<0>(v[s].im)},
+                        T{quad_bcast<1>(v[s].re), quad_bcast<1>(v[s].im)},
+                        T{quad_bcast<2>(v[s].re), quad_bcast<2>(v[s].im)},
+                        T{quad_bcast<3>(v[s].re), quad_bcast<3>(v[s].im)}};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const T* u = &Ls[ib + 4 * h + g][4 * s];
+          const T l[4] = {u[0], u[1], u[2], u[3]};
+          cnma_sum_<4>(v[s0 + h], l, x);
+        }
+        // the next solved rows are broadcast after this point, not all at the start
+        if constexpr (s < 7) asm volatile("" : "+v"(v[s + 1].re), "+v"(v[s + 1].im)::"memory");
       });
       static_for<0, 8>([&](auto aa) {
         constexpr int a = 7 - decltype(aa)::value, sa = s0 + (a >> 2);
         T x = v[sa];
-        static_for<a + 1, 8>([&](auto cc) {
-          constexpr int c = decltype(cc)::value, sc = s0 + (c >> 2);
-          const T xc = T{quad_bcast<(c & 3)>(v[sc].re), quad_bcast<(c & 3)>(v[sc].im)};
-          cnma_(x, Ls[ib + a][ib + c], xc);
-        });
+        if constexpr (a < 7) {  // the row solved last comes last
+          T l[7 - a], xs[7 - a];
+          static_for<0, 7 - a>([&](auto uu) {
+            constexpr int u = decltype(uu)::value, c = 7 - u, sc = s0 + (c >> 2);
+            l[u] = Ls[ib + a][ib + c];
+            xs[u] = T{quad_bcast<(c & 3)>(v[sc].re), quad_bcast<(c & 3)>(v[sc].im)};
+          });
+          cnma_sum_<7 - a>(x, l, xs);
+        }
         const T d = Ls[ib + a][ib + a];
         x = cmul_(x, d);
         v[sa].re = g == (a & 3) ? x.re : v[sa].re;
