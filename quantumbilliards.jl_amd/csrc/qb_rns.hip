@@ -279,7 +279,7 @@ __global__ void __launch_bounds__(512, 2)
           "global_load_lds_dwordx4 %1, %2"
           :
           : "s"(lds0 + ld_off + (3 * w + u) * 1024), "v"(voff), "s"(src[u])
-          : "memory");
+          : "memory", "m0");
       src[u] += 4096;
     }
     ld_off = ld_off == (RNS_S - 1) * RNS_STAGE ? 0 : ld_off + RNS_STAGE;
