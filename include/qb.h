@@ -108,9 +108,13 @@ int qb_ctx_set_graphs(qb_ctx* ctx, int32_t on);
 
 /* Let large FP64 factorisations take residue buffers for the time of the LU
  * (on by default): their trailing updates then run on the int8 matrix cores,
- * at FP64 accuracy and about 1.4 times the speed of the FP64 ones.  Off, or
- * where the buffers do not fit, they run on the FP64 matrix cores.  No
- * reference counterpart. */
+ * at about 1.4 times the speed of the FP64 ones, with errors of at most a few
+ * 2^-53 of (largest entry of the row) x (largest entry of the column) per
+ * term, which on the matrices of these operators is less than the FP64
+ * updates' own.  Off, or where the buffers do not fit, they run on the FP64
+ * matrix cores; the two differ in rounding, so a caller that wants the same
+ * bits whatever memory is free sets it off (the launches of QB_K_GEMM_C128_I8
+ * tell which ran).  No reference counterpart. */
 int qb_ctx_set_residue_buffers(qb_ctx* ctx, int32_t on);
 
 /* Free and total device memory of the context's GPU (hipMemGetInfo); the

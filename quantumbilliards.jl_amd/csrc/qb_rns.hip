@@ -6,9 +6,19 @@
 // to integers, column j of B likewise; the product of the integers is formed
 // exactly modulo M = prod m_l (117.7 bits) by the Chinese remainder theorem
 // (the scheme of Ozaki, Uchino and Imamura, "Ozaki scheme II"), scaled back and
-// subtracted.  The only errors are the rounding of the operands to 53 bits
-// below the row's / column's largest entry and of the result: for K = 512 no
-// more than the FP64 kernel's, whose sums round at every step.
+// subtracted.
+//
+// Accuracy.  An operand's entry keeps 53 bits below the largest component of its row
+// (A) or column (B), m_i = max_k |a_ik|, n_j = max_k |b_kj|, and the product itself is
+// exact to about u m_i n_j (u = 2^-53), so that
+//   |error_ij| <= 2 u (m_i sum_k |b_kj| + n_j sum_k |a_ik|) + 16 u m_i n_j
+// and a rounding of C.  An FP64 sum errs by multiples of u sum_k |a_ik| |b_kj|: this is
+// less unless entries grow along k in A and fall in B alike (rows of very unequal
+// scales, before the LU).  With products of equal size, graded by 2^10 / 2^20 / 2^40
+// along k, the residues err by 9e-15 / 6e-12 / 4e-6 of sum |a||b|, an FP64 sum by 1e-16.
+// The factors of this library's operators are not graded so (row maximum 1.4 to 2.5
+// times the median): there the error is 1/15 to 1/150 of that of the three-product FP64
+// tiles, and no more with growths e^(|Im k| r) of 1e18 across a matrix.
 //
 // Every modulus is a product of primes = 1 mod 4, so -1 has a square root j_l
 // modulo m_l, and a + b i -> (a + j_l b, a - j_l b) maps the complex numbers
