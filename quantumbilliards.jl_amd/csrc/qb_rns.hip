@@ -283,13 +283,11 @@ __global__ void __launch_bounds__(512, 2)
   auto load_stage = [&] {
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
-      asm volatile(
-          "s_mov_b32 m0, %0\n\t"
-          "s_nop 0\n\t"
-          "global_load_lds_dwordx4 %1, %2"
-          :
-          : "s"(lds0 + ld_off + (3 * w + u) * 1024), "v"(voff), "s"(src[u])
-          : "memory", "m0");
+      // m0 holds the LDS address (an operand: the compiler sets it); one wait state
+      asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :
+                   : "v"(voff), "s"(src[u]), "{m0}"(lds0 + ld_off + (3 * w + u) * 1024)
+                   : "memory");
       src[u] += 4096;
     }
     ld_off = ld_off == (RNS_S - 1) * RNS_STAGE ? 0 : ld_off + RNS_STAGE;

@@ -1,5 +1,6 @@
-"""Inline assembly that writes m0 says so: the compiler keeps values of its own there
-(LDS loads, indexed moves) and does not look into the text."""
+"""Inline assembly that needs m0 (global loads into LDS take their LDS address from it)
+says so, as an operand or as overwritten: the compiler keeps values of its own there and
+does not look into the text."""
 import glob
 import os
 import re
@@ -21,8 +22,10 @@ def test_m0_is_declared():
     seen = 0
     for f in sorted(glob.glob(os.path.join(CSRC, "*.h*"))):
         for s in _statements(open(f).read()):
-            if not re.search(r"s_mov\w*\s+m0\s*,", s):
+            if not re.search(r"\bm0\s*,|_load_lds_", s):
                 continue
             seen += 1
-            assert '"m0"' in s.rsplit(":", 1)[-1], (os.path.basename(f), s)
+            written = re.search(r"\bs_\w+\s+m0\s*,", s)
+            ok = '"m0"' in s.rsplit(":", 1)[-1] if written else '"{m0}"(' in s
+            assert ok, (os.path.basename(f), s)
     assert seen
