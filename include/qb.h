@@ -231,10 +231,14 @@ int64_t qb_geom_dim(const qb_geom* g);
  * out[q*N*N + i + j*N] = T(z_q)[i,j] (overwrites, like the reference).  With
  * flags & QB_OUT_DEVICE, out is a device pointer; otherwise host memory.
  * rminmax (may be NULL) receives the padded table range [rmin, rmax].
- * Where tables of the given sizes would resolve H and J to about 1e-12 (the
- * estimate of qb_env_stands_in), on a plain geometry, the values come from
- * envelope tables instead (1e-14), also in qb_assemble_deriv and
- * qb_residuals; coarser tables are interpolated as the reference does. */
+ * On a plain geometry, a wavenumber at which tables of the given sizes would
+ * resolve H and J to about 1e-12 (the estimate of qb_env_stands_in; the sizes
+ * that qb_cheb_tune returns for tol <= 1e-12) takes its values from envelope
+ * tables instead (1e-14, and 2 to 4 times faster), also in qb_assemble_deriv
+ * and qb_residuals.  Coarser tables, those of the default tolerance 1e-10
+ * among them, are interpolated as the reference does.  Each wavenumber is
+ * judged by itself: a matrix does not depend on the others of the call, but
+ * for a last bit where its conjugate is among them. */
 int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const double* z,
                 int64_t nz, const qb_cheb_params* cheb, double* out,
                 int32_t flags, double* rminmax);

@@ -701,6 +701,24 @@ static int check_cheb(qb_ctx* ctx, const qb_cheb_params* c) {
   return QB_OK;
 }
 
+// f(a, n, envelope) for the runs [a, a + n) of wavenumbers that take one route: the
+// envelope tables where they may be taken (`may`) and stand in for tables of the sizes
+// cp, else the uniform ones.
+template <typename F>
+static int by_route(bool may, bool direct, const cd* z, int64_t nz, double rmin, double rmax,
+                    const qb_cheb_params& cp, F&& f) {
+  auto env = [&](int64_t q) { return may && qb_env_stands_in(direct, z[q], rmin, rmax, cp); };
+  for (int64_t a = 0; a < nz;) {
+    const bool e = env(a);
+    int64_t b = may ? a + 1 : nz;
+    while (b < nz && env(b) == e) ++b;
+    const int rc = f(a, b - a, e);
+    if (rc) return rc;
+    a = b;
+  }
+  return QB_OK;
+}
+
 extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const double* z, int64_t nz,
                            const qb_cheb_params* cheb, double* out, int32_t flags,
                            double* rminmax) {
@@ -734,9 +752,7 @@ extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const doub
   // its own (QB_ASM_TABLES=1: the uniform Hankel tables, as the windows then)
   const bool pairs = (flags & QB_ASM_CONJ_PAIRS) != 0;
   const bool env = pairs && getenv("QB_ASM_TABLES") == nullptr;
-  const bool fine = !pairs && g->sym.m == 0 &&
-                    qb_env_stands_in(op == QB_CFIE_KRESS, (const cd*)z, nz, rmin, rmax, *cheb);
-  if (!rc && !env && !fine)
+  if (!rc && pairs && !env)
     rc = qb_tables_build(ctx, (const double*)zd, nz, rmin, rmax, *cheb, true, &t);
   if (!rc) {
     if (on_dev)
@@ -752,10 +768,18 @@ extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const doub
         rc = qb_fail(ctx, QB_E_ARG,
                      "QB_ASM_CONJ_PAIRS needs nodes closed under conjugation and no symmetry "
                      "orbits (with QB_ASM_TABLES: tables with M_h = M_j in {5, 7})");
-    } else if (fine) {
-      rc = qb_assemble_env_list(ctx, g, op, (const cd*)z, nz, rmin, rmax, od);
     } else {
-      rc = qb_assemble_dev(ctx, g, op, zd, nz, t, od, nullptr);
+      rc = by_route(g->sym.m == 0, op == QB_CFIE_KRESS, (const cd*)z, nz, rmin, rmax, *cheb,
+                    [&](int64_t a, int64_t n, bool fine) {
+                      cd* o = od + a * N * N;
+                      if (fine)
+                        return qb_assemble_env_list(ctx, g, op, (const cd*)z + a, n, rmin, rmax, o);
+                      DevTables tn;
+                      int r = qb_tables_build(ctx, (const double*)(zd + a), n, rmin, rmax, *cheb, true, &tn);
+                      if (!r) r = qb_assemble_dev(ctx, g, op, zd + a, n, tn, o, nullptr);
+                      qb_tables_free(ctx, &tn);
+                      return r;
+                    });
     }
   }
   if (!rc && !on_dev) {
@@ -821,16 +845,22 @@ extern "C" int qb_assemble_noalloc(qb_ctx* ctx, const qb_geom* g, int32_t op,
           hipSuccess ||
       hipStreamSynchronize(ctx->stream) != hipSuccess)
     return qb_fail(ctx, QB_E_HIP, "wavenumber download failed");
-  rc = 1;
-  if (g->sym.m == 0 && qb_env_stands_in(op == QB_CFIE_KRESS, zh.data(), nz, rmin, rmax, *cheb))
-    rc = qb_assemble_env_list(ctx, g, op, zh.data(), nz, rmin, rmax, (cd*)out_dev, mem,
-                              (size_t)QB_NOALLOC_SCRATCH_BYTES);
-  if (rc == 1) {
-    DevTables t;
-    rc = qb_tables_build_in(ctx, z_dev, nz, rmin, rmax, *cheb, mem,
-                            (size_t)QB_NOALLOC_SCRATCH_BYTES, &t);
-    if (!rc) rc = qb_assemble_dev(ctx, g, op, (const cd*)z_dev, nz, t, (cd*)out_dev, nullptr);
-  }
+  const int64_t N = qb_dim(g);
+  rc = by_route(g->sym.m == 0, op == QB_CFIE_KRESS, zh.data(), nz, rmin, rmax, *cheb,
+                [&](int64_t a, int64_t n, bool fine) {
+                  cd* o = (cd*)out_dev + a * N * N;
+                  const size_t bytes = (size_t)QB_NOALLOC_SCRATCH_BYTES;
+                  int r = 1;
+                  if (fine)
+                    r = qb_assemble_env_list(ctx, g, op, zh.data() + a, n, rmin, rmax, o, mem, bytes);
+                  if (r == 1) {
+                    DevTables t;
+                    const double* za = z_dev + 2 * a;
+                    r = qb_tables_build_in(ctx, za, n, rmin, rmax, *cheb, mem, bytes, &t);
+                    if (!r) r = qb_assemble_dev(ctx, g, op, (const cd*)za, n, t, o, nullptr);
+                  }
+                  return r;
+                });
   // complete on return, as qb_assemble is
   const hipError_t e = hipStreamSynchronize(ctx->stream);
   if (!rc && e != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));
@@ -865,15 +895,10 @@ extern "C" int qb_assemble_deriv(qb_ctx* ctx, const qb_geom* g, int32_t op, cons
   cd* zd = nullptr;
   cd* od[3] = {nullptr, nullptr, nullptr};
   double* host[3] = {out, dout, ddout};
-  DevTables t;
   rc = qb_dev_alloc(ctx, (void**)&zd, nz * sizeof(cd));
   if (!rc && hipMemcpyAsync(zd, z, nz * sizeof(cd), hipMemcpyHostToDevice, ctx->stream) !=
                  hipSuccess)
     rc = qb_fail(ctx, QB_E_HIP, "upload failed");
-  const bool fine =
-      g->sym.m == 0 && qb_env_stands_in(true, (const cd*)z, nz, rmin, rmax, *cheb);
-  if (!rc && !fine)
-    rc = qb_tables_build(ctx, (const double*)zd, nz, rmin, rmax, *cheb, true, &t);
   for (int m = 0; m < 3 && !rc; ++m) {
     if (on_dev)
       od[m] = (cd*)host[m];
@@ -882,9 +907,19 @@ extern "C" int qb_assemble_deriv(qb_ctx* ctx, const qb_geom* g, int32_t op, cons
   }
   const bool ref_sign = (flags & QB_DERIV_MATRIX_SIGN) == 0;
   if (!rc)
-    rc = fine ? qb_assemble_deriv_env(ctx, g, op, (const cd*)z, nz, rmin, rmax, od[0], od[1], od[2],
-                                      ref_sign)
-              : qb_assemble_deriv_dev(ctx, g, op, zd, nz, t, od[0], od[1], od[2], ref_sign);
+    rc = by_route(g->sym.m == 0, true, (const cd*)z, nz, rmin, rmax, *cheb,
+                  [&](int64_t a, int64_t n, bool fine) {
+                    const int64_t o = a * N * N;
+                    cd *o0 = od[0] + o, *o1 = od[1] + o, *o2 = od[2] + o;
+                    if (fine)
+                      return qb_assemble_deriv_env(ctx, g, op, (const cd*)z + a, n, rmin, rmax, o0, o1,
+                                                   o2, ref_sign);
+                    DevTables t;
+                    int r = qb_tables_build(ctx, (const double*)(zd + a), n, rmin, rmax, *cheb, true, &t);
+                    if (!r) r = qb_assemble_deriv_dev(ctx, g, op, zd + a, n, t, o0, o1, o2, ref_sign);
+                    qb_tables_free(ctx, &t);
+                    return r;
+                  });
   for (int m = 0; m < 3 && !rc && !on_dev; ++m)
     if (hipMemcpyAsync(host[m], od[m], obytes, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
       rc = qb_fail(ctx, QB_E_HIP, "download failed");
@@ -892,7 +927,6 @@ extern "C" int qb_assemble_deriv(qb_ctx* ctx, const qb_geom* g, int32_t op, cons
     rc = qb_fail(ctx, QB_E_HIP, "assembly failed");
   if (!on_dev)
     for (int m = 0; m < 3; ++m) qb_dev_free(ctx, od[m], obytes);
-  qb_tables_free(ctx, &t);
   qb_dev_free(ctx, zd, nz * sizeof(cd));
   return rc;
 }
@@ -945,21 +979,23 @@ extern "C" int qb_residuals(qb_ctx* ctx, const qb_geom* g, int32_t op, const dou
       rc = qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));
       break;
     }
-    DevTables t;
     const cd* lz = (const cd*)lam + q0;
-    if (g->sym.m == 0 && qb_env_stands_in(op == QB_CFIE_KRESS, lz, nb, rmin, rmax, *cheb)) {
-      rc = qb_assemble_env_list(ctx, g, op, lz, nb, rmin, rmax, Td);
-    } else {
-      rc = qb_tables_build(ctx, (const double*)zd, nb, rmin, rmax, *cheb, true, &t);
-      if (!rc) rc = qb_assemble_dev(ctx, g, op, zd, nb, t, Td, nullptr);
-    }
+    rc = by_route(g->sym.m == 0, op == QB_CFIE_KRESS, lz, nb, rmin, rmax, *cheb,
+                  [&](int64_t a, int64_t n, bool fine) {
+                    cd* o = Td + a * N * N;
+                    if (fine) return qb_assemble_env_list(ctx, g, op, lz + a, n, rmin, rmax, o);
+                    DevTables t;
+                    int r = qb_tables_build(ctx, (const double*)(zd + a), n, rmin, rmax, *cheb, true, &t);
+                    if (!r) r = qb_assemble_dev(ctx, g, op, zd + a, n, t, o, nullptr);
+                    qb_tables_free(ctx, &t);
+                    return r;
+                  });
     if (!rc) rc = qb_gemv_norms(ctx, Td, phid, N, (int)nb, nsplit, work, nrm);
     if (!rc && hipMemcpyAsync(nrm_h.data(), nrm, 5 * nb * sizeof(double), hipMemcpyDeviceToHost,
                               ctx->stream) != hipSuccess)
       rc = qb_fail(ctx, QB_E_HIP, "norm download failed");
     e = hipStreamSynchronize(ctx->stream);
     if (!rc && e != hipSuccess) rc = qb_fail(ctx, QB_E_HIP, hipGetErrorString(e));
-    qb_tables_free(ctx, &t);
     if (rc) break;
     double* const res[5] = {res2, resn1, resninf, opn1, opninf};
     for (int64_t b = 0; b < nb; ++b)
@@ -1219,9 +1255,24 @@ static int win_create(qb_ctx* ctx, const qb_geom* g, int32_t op, int32_t nwin, c
       crc = qb_assemble_env_dev(ctx, g, op, w->zj.data(), w->z_dev, nz, rmin, rmax, w->T64, o32,
                                 ahead ? nb : 0,
                                 ahead ? std::function<int()>(first_panel) : std::function<int()>());
-    if (crc == 1 && !no_conj &&
-        qb_env_stands_in(op == QB_CFIE_KRESS, w->zj.data(), nz, rmin, rmax, *cheb))
-      crc = qb_assemble_red_env(ctx, g, op, w->zj.data(), nz, rmin, rmax, w->T64, o32);
+    // two to eight irreps: node by node, from envelope tables where they stand in
+    if (crc == 1 && !no_conj && g->sym.m > 0 && g->sym.pair && g->sym.nirr >= 2 && g->sym.nirr <= 8)
+      crc = by_route(true, op == QB_CFIE_KRESS, w->zj.data(), nz, rmin, rmax, *cheb,
+                     [&](int64_t a, int64_t n, bool fine) {
+                       cd* o = w->T64 + a * NN;
+                       cf* p = o32 ? o32 + a * NN : nullptr;
+                       int r = 1;
+                       if (fine)
+                         r = qb_assemble_red_env(ctx, g, op, w->zj.data() + a, n, nz, rmin, rmax, o, p);
+                       if (r == 1) {
+                         DevTables t;
+                         const cd* za = w->z_dev + a;
+                         r = qb_tables_build(ctx, (const double*)za, n, rmin, rmax, *cheb, true, &t);
+                         if (!r) r = qb_assemble_red_dev(ctx, g, op, za, n, t, o, p, nz);
+                         qb_tables_free(ctx, &t);
+                       }
+                       return r;
+                     });
     if (crc == 1) {
       QB_TRY(qb_tables_build(ctx, (const double*)w->z_dev, nz, rmin, rmax, *cheb, true, &tab));
       crc = no_conj ? 1 : qb_assemble_conj_dev(ctx, g, op, w->zj.data(), w->z_dev, nz, tab,

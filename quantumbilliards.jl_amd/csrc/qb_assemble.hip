@@ -881,23 +881,21 @@ static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z
   return QB_OK;
 }
 
-// Whether uniform tables of the sizes cp would give the Hankel and Bessel values
-// of these wavenumbers so exactly (tables tuned to an absolute error of 1e-12)
-// that the envelope tables may stand in for them: they are within 1e-14 of the
-// functions, built in 25 us and read from LDS.  Coarser tables are interpolated
-// as the caller asked.  The error of a panel of
-// half-width d is about its last coefficient (entering whole, as in the
-// reference): for the pole of H_1, at the first distance that the operator reads
-// from the table, 2 rho^-M / (s^2 - 1)^(1/2) with s the pole's distance in
-// half-widths, for e^{ikr} 2 (|k| d / 2)^M / M!.  Against the actual errors of
-// tables of 500 to 75000 panels the estimate is 1.5 to 10 times them, hence the
-// bound 1.2e-11.  Both routes, tables included: 16 DLP matrices of N = 4096 6.55
-// (uniform) and 1.45 ms, 24 CFIE ones of 1562 1.34 and 0.51 ms, 32 near-real ones
-// of 2050 6.15 and 2.05 ms, one of 128 98 and 38 us, six of 1500 with both
-// derivatives 0.74 and 0.37 ms: what bounds the uniform route is the L1 request
-// per lane and coefficient.
-bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double rmax,
-                      const qb_cheb_params& cp) {
+// Whether uniform tables of the sizes cp would give the Hankel and Bessel values at the
+// wavenumber z so exactly (tables tuned to an absolute error of 1e-12) that the envelope
+// tables may stand in for them: they are within 1e-14 of the functions, built in 25 us
+// and read from LDS.  Coarser tables are interpolated as the caller asked.  Each
+// wavenumber of a call is judged by itself, so a matrix does not change with the others.
+// The error of a panel of half-width d is about its last coefficient (entering whole,
+// as in the reference): for the pole of H_1, at the first distance that the operator
+// reads from the table, 2 rho^-M / (s^2 - 1)^(1/2) with s the pole's distance in
+// half-widths, for e^{ikr} 2 (|k| d / 2)^M / M!.  Against the actual errors of tables of
+// 500 to 75000 panels the estimate is 1.5 to 10 times them, hence the bound 1.2e-11.
+// Both routes, tables included: 16 DLP matrices of N = 4096 6.55 (uniform) and 1.45 ms,
+// 24 CFIE ones of 1562 1.34 and 0.51 ms, 32 near-real ones of 2050 6.15 and 2.05 ms, one
+// of 128 98 and 38 us, six of 1500 with both derivatives 0.74 and 0.37 ms: what bounds
+// the uniform route is the L1 request per lane and coefficient.
+bool qb_env_stands_in(bool direct, cd z, double rmin, double rmax, const qb_cheb_params& cp) {
   int o0, P;
   if (getenv("QB_ASM_TABLES") || !env_range(rmin, rmax, &o0, &P)) return false;
   const double dh = (rmax - rmin) / (2.0 * cp.n_panels_h), dj = rmax / (2.0 * cp.n_panels_j);
@@ -906,21 +904,18 @@ bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double 
     for (int n = 1; n <= M; ++n) v *= q / n;
     return q < 0.5 * (M + 1) ? v / (1.0 - q / (M + 1)) : INFINITY;
   };
-  for (int64_t i = 0; i < nz; ++i) {
-    const double ak = hypot(z[i].re, z[i].im);
-    if (!(z[i].re > 0.0) || !(fabs(z[i].im) * rmax < 50.0) || !(ak < 1e12)) return false;
-    const double grow = exp(fabs(z[i].im) * rmax);
-    const double r1 = direct && 0.2 / ak > rmin ? 0.2 / ak : rmin;  // first distance read
-    const double c = fmax(rmin + dh, r1 - dh), s = c / dh;
-    if (!(s > 1.0)) return false;
-    const double w = sqrt(s * s - 1.0), rho = s + w;
-    const double pole = 2.0 * s / w * pow(rho, -cp.M_h) * rho / (rho - 1.0);
-    const double amp = 2.0 / (QB_PI * ak * c) + sqrt(2.0 / (QB_PI * ak * c));
-    const double eh = grow * amp * (pole + osc(0.5 * ak * dh, cp.M_h));
-    const double ej = grow * osc(0.5 * ak * dj, cp.M_j);
-    if (!(eh < 1.2e-11) || !(ej < 1.2e-11)) return false;
-  }
-  return true;
+  const double ak = hypot(z.re, z.im);
+  if (!(z.re > 0.0) || !(fabs(z.im) * rmax < 50.0) || !(ak < 1e12)) return false;
+  const double grow = exp(fabs(z.im) * rmax);
+  const double r1 = direct && 0.2 / ak > rmin ? 0.2 / ak : rmin;  // first distance read
+  const double c = fmax(rmin + dh, r1 - dh), s = c / dh;
+  if (!(s > 1.0)) return false;
+  const double w = sqrt(s * s - 1.0), rho = s + w;
+  const double pole = 2.0 * s / w * pow(rho, -cp.M_h) * rho / (rho - 1.0);
+  const double amp = 2.0 / (QB_PI * ak * c) + sqrt(2.0 / (QB_PI * ak * c));
+  const double eh = grow * amp * (pole + osc(0.5 * ak * dh, cp.M_h));
+  const double ej = grow * osc(0.5 * ak * dj, cp.M_j);
+  return eh < 1.2e-11 && ej < 1.2e-11;
 }
 
 static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd* zd) {
@@ -930,11 +925,12 @@ static int env_upload_z(qb_ctx* ctx, const std::vector<cd>& zs, cd* zd) {
   return QB_OK;
 }
 
-// Matrices of any wavenumbers (Re z > 0) of a plain geometry from envelope
-// tables.  A wavenumber whose conjugate is in the list to rounding (equal real
-// parts, imaginary parts within u |k| of opposite: less than the rounding of k r
-// moves the argument at every r) is assembled with it; for the others the conjugate's table is built beside their own
-// (J_n = (H_n(k r) + conj H_n(conj(k) r)) / 2) and only their matrix is written.
+// Matrices of any wavenumbers (Re z > 0) of a plain geometry from envelope tables.  A
+// wavenumber whose conjugate is in the list to rounding (equal real parts, imaginary
+// parts within u |k| of opposite: less than the rounding of k r moves the argument at
+// every r) is assembled with it, which may change its last bit; for the others the
+// conjugate's table is built beside their own (J_n = (H_n(k r) + conj H_n(conj(k) r)) / 2)
+// and only their matrix is written.
 // mem: mem_bytes of device memory to work in, or null; 1 when too few.
 int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
                          double rmin, double rmax, cd* out64, void* mem, size_t mem_bytes) {
@@ -1923,9 +1919,10 @@ struct RedPairMulti {
 };
 
 // Reduced matrices of 2 to 8 irreps with pair sharing, from envelope tables;
-// other geometries return 1.
+// other geometries return 1.  nz_out: wavenumbers of the whole output (irrep e's
+// matrices start at e * nz_out).
 int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
-                        double rmin, double rmax, cd* out64, cf* out32) {
+                        int64_t nz_out, double rmin, double rmax, cd* out64, cf* out32) {
   const int64_t m = g->sym.m;
   const int nirr = g->sym.nirr;
   if (m <= 0 || !g->sym.pair || nirr < 2 || nirr > 8 || nz > 1024) return 1;
@@ -1945,7 +1942,7 @@ int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds);
     hipLaunchKernelGGL(kern, dim3(Tm * (Tm + 1) / 2, 1, (unsigned)nz), dim3(256), lds, ctx->stream,
-                       g->d, g->sym, e.z, tb, (int64_t)0, nz, (int)Tm, out64, out32);
+                       g->d, g->sym, e.z, tb, (int64_t)0, nz_out, (int)Tm, out64, out32);
   };
   if (op == QB_CFIE_KRESS)
     launch(RedPairMulti<QB_CFIE_KRESS>());
@@ -1960,24 +1957,25 @@ int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
 }
 
 int qb_assemble_red_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
-                        const DevTables& t, cd* out64, cf* out32) {
+                        const DevTables& t, cd* out64, cf* out32, int64_t nz_out) {
+  if (nz_out == 0) nz_out = nz;
   for (int64_t q0 = 0; q0 < nz; q0 += 1024) {
     const int64_t nzc = nz - q0 < 1024 ? nz - q0 : 1024;
     const int mh = t.M_h, mj = t.M_j;
     if (op == QB_CFIE_KRESS) {
       if (mh == 7 && mj == 7)
-        launch_red<QB_CFIE_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, nz, t, out64, out32);
+        launch_red<QB_CFIE_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, nz_out, t, out64, out32);
       else if (mh == 5 && mj == 5)
-        launch_red<QB_CFIE_KRESS, 5, 5>(ctx, g, z_dev, q0, nzc, nz, t, out64, out32);
+        launch_red<QB_CFIE_KRESS, 5, 5>(ctx, g, z_dev, q0, nzc, nz_out, t, out64, out32);
       else
-        launch_red<QB_CFIE_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, nz, t, out64, out32);
+        launch_red<QB_CFIE_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, nz_out, t, out64, out32);
     } else {
       if (mh == 7 && mj == 7)
-        launch_red<QB_DLP_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, nz, t, out64, out32);
+        launch_red<QB_DLP_KRESS, 7, 7>(ctx, g, z_dev, q0, nzc, nz_out, t, out64, out32);
       else if (mh == 5 && mj == 5)
-        launch_red<QB_DLP_KRESS, 5, 5>(ctx, g, z_dev, q0, nzc, nz, t, out64, out32);
+        launch_red<QB_DLP_KRESS, 5, 5>(ctx, g, z_dev, q0, nzc, nz_out, t, out64, out32);
       else
-        launch_red<QB_DLP_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, nz, t, out64, out32);
+        launch_red<QB_DLP_KRESS, 0, 0>(ctx, g, z_dev, q0, nzc, nz_out, t, out64, out32);
     }
     QB_HIP(ctx, hipGetLastError());
   }

@@ -214,20 +214,19 @@ int qb_assemble_env_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host,
                         const std::function<int()>& between = std::function<int()>());
 // Envelope tables in the place of uniform ones of the sizes cp (direct: the
 // operator evaluates below |k r| = 0.2 directly), and the assemblies from them.
-bool qb_env_stands_in(bool direct, const cd* z, int64_t nz, double rmin, double rmax,
-                      const qb_cheb_params& cp);
+bool qb_env_stands_in(bool direct, cd z, double rmin, double rmax, const qb_cheb_params& cp);
 int qb_assemble_env_list(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
                          double rmin, double rmax, cd* out64, void* mem = nullptr,
                          size_t mem_bytes = 0);
 int qb_assemble_deriv_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
                           double rmin, double rmax, cd* out, cd* dout, cd* ddout, bool ref_sign);
 int qb_assemble_red_env(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_host, int64_t nz,
-                        double rmin, double rmax, cd* out64, cf* out32);
+                        int64_t nz_out, double rmin, double rmax, cd* out64, cf* out32);
 // Pairs (a, b) of wavenumbers with z_b = conj(z_a) (a real one with itself),
 // flattened; false when some wavenumber has no partner.
 bool qb_conj_pairs(const cd* z_host, int64_t nz, std::vector<int>* pr);
 int qb_assemble_red_dev(qb_ctx* ctx, const qb_geom* g, int op, const cd* z_dev, int64_t nz,
-                        const DevTables& t, cd* out64, cf* out32);
+                        const DevTables& t, cd* out64, cf* out32, int64_t nz_out = 0);
 // Checks |x_{rep_a} - x_{img[b,l]}| = |x_{rep_b} - x_{img[a,inv[l]]}| to
 // 1e-13 r + floor_abs for every (a, b, l) on the device; ok = 1 if it holds.
 int qb_orbit_pairs_ok(qb_ctx* ctx, const DevGeom& g, const DevSym& s, double floor_abs, int* ok);

@@ -256,7 +256,10 @@ def chebyshev_params(solver, pts, zj, *, npanels_h_init=15000, M_h_init=5, npane
                      M_j_init=5, tol=1e-10, sampling_points=50000, max_iter=20,
                      geom: Optional[Geometry] = None, ctx: Optional[Context] = None):
     """chebyshev_params (chebyshev_optimal_panelization.jl:221-262) on the
-    device: returns (nh, Mh, nj, Mj, errs[4])."""
+    device: returns (nh, Mh, nj, Mj, errs[4]).  Sizes found for tol <= 1e-12 let the
+    assemblies of plain geometries take envelope tables in their place, which are
+    exact to 1e-14 and 2 to 4 times faster; those of the default tolerance are
+    interpolated."""
     ctx = ctx or (geom.ctx if geom is not None else default_context())
     g = geom or Geometry(pts, ctx)
     zj = np.ascontiguousarray(np.asarray(zj, dtype=np.complex128).ravel())
