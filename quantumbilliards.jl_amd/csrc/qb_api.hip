@@ -52,8 +52,9 @@ int qb_dev_alloc(qb_ctx* ctx, void** p, size_t bytes) {
     }
   }
   hipError_t e = hipMallocAsync(p, bytes, ctx->stream);
-  if (e != hipSuccess && !ctx->cache.empty()) {
+  if (e != hipSuccess && (!ctx->cache.empty() || (ctx->block && !ctx->block_used))) {
     (void)hipGetLastError();
+    qb_block_release(ctx);
     cache_release(ctx);
     // the released blocks return to the pool once this stream reaches them
     (void)hipStreamSynchronize(ctx->stream);
@@ -83,6 +84,34 @@ void qb_dev_free(qb_ctx* ctx, void* p, size_t bytes) {
   (void)hipFreeAsync(p, ctx->stream);
   ctx->bytes -= (int64_t)bytes;
 }
+
+// Allocations of some gigabytes take up to seconds while the driver clears memory that
+// was freed (measured in a serving stream without a cache: 58 of them 0 to 5 s in all,
+// 27 more for the residues 3 to 7 s more), so that the residues of a window's LU and its
+// moment solutions share one.
+void qb_block_release(qb_ctx* ctx) {
+  if (!ctx->block || ctx->block_used) return;
+  void* p = ctx->block;
+  ctx->block = nullptr;
+  qb_dev_free(ctx, p, ctx->block_bytes);
+  ctx->block_bytes = 0;
+}
+
+void qb_block_reserve(qb_ctx* ctx, size_t bytes) {
+  if (ctx->block_used || ctx->block_bytes >= bytes) return;
+  qb_block_release(ctx);
+  const std::string err = ctx->err;
+  if (qb_dev_alloc(ctx, &ctx->block, bytes) == QB_OK) ctx->block_bytes = bytes;
+  ctx->err = err;  // no room: the callers do without
+}
+
+void* qb_block_take(qb_ctx* ctx, size_t bytes) {
+  if (!ctx->block || ctx->block_used || ctx->block_bytes < bytes) return nullptr;
+  ctx->block_used = true;
+  return ctx->block;
+}
+
+void qb_block_put(qb_ctx* ctx) { ctx->block_used = false; }
 
 // ---------------------------------------------------------------------------
 // launch accounting
@@ -201,6 +230,7 @@ void qb_ctx_destroy(qb_ctx* ctx) {
   }
   (void)hipStreamSynchronize(ctx->stream);
   qb_graphs_clear(ctx);
+  qb_block_release(ctx);
   cache_release(ctx);
   (void)hipStreamSynchronize(ctx->stream);
   if (ctx->ev_main) (void)hipEventDestroy(ctx->ev_main);
@@ -1085,9 +1115,11 @@ static size_t win_bytes_moments(int64_t N, int nq, int precision, int r) {
 }
 
 extern "C" int64_t qb_window_residue_extra(int64_t N, int32_t nq, int32_t precision, int32_t r) {
-  // the LU has given its residue buffers back when the moments begin
+  // the moment solutions take the residues' place; V, the moments and the QR block stand
+  // beside them
   if (precision != QB_FP64) return 0;
-  const int64_t e = qb_getrf_rns_bytes(N, nq) - (int64_t)win_bytes_moments(N, nq, precision, r);
+  const int64_t b = qb_getrf_rns_bytes(N, nq), rest = 5 * (int64_t)sizeof(cd) * N * r;
+  const int64_t e = b ? b + rest - (int64_t)win_bytes_moments(N, nq, precision, r) : 0;
   return e > 0 ? e : 0;
 }
 
@@ -1101,6 +1133,7 @@ extern "C" int64_t qb_window_footprint(int64_t N, int32_t nq, int32_t precision,
 
 static void win_free(qb_window* w) {
   qb_ctx* ctx = w->ctx;
+  qb_block_release(ctx);
   size_t NN = (size_t)w->N * w->N;
   qb_dev_free(ctx, w->z_dev, (size_t)w->nwin * w->nc * sizeof(cd));
   qb_dev_free(ctx, w->w_dev, 2 * (size_t)w->nwin * w->nc * sizeof(cd));
@@ -1219,6 +1252,8 @@ static int win_create(qb_ctx* ctx, const qb_geom* g, int32_t op, int32_t nwin, c
   QB_TRY(qb_dev_alloc(ctx, (void**)&w->perm, (size_t)nq * N * sizeof(int)));
   QB_TRY(qb_dev_alloc(ctx, (void**)&w->info, nq * sizeof(int)));
   QB_TRY(qb_dev_alloc(ctx, (void**)&w->scratch_d, 3 * nq * sizeof(double)));
+  if (precision == QB_FP64 && ctx->residues && !ctx->graphs && qb_getrf_rns_bytes(N, nq) > 0)
+    qb_block_reserve(ctx, (size_t)qb_getrf_rns_bytes(N, nq));
   if (hipMemcpyAsync(w->z_dev, w->zj.data(), nz * sizeof(cd), hipMemcpyHostToDevice,
                      ctx->stream) != hipSuccess ||
       hipMemcpyAsync(w->w_dev, wbuf.data(), 2 * nz * sizeof(cd), hipMemcpyHostToDevice,
@@ -1448,8 +1483,15 @@ static int win_moments(qb_window* w, int32_t r, const double* V, double* A0, dou
   int iters_max = 0;
   double resid_max = 0.0;
   std::vector<double> h3(3 * nq);
+  const size_t xbytes = (size_t)nq * nv * sizeof(cd);
+  bool x_block = false;
   QB_TRY(qb_dev_alloc(ctx, (void**)&Vd, nv * sizeof(cd)));
-  QB_TRY(qb_dev_alloc(ctx, (void**)&X, (size_t)nq * nv * sizeof(cd)));
+  X = (cd*)qb_block_take(ctx, xbytes);
+  x_block = X != nullptr;
+  if (!X) {
+    qb_block_release(ctx);
+    QB_TRY(qb_dev_alloc(ctx, (void**)&X, xbytes));
+  }
   // moments per block b: device output [A0_b | A1_b] blocks (2 nv each); host
   // outputs A0 and A1 hold the nblk blocks one after the other
   if (!dev_out) {
@@ -1651,7 +1693,10 @@ fail:
   (void)hipStreamSynchronize(ctx->stream_aux);
   qb_dev_free(ctx, actd, nq * sizeof(int));
   qb_dev_free(ctx, Vd, nv * sizeof(cd));
-  qb_dev_free(ctx, X, (size_t)nq * nv * sizeof(cd));
+  if (x_block)
+    qb_block_put(ctx);
+  else
+    qb_dev_free(ctx, X, xbytes);
   qb_dev_free(ctx, Rr, (size_t)nq * nv * sizeof(cd));
   qb_dev_free(ctx, D32, (size_t)nq * nv * sizeof(cf));
   qb_dev_free(ctx, ozB, oz_bc / 2);

@@ -88,6 +88,12 @@ struct qb_ctx {
   // autotuner changes a tile pick, so stale captures are not replayed.
   bool graphs = false;
   bool residues = true;  // LUs may take residue buffers (qb_ctx_set_residue_buffers)
+  // A window's block for the residues of its LU and then, where it is large enough, for
+  // its moment solutions: one per context, from qb_window_create until a window of the
+  // context is destroyed or an allocation needs the room (qb_block_reserve).
+  void* block = nullptr;
+  size_t block_bytes = 0;
+  bool block_used = false;
   uint64_t gemm_epoch = 0;
   struct GraphRec {
     int ty;
@@ -167,6 +173,12 @@ int qb_fail(qb_ctx* ctx, int code, const std::string& msg);
 
 int qb_dev_alloc(qb_ctx* ctx, void** p, size_t bytes);
 void qb_dev_free(qb_ctx* ctx, void* p, size_t bytes);
+// ctx->block of at least `bytes`, unless it is in use or there is no room.
+void qb_block_reserve(qb_ctx* ctx, size_t bytes);
+void qb_block_release(qb_ctx* ctx);  // not while it is in use
+// The block for the caller until qb_block_put, or null when it is too small or in use.
+void* qb_block_take(qb_ctx* ctx, size_t bytes);
+void qb_block_put(qb_ctx* ctx);
 
 // tables (qb_tables.hip) ----------------------------------------------------
 int qb_tables_build(qb_ctx* ctx, const double* z_dev_or_host, int64_t nz,

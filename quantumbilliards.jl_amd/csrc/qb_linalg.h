@@ -51,7 +51,8 @@ int qb_trsm_lu_batched(qb_ctx* ctx, const T* LU, int n, int64_t lda, int64_t sA,
 
 // complex128 C[b] -= A[b] B[b] on the int8 matrix cores (qb_rns.hip) for inner
 // dimension 512.  qb_rns_open takes the residue buffers for up to M x 512 and 512 x N
-// operands of `batch` matrices (QB_E_NOMEM: no room, nothing changed);
+// operands of `batch` matrices, ctx->block or memory of its own (QB_E_NOMEM: no room,
+// nothing changed);
 // qb_rns_set_a slices the A operands (of ctx->bix's matrices when set), after
 // which qb_rns_sub subtracts their products with any number of B's.  All on
 // ctx->stream.
@@ -60,6 +61,7 @@ struct QbRns {
   double *scA = nullptr, *scB = nullptr;
   int64_t strideA = 0, strideB = 0, maxM = 0, maxN = 0;
   size_t bytes = 0;
+  bool own = false;  // mem is the handle's, not the context's block
   int batch = 0, nb = 0, M = 0;
 };
 int64_t qb_rns_bytes(int64_t M, int64_t N, int batch);

@@ -501,12 +501,16 @@ int qb_rns_open(qb_ctx* ctx, QbRns* h, int64_t M, int64_t N, int batch) {
   h->strideB = rns_plane_bytes(rns_blocks(N, 2));
   h->nb = rns_b_nodes(h->strideB, batch);
   h->bytes = (size_t)qb_rns_bytes(M, N, batch);
-  const std::string err = ctx->err;
-  const int rc = qb_dev_alloc(ctx, (void**)&h->mem, h->bytes);
-  if (rc) {  // no room: the caller takes its FP64 kernels
-    ctx->err = err;
-    h->mem = nullptr;
-    return rc;
+  h->mem = (signed char*)qb_block_take(ctx, h->bytes);
+  h->own = h->mem == nullptr;
+  if (h->own) {
+    const std::string err = ctx->err;
+    const int rc = qb_dev_alloc(ctx, (void**)&h->mem, h->bytes);
+    if (rc) {  // no room: the caller takes its FP64 kernels
+      ctx->err = err;
+      h->mem = nullptr;
+      return rc;
+    }
   }
   h->A = h->mem;
   h->B = h->A + batch * h->strideA;
@@ -517,7 +521,10 @@ int qb_rns_open(qb_ctx* ctx, QbRns* h, int64_t M, int64_t N, int batch) {
 
 void qb_rns_close(qb_ctx* ctx, QbRns* h) {
   if (!h->mem) return;
-  qb_dev_free(ctx, h->mem, h->bytes);
+  if (h->own)
+    qb_dev_free(ctx, h->mem, h->bytes);
+  else
+    qb_block_put(ctx);
   h->mem = nullptr;
 }
 
