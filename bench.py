@@ -35,9 +35,8 @@ import numpy as np  # noqa: E402
 PEAK = {"c64": 157.3, "c128": 78.6, "i8": 5000.0}  # dense MFMA TFLOP/s (fp32, fp64), int8 TOPS
 # HBM bytes per GEMM launch over the windows of the default workload, from
 # FETCH_SIZE / WRITE_SIZE counter runs scaled by a copy kernel of known size
-# (profiles/beyn_window_star_N8192_pmc_traffic.txt; its c128 figure is of the
-# launches before the LU's trailing updates left for the int8 matrix cores)
-TRAFFIC_PER_LAUNCH = {"c64": 467.3e6}
+# (profiles/beyn_window_star_N8192_pmc_traffic.txt)
+TRAFFIC_PER_LAUNCH = {"c128": 560.6e6, "c64": 515.8e6}
 
 
 def parse():

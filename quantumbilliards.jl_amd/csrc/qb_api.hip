@@ -749,6 +749,16 @@ static int by_route(bool may, bool direct, const cd* z, int64_t nz, double rmin,
   return QB_OK;
 }
 
+// Matrices of n wavenumbers (device) from uniform tables of the sizes cp.
+static int assemble_tables(qb_ctx* ctx, const qb_geom* g, int op, const cd* zd, int64_t n,
+                           double rmin, double rmax, const qb_cheb_params& cp, cd* out) {
+  DevTables t;
+  int rc = qb_tables_build(ctx, (const double*)zd, n, rmin, rmax, cp, true, &t);
+  if (!rc) rc = qb_assemble_dev(ctx, g, op, zd, n, t, out, nullptr);
+  qb_tables_free(ctx, &t);
+  return rc;
+}
+
 extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const double* z, int64_t nz,
                            const qb_cheb_params* cheb, double* out, int32_t flags,
                            double* rminmax) {
@@ -802,13 +812,9 @@ extern "C" int qb_assemble(qb_ctx* ctx, const qb_geom* g, int32_t op, const doub
       rc = by_route(g->sym.m == 0, op == QB_CFIE_KRESS, (const cd*)z, nz, rmin, rmax, *cheb,
                     [&](int64_t a, int64_t n, bool fine) {
                       cd* o = od + a * N * N;
-                      if (fine)
-                        return qb_assemble_env_list(ctx, g, op, (const cd*)z + a, n, rmin, rmax, o);
-                      DevTables tn;
-                      int r = qb_tables_build(ctx, (const double*)(zd + a), n, rmin, rmax, *cheb, true, &tn);
-                      if (!r) r = qb_assemble_dev(ctx, g, op, zd + a, n, tn, o, nullptr);
-                      qb_tables_free(ctx, &tn);
-                      return r;
+                      return fine ? qb_assemble_env_list(ctx, g, op, (const cd*)z + a, n, rmin,
+                                                         rmax, o)
+                                  : assemble_tables(ctx, g, op, zd + a, n, rmin, rmax, *cheb, o);
                     });
     }
   }
@@ -882,7 +888,8 @@ extern "C" int qb_assemble_noalloc(qb_ctx* ctx, const qb_geom* g, int32_t op,
                   const size_t bytes = (size_t)QB_NOALLOC_SCRATCH_BYTES;
                   int r = 1;
                   if (fine)
-                    r = qb_assemble_env_list(ctx, g, op, zh.data() + a, n, rmin, rmax, o, mem, bytes);
+                    r = qb_assemble_env_list(ctx, g, op, zh.data() + a, n, rmin, rmax, o, mem,
+                                             bytes);
                   if (r == 1) {
                     DevTables t;
                     const double* za = z_dev + 2 * a;
@@ -942,11 +949,12 @@ extern "C" int qb_assemble_deriv(qb_ctx* ctx, const qb_geom* g, int32_t op, cons
                     const int64_t o = a * N * N;
                     cd *o0 = od[0] + o, *o1 = od[1] + o, *o2 = od[2] + o;
                     if (fine)
-                      return qb_assemble_deriv_env(ctx, g, op, (const cd*)z + a, n, rmin, rmax, o0, o1,
-                                                   o2, ref_sign);
+                      return qb_assemble_deriv_env(ctx, g, op, (const cd*)z + a, n, rmin, rmax, o0,
+                                                   o1, o2, ref_sign);
                     DevTables t;
-                    int r = qb_tables_build(ctx, (const double*)(zd + a), n, rmin, rmax, *cheb, true, &t);
-                    if (!r) r = qb_assemble_deriv_dev(ctx, g, op, zd + a, n, t, o0, o1, o2, ref_sign);
+                    const cd* za = zd + a;
+                    int r = qb_tables_build(ctx, (const double*)za, n, rmin, rmax, *cheb, true, &t);
+                    if (!r) r = qb_assemble_deriv_dev(ctx, g, op, za, n, t, o0, o1, o2, ref_sign);
                     qb_tables_free(ctx, &t);
                     return r;
                   });
@@ -1013,12 +1021,8 @@ extern "C" int qb_residuals(qb_ctx* ctx, const qb_geom* g, int32_t op, const dou
     rc = by_route(g->sym.m == 0, op == QB_CFIE_KRESS, lz, nb, rmin, rmax, *cheb,
                   [&](int64_t a, int64_t n, bool fine) {
                     cd* o = Td + a * N * N;
-                    if (fine) return qb_assemble_env_list(ctx, g, op, lz + a, n, rmin, rmax, o);
-                    DevTables t;
-                    int r = qb_tables_build(ctx, (const double*)(zd + a), n, rmin, rmax, *cheb, true, &t);
-                    if (!r) r = qb_assemble_dev(ctx, g, op, zd + a, n, t, o, nullptr);
-                    qb_tables_free(ctx, &t);
-                    return r;
+                    return fine ? qb_assemble_env_list(ctx, g, op, lz + a, n, rmin, rmax, o)
+                                : assemble_tables(ctx, g, op, zd + a, n, rmin, rmax, *cheb, o);
                   });
     if (!rc) rc = qb_gemv_norms(ctx, Td, phid, N, (int)nb, nsplit, work, nrm);
     if (!rc && hipMemcpyAsync(nrm_h.data(), nrm, 5 * nb * sizeof(double), hipMemcpyDeviceToHost,
@@ -1296,13 +1300,13 @@ static int win_create(qb_ctx* ctx, const qb_geom* g, int32_t op, int32_t nwin, c
                      [&](int64_t a, int64_t n, bool fine) {
                        cd* o = w->T64 + a * NN;
                        cf* p = o32 ? o32 + a * NN : nullptr;
+                       const cd *zh = w->zj.data() + a, *za = w->z_dev + a;
                        int r = 1;
-                       if (fine)
-                         r = qb_assemble_red_env(ctx, g, op, w->zj.data() + a, n, nz, rmin, rmax, o, p);
+                       if (fine) r = qb_assemble_red_env(ctx, g, op, zh, n, nz, rmin, rmax, o, p);
                        if (r == 1) {
                          DevTables t;
-                         const cd* za = w->z_dev + a;
-                         r = qb_tables_build(ctx, (const double*)za, n, rmin, rmax, *cheb, true, &t);
+                         r = qb_tables_build(ctx, (const double*)za, n, rmin, rmax, *cheb, true,
+                                             &t);
                          if (!r) r = qb_assemble_red_dev(ctx, g, op, za, n, t, o, p, nz);
                          qb_tables_free(ctx, &t);
                        }

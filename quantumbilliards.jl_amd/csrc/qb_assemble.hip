@@ -840,8 +840,8 @@ static int assemble_env_pairs(qb_ctx* ctx, const qb_geom* g, int op, const cd* z
                                 (int)lds);
       hipLaunchKernelGGL(kern, dim3((unsigned)npairs, env_split(npairs * npair, occ3 ? 16 : 4),
                                     (unsigned)npair),
-                         dim3(256), lds, ctx->stream, g->d, z_dev, env, o0, P, pd, (int)nout, T, J0, first, out64,
-                         out32);
+                         dim3(256), lds, ctx->stream, g->d, z_dev, env, o0, P, pd, (int)nout, T, J0,
+                         first, out64, out32);
     };
     auto launch_all = [&](int64_t npairs, int first) {
       if (op == QB_CFIE_KRESS) {
@@ -1226,11 +1226,9 @@ __device__ __forceinline__ D3 diag_deriv(const DevGeom& g, int64_t j, cd k) {
 // = 50 KB; 8 beside envelope tables, so that two workgroups fit in a CU) and
 // written CW contiguous rows per column.
 template <int OP, int MH, int MJ>
-__global__ void __launch_bounds__(256, MH < 0 ? 2 : 1) k_assemble_deriv(DevGeom g, const cd* __restrict__ zk,
-                                                        AsmTabs tb, int64_t q0,
-                                                        int T, cd* __restrict__ o0,
-                                                        cd* __restrict__ o1,
-                                                        cd* __restrict__ o2, double off_sign) {
+__global__ void __launch_bounds__(256, MH < 0 ? 2 : 1)
+k_assemble_deriv(DevGeom g, const cd* __restrict__ zk, AsmTabs tb, int64_t q0, int T,
+                 cd* __restrict__ o0, cd* __restrict__ o1, cd* __restrict__ o2, double off_sign) {
   constexpr int CW = MH < 0 ? 8 : 16;
   __shared__ cd mir[3][CW][65];  // mir[out][j_local - CW ch][i_local] = A[j, i]
   extern __shared__ __align__(16) cd smem[];

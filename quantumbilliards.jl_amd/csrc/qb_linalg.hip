@@ -984,7 +984,9 @@ const char* qb_gemm_variant_name(int ty, int v) {
   return (ty >= 0 && ty < 2 && v >= 0 && v < QB_GEMM_VARIANTS) ? kGemmNames[ty][v] : "?";
 }
 
-__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 // Explicit fused operations: every kernel that forms these rounds alike.
 template <typename T>
@@ -1054,7 +1056,8 @@ __device__ __forceinline__ double dpp_max(double x) {
 template <int CTRL, int ROWS>
 __device__ __forceinline__ float dpp_max(float x) {
   const int i = __float_as_int(x);
-  return __builtin_fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false)));
+  const int o = __builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false);
+  return __builtin_fmaxf(x, __int_as_float(o));
 }
 __device__ __forceinline__ double lane_value(double x, int l) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
@@ -1791,10 +1794,11 @@ static bool panel_lean_beside(const qb_ctx* ctx, int M, int N, int K) {
 // The complex128 trailing updates that run on the int8 matrix cores (qb_rns.hip):
 // steps of the full panel width of 512 with at least kRnsMin rows left.  An
 // update takes 33 to 36 ps per entry there against 48.8 ps, and its slices 12.5
-// ps for each of 512 (M + N) elements: at 1024 rows the two meet.  Matrices
-// below 4096 rows have panels of 256 columns, where the residues gain nothing,
-// and panels of 512 cost them what the updates would win (1141 rows: 12.8 ms for
-// a window of 32 matrices against 12.4, 1792 rows: 24.6 against 24.1).
+// ps for each of 512 (M + N) elements: at 1024 rows the two meet.  They come with
+// the panels of 512 columns (qb_lu_nb), whose line lies at 4096 rows.  Windows of 32
+// matrices with panels of 512 and residues against panels of 256: 1536, 1792 and 2100
+// rows 3 % slower, 2600, 3100, 3600 and 4095 rows 2, 4, 6 and 10 % faster, 4096 10 %: a
+// line of its own at about 2400 rows would be the better one for complex128.
 static const int kRnsMin = 1024;
 static bool lu_rns(int n) { return qb_lu_nb(n) == 512 && n - 512 >= kRnsMin; }
 

@@ -18,7 +18,8 @@
 
 // zlarfg of x = A[:, j], rows j..N-1, by the NT threads of a workgroup.
 template <int NT>
-__device__ __forceinline__ void reflector(cd* __restrict__ x, int64_t N, int j, cd* __restrict__ tau) {
+__device__ __forceinline__ void reflector(cd* __restrict__ x, int64_t N, int j,
+                                          cd* __restrict__ tau) {
   __shared__ double red[NT / 64];
   __shared__ cd s_scale;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -147,8 +148,10 @@ __global__ void k_qr_form_v(const cd* __restrict__ A, int64_t N, int j0, int jb,
 // What bounds it: the 32 columns one after the other (24 us; with loads column by
 // column and one chain of sums 43).
 template <bool ADJ>
-__global__ void __launch_bounds__(256) k_qr_form_t(const cd* __restrict__ G, const cd* __restrict__ tau, int j0, int jb,
-                            cd* __restrict__ Th, int64_t gstride, int64_t tstride) {
+__global__ void __launch_bounds__(256) k_qr_form_t(const cd* __restrict__ G,
+                                                   const cd* __restrict__ tau, int j0, int jb,
+                                                   cd* __restrict__ Th, int64_t gstride,
+                                                   int64_t tstride) {
   __shared__ cd T[QB_QR_NB][QB_QR_NB + 1], Gs[QB_QR_NB][QB_QR_NB + 1];
   __shared__ cd ts[QB_QR_NB];
   G += (int64_t)blockIdx.x * gstride;

@@ -130,7 +130,8 @@ __device__ __forceinline__ int mod_byte(float t, float m, float inv) {
 }
 // low bytes of four words
 __device__ __forceinline__ int pack4(int a, int b, int c, int d) {
-  const int lo = __builtin_amdgcn_perm(b, a, 0x0c0c0400), hi = __builtin_amdgcn_perm(d, c, 0x04000c0c);
+  const int lo = __builtin_amdgcn_perm(b, a, 0x0c0c0400);
+  const int hi = __builtin_amdgcn_perm(d, c, 0x04000c0c);
   return lo | hi;
 }
 
@@ -141,9 +142,9 @@ __device__ __forceinline__ int pack4(int a, int b, int c, int d) {
 // 16 bytes per plane: the 1 KB of a (plane, k / 32) is what a wave's MFMA
 // 32x32x32 operand takes, lane by lane.  The planes of 32 rows stand together,
 // [i / 32][plane][k / 32], so that a tile of the product reads a few megabytes
-// in one piece (plane by plane over all rows, every plane is another page).  scale[i] = 2^(e-1) with
-// e the exponent of the largest component (NaN when the row holds an infinity
-// or NaN, which makes every result of the row NaN).
+// in one piece (plane by plane over all rows, every plane is another page).
+// scale[i] = 2^(e-1) with e the exponent of the largest component (NaN when the
+// row holds an infinity or NaN, which makes every result of the row NaN).
 // What bounds it: about 290 FP64 / FP32 operations per element for its 32
 // bytes of residues.  12.5 ps per element (7680 x 512 rows of 48 matrices),
 // 3.8 TB/s of reads and writes; an update of 7680 x 7680 spends 4.5 % of its
@@ -274,8 +275,8 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
   for (int u = 0; u < 3; ++u) {
     const int i = 3 * w + u;
-    src[u] = i < 16 ? Ap + y * strideA + ((int64_t)(mt * 4 + i / 4) * 2 * RNS_L * KB + i % 4) * 1024
-                    : Bp + y * strideB + ((int64_t)(nt * 2 + (i - 16) / 4) * 2 * RNS_L * KB + i % 4) * 1024;
+    const int64_t rows = i < 16 ? mt * 4 + i / 4 : nt * 2 + (i - 16) / 4;
+    src[u] = (i < 16 ? Ap + y * strideA : Bp + y * strideB) + (rows * 2 * RNS_L * KB + i % 4) * 1024;
   }
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) signed char*)ring;
   const unsigned voff = lane * 16;
