@@ -1112,7 +1112,7 @@ __device__ __forceinline__ int swap_source(int x, int k0, const int* p, int kb, 
 // reads 32/W * 16 columns.  Four waves of 256 VGPRs (half a CU) find room beside
 // a trailing-update workgroup that ends; eight wait for both of a CU's, unless the
 // update leaves places often (qb_panel_leaf_form).  Per leaf of N = 530 and N = 1792
-// windows (32 matrices), on average: 91 and 95 us (up to 512 rows), 113 (1024) and 179
+// windows (32 matrices), on average: 91 and 94 us (up to 512 rows), 107 (1024) and 179
 // (2048); with the columns in global memory (k_getf2_long's order) 172 and 254 us.
 // ---------------------------------------------------------------------------
 template <typename T, int NT, int RPT, int W>
@@ -1808,10 +1808,10 @@ static bool lu_rns(int n) { return qb_lu_nb(n) == 512 && n - 512 >= kRnsMin; }
 // the panel runs beside an FP64 trailing update.
 //   complex128 with 512-wide panels, 1025 to 4096 rows: eight waves, twice the columns
 //   at a time and half the reads of L.  Per leaf of N = 4100 (32 matrices) beside the
-//   residue updates, 2049 to 4096 rows: 314 us, four waves 484; 1025 to 2048: 147 and
-//   180; up to 1024 101 either way.  Beside FP64 updates a window of 4100 takes 155 ms,
-//   with four waves 161.
-//   complex128, 4097 to 8192 rows: 0.99 ms per leaf beside the residue updates (N =
+//   residue updates, 2049 to 4096 rows: 333 us; 1025 to 2048: 158 (with four waves half
+//   as much again and a fifth more; up to 1024 100 either way).  Beside FP64 updates a
+//   window of 4100 takes 155 ms, with four waves 161.
+//   complex128, 4097 to 8192 rows: 0.95 ms per leaf beside the residue updates (N =
 //   8192, 48 matrices), k_getf2_long 2.56; beside FP64 updates k_getf2_long, whose
 //   registers leave room for their waves: windows of 6000 and 8192 394 ms and 1.245 s,
 //   against 417 ms and 1.30 s.
